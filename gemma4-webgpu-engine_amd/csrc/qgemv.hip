@@ -16,8 +16,8 @@
 // [x0 x2 x4 x6 | x1 x3 x5 x7]. The int32 row sum is exact (|sum| <= K * 8 * 128 < 2^31), so the
 // order of the reduction does not matter, and the epilogue is the reference's expression.
 //
-// The uncalibrated (inScale == 0) path keeps the f32 code dot: per lane in k order, then the fixed
-// 16-lane DPP tree (row16_sum_f32).
+// The uncalibrated (inScale == 0) path keeps the f32 code dot (qgemv_f32_kernel): FMA along each
+// lane's chunks, then the fixed 16-lane DPP tree (row16_sum_f32).
 #include "g4_internal.h"
 
 #include <algorithm>
@@ -352,58 +352,160 @@ __global__ __launch_bounds__(kGemvThreads) void qgemv_int_kernel(GemvLaunch L) {
     }
 }
 
-// The uncalibrated f32 code dot (inScale == 0, qgemv.ts:666-675): x stays f32 in LDS, each lane
-// sums code * x over its chunks in k order (separate rounded multiply and add), then the 16-lane
-// tree. One column per blockIdx.z. Parity against the reference's order is unpinned beyond the
-// exact-grid fixtures (the reference's own f32 order is adapter dependent).
-__global__ __launch_bounds__(kGemvThreads) void qgemv_f32_kernel(GemvLaunch L) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    float *xs = reinterpret_cast<float *>(smem);
+// The uncalibrated f32 code dot (inScale == 0, qgemv.ts:666-675). Bound: HBM, with the arithmetic
+// close behind: every weight code becomes an f32 and one FMA per column, 2.1 VALU instructions per
+// 4-bit code (22 us of issue for the 262144 x 1536 head, whose 201 MB take about 30 us).
+// - 16 lanes serve a row; a lane keeps the x values of its chunks (chunk t * 16 + lane16 of a slab of
+//   16 * CPL chunks) in registers and walks down the rows, so the loop reads nothing but weights.
+//   x read from LDS per row instead (128 bytes apart across lanes, so 16 lanes on 4 banks) took the
+//   head 341 us; now 42.0 us (4.8 TB/s), and 55.7 us for two columns (672 us in one pass each).
+// - A nibble becomes an exact f16 in place: (w & 0x000F000F) | 0x6400 6400 is the pair 1024 + u, the
+//   next nibble at the same bits under 0x5400 is 64 + u, one packed f16 subtract leaves both codes,
+//   and the FMA takes f16 x f32 + f32 (v_fma_mix_f32: the product and sum are f32, one rounding).
+// - Rows come in groups of 4 per wave, the next group's chunks requested before the current dot
+//   (the two buffers by name in an unrolled pair: as one buffer copied each turn, 56 us);
+//   a lane keeps one result of 16 groups, so scales and outputs move as 64 consecutive rows.
+// - The grid is what is resident (f32_blocks_per_cu), each wave an equal run of groups; longer K runs
+//   in slabs over 16 groups at a time, each slab's x staged once per block.
+// The order depends on K alone (FMA along each lane's chunk, the lane's chunks, the 16-lane tree, the
+// slabs), so a token column has the same bits at M = 1 and M = 2. Parity against the reference's order
+// is unpinned beyond the exact-grid fixtures (the reference's own f32 order is adapter dependent).
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+
+constexpr int kF32Strip = 16;  // row groups per stored run
+constexpr int kF32Depth = 2;   // groups' weights held at once: 42.0 us on the head (3: 42.9)
+// x values per lane and column: 96 (3 chunks of 32 4-bit codes, 6 of 16 8-bit ones would hold as
+// many; 4 keeps the double-buffered weights of two columns in 256 registers).
+template <int BITS> constexpr int f32_max_cpl() { return BITS == 4 ? 3 : 4; }
+template <int COLS> constexpr int f32_blocks_per_cu() { return COLS == 1 ? 3 : 2; }
+
+template <int BITS, int CPL, int COLS>
+__global__ __launch_bounds__(kGemvThreads, f32_blocks_per_cu<COLS>()) void qgemv_f32_kernel(GemvLaunch L) {
+    constexpr int CPC = BITS == 4 ? 32 : 16;  // codes per 16-byte chunk
+    constexpr int XSTR = CPC + 4;             // LDS words per chunk: 16 lanes' b128 reads on distinct banks
+    constexpr int SLAB = 16 * CPL;            // chunks per slab
+    __shared__ __align__(16) float xs[COLS][SLAB * XSTR];
     const int j = find_job(L, blockIdx.x);
     const GemvJob &J = L.job[j];
     const int tid = threadIdx.x;
-    const int k = J.k;
-    const int col = blockIdx.z;
-    for (int i = tid; i < k; i += kGemvThreads) {
-        const int64_t e = (int64_t)col * k + i;
-        xs[i] = J.act.up ? gelu_act_value(J.act, J.x, J.x_kind, e) : load_act(J.x, J.x_kind, e);
-    }
-    __syncthreads();
     const int lane = tid & 63, wave = tid >> 6, lane16 = lane & 15;
-    const int bits = J.bits;
-    const int row_bytes = bits == 4 ? (k >> 1) : k;
-    const int cpc = bits == 4 ? 32 : 16;
-    const int nch = k / cpc;
-    const int row_block = (blockIdx.x - J.wg_begin) * (J.passes * kRowsPerPass);
-    for (int p = 0; p < J.passes; ++p) {
-        const int wave_row0 = row_block + p * kRowsPerPass + wave * 4;
-        if (wave_row0 >= J.rows) break;
-        const int row = wave_row0 + (lane >> 4);
-        const int rrow = min(row, J.rows - 1);
-        const uint8_t *wrow = J.w + (int64_t)rrow * row_bytes;
-        float acc = 0.0f;
-        for (int ch = lane16; ch < nch; ch += 16) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(wrow + (int64_t)ch * 16);
-            const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
-            const float *xc = xs + ch * cpc;
-            if (bits == 4) {
+    const int k = J.k;
+    const int nch = k / CPC;
+    const int slabs = (nch + SLAB - 1) / SLAB;
+    const int64_t row_bytes = BITS == 4 ? (k >> 1) : k;
+    const int per = J.passes;  // row groups per wave (block uniform)
+    const int groups = (J.rows + 3) >> 2;
+    const int g_beg = ((blockIdx.x - J.wg_begin) * 4 + wave) * per;
+    const int g_end = min(g_beg + per, groups);
+
+    float xr[COLS][CPL][CPC];
+    for (int s0 = 0; s0 < per; s0 += kF32Strip) {
+        const int g0 = g_beg + s0;
+        const int n = min(kF32Strip, g_end - g0);  // <= 0: only the barriers
+        float tot[COLS];
 #pragma unroll
-                for (int i = 0; i < 32; ++i) {
-                    const int code = (int)((wv[i >> 3] >> (4 * (i & 7))) & 0xf) - 8;
-                    acc = __fadd_rn(acc, __fmul_rn((float)code, xc[i]));
+        for (int c = 0; c < COLS; ++c) tot[c] = 0.0f;
+        for (int sl = 0; sl < slabs; ++sl) {
+            const int ch0 = sl * SLAB;
+            if (slabs > 1 || s0 == 0) {
+                __syncthreads();  // the previous slab's x is in registers
+                for (int i = tid; i < COLS * SLAB * CPC; i += kGemvThreads) {
+                    const int c = i / (SLAB * CPC), e = i - c * (SLAB * CPC);
+                    const int kk = ch0 * CPC + e;
+                    float v = 0.0f;  // past K: zero times a clamped chunk's finite codes
+                    if (kk < k) {
+                        const int64_t at = (int64_t)c * k + kk;
+                        v = J.act.up ? gelu_act_value(J.act, J.x, J.x_kind, at) : load_act(J.x, J.x_kind, at);
+                    }
+                    xs[c][(e / CPC) * XSTR + e % CPC] = v;
                 }
-            } else {
+                __syncthreads();
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int code = (int)(int8_t)((wv[i >> 2] >> (8 * (i & 3))) & 0xff);
-                    acc = __fadd_rn(acc, __fmul_rn((float)code, xc[i]));
+                for (int c = 0; c < COLS; ++c)
+#pragma unroll
+                    for (int t = 0; t < CPL; ++t)
+#pragma unroll
+                        for (int q = 0; q < CPC / 4; ++q) {
+                            const float4 v = *reinterpret_cast<const float4 *>(&xs[c][(t * 16 + lane16) * XSTR + 4 * q]);
+                            xr[c][t][4 * q] = v.x, xr[c][t][4 * q + 1] = v.y;
+                            xr[c][t][4 * q + 2] = v.z, xr[c][t][4 * q + 3] = v.w;
+                        }
+            }
+            if (n <= 0) continue;
+            const uint8_t *wl[CPL];
+#pragma unroll
+            for (int t = 0; t < CPL; ++t) wl[t] = J.w + (int64_t)min(ch0 + t * 16 + lane16, nch - 1) * 16;
+            u32x4 buf[kF32Depth][CPL];
+            auto request = [&](u32x4 (&b)[CPL], int it) {
+                const int row = min((g0 + min(it, n - 1)) * 4 + (lane >> 4), J.rows - 1);
+#pragma unroll
+                for (int t = 0; t < CPL; ++t) b[t] = load16_stream(wl[t] + row * row_bytes);
+            };
+#pragma unroll
+            for (int d = 0; d < kF32Depth - 1; ++d) request(buf[d], d);
+            float keep[COLS];
+#pragma unroll
+            for (int c = 0; c < COLS; ++c) keep[c] = 0.0f;
+            for (int it0 = 0; it0 < n; it0 += kF32Depth) {
+#pragma unroll
+                for (int d = 0; d < kF32Depth; ++d) {
+                    const int it = it0 + d;
+                    if (it >= n) break;
+                    const u32x4 (&cur)[CPL] = buf[d];
+                    request(buf[(d + kF32Depth - 1) % kF32Depth], it + kF32Depth - 1);
+                    float sum[COLS];
+#pragma unroll
+                    for (int t = 0; t < CPL; ++t) {
+                        const uint32_t wv[4] = {cur[t].x, cur[t].y, cur[t].z, cur[t].w};
+                        float acc[COLS];
+#pragma unroll
+                        for (int c = 0; c < COLS; ++c) acc[c] = 0.0f;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if constexpr (BITS == 4) {
+                                const uint32_t w8 = wv[i] >> 8;
+                                const h2 k04 = __builtin_bit_cast(h2, (wv[i] & 0x000F000Fu) | 0x64006400u) - h2{1032, 1032};
+                                const h2 k15 = __builtin_bit_cast(h2, (wv[i] & 0x00F000F0u) | 0x54005400u) - h2{72, 72};
+                                const h2 k26 = __builtin_bit_cast(h2, (w8 & 0x000F000Fu) | 0x64006400u) - h2{1032, 1032};
+                                const h2 k37 = __builtin_bit_cast(h2, (w8 & 0x00F000F0u) | 0x54005400u) - h2{72, 72};
+                                const h2 code[4] = {k04, k15, k26, k37};
+#pragma unroll
+                                for (int c = 0; c < COLS; ++c)
+#pragma unroll
+                                    for (int e = 0; e < 4; ++e) {
+                                        acc[c] = __builtin_fmaf((float)code[e].x, xr[c][t][8 * i + e], acc[c]);
+                                        acc[c] = __builtin_fmaf((float)code[e].y, xr[c][t][8 * i + 4 + e], acc[c]);
+                                    }
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const float code = (float)(int8_t)((wv[i] >> (8 * e)) & 0xff);
+#pragma unroll
+                                    for (int c = 0; c < COLS; ++c) acc[c] = __builtin_fmaf(code, xr[c][t][4 * i + e], acc[c]);
+                                }
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < COLS; ++c) sum[c] = t == 0 ? acc[c] : __fadd_rn(sum[c], acc[c]);
+                    }
+#pragma unroll
+                    for (int c = 0; c < COLS; ++c) {
+                        sum[c] = row16_sum_f32(sum[c]);  // in every lane of the row's 16
+                        keep[c] = lane16 == it ? sum[c] : keep[c];
+                    }
                 }
             }
+#pragma unroll
+            for (int c = 0; c < COLS; ++c) tot[c] = sl == 0 ? keep[c] : __fadd_rn(tot[c], keep[c]);
         }
-        const float sum = row16_sum_f32(acc);
-        if (lane16 == 0 && row < J.rows) {
-            const float y = linear_epilogue(1.0f, J.scales[row], sum);
-            store_linear_out(J.dst, (int64_t)col * J.rows + row, J.out_kind, y, 0, J.out_scale);
+        // lane (r = lane / 16, lane16) holds row r of group g0 + lane16
+        const int row = (g0 + lane16) * 4 + (lane >> 4);
+        if (lane16 < n && row < J.rows) {
+            const float scale = J.scales[row];
+#pragma unroll
+            for (int c = 0; c < COLS; ++c)
+                store_linear_out(J.dst, (int64_t)c * J.rows + row, J.out_kind,
+                                 linear_epilogue(1.0f, scale, tot[c]), 0, J.out_scale);
         }
     }
 }
@@ -556,10 +658,10 @@ static int kwaves_for(int k) { return k >= 6144 ? 4 : k >= 3072 ? 2 : 1; }
 static int rows_per_block(const GemvJob &J) { return J.passes * (kRowsPerPass / J.kwaves); }
 
 // Picks passes per block so the launch offers a few blocks per CU without starving small jobs.
-static void plan_blocks(GemvLaunch &L, int max_passes, bool split_k_waves) {
+static void plan_blocks(GemvLaunch &L, int max_passes) {
     int64_t total_groups = 0;
     for (int i = 0; i < L.count; ++i) {
-        L.job[i].kwaves = split_k_waves ? kwaves_for(L.job[i].k) : 1;
+        L.job[i].kwaves = kwaves_for(L.job[i].k);
         total_groups += (L.job[i].rows + kRowsPerPass / L.job[i].kwaves - 1) /
                         (kRowsPerPass / L.job[i].kwaves);
     }
@@ -579,6 +681,35 @@ static int total_blocks(const GemvLaunch &L) {
     return last.wg_begin + (last.rows + rows_per_block(last) - 1) / rows_per_block(last);
 }
 
+// Lays the uncalibrated jobs out (one K and width per launch: a single linear, or a batch over one x)
+// and launches the f32 kernel of their slab shape.
+template <int BITS, int COLS> static void launch_f32_t(GemvLaunch &L, hipStream_t stream) {
+    constexpr int MAX = f32_max_cpl<BITS>();
+    const int nch = L.job[0].k / (BITS == 4 ? 32 : 16);
+    const int slabs = (nch + 16 * MAX - 1) / (16 * MAX);
+    const int cpl = (nch + 16 * slabs - 1) / (16 * slabs);
+    int64_t groups = 0;
+    for (int i = 0; i < L.count; ++i) groups += (L.job[i].rows + 3) / 4;
+    const int64_t waves = 4LL * f32_blocks_per_cu<COLS>() * device_cu_count();
+    const int per = (int)std::max<int64_t>(1, (groups + waves - 1) / waves);
+    int wg = 0;
+    for (int i = 0; i < L.count; ++i) {
+        L.job[i].passes = per;
+        L.job[i].wg_begin = wg;
+        wg += ((L.job[i].rows + 3) / 4 + 4 * per - 1) / (4 * per);
+    }
+    const dim3 grid(wg), block(kGemvThreads);
+    if (cpl == 1) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 1, COLS>), grid, block, 0, stream, L);
+    else if (cpl == 2) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 2, COLS>), grid, block, 0, stream, L);
+    else if (cpl == 3) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 3, COLS>), grid, block, 0, stream, L);
+    else hipLaunchKernelGGL((qgemv_f32_kernel<BITS, MAX, COLS>), grid, block, 0, stream, L);
+}
+
+static void launch_f32(GemvLaunch &L, int cols, hipStream_t stream) {
+    if (L.job[0].bits == 4) cols == 1 ? launch_f32_t<4, 1>(L, stream) : launch_f32_t<4, 2>(L, stream);
+    else cols == 1 ? launch_f32_t<8, 1>(L, stream) : launch_f32_t<8, 2>(L, stream);
+}
+
 // Launches the integer or f32 GEMV over L.count jobs with `cols` token columns (1 or 2).
 int launch_gemv(GemvLaunch &L, int cols, hipStream_t stream) {
     if (L.count < 1 || L.count > G4_MAX_GROUP)
@@ -595,11 +726,11 @@ int launch_gemv(GemvLaunch &L, int cols, hipStream_t stream) {
         int rc = try_stream(L, cols, stream, &launched);
         if (rc || launched) return rc;
     }
-    plan_blocks(L, L.splits > 1 ? 1 : kMaxPasses, calibrated);
-    const int blocks = total_blocks(L);
-    int max_k = 0;
-    for (int i = 0; i < L.count; ++i) max_k = std::max(max_k, L.job[i].k);
     if (calibrated) {
+        plan_blocks(L, L.splits > 1 ? 1 : kMaxPasses);
+        const int blocks = total_blocks(L);
+        int max_k = 0;
+        for (int i = 0; i < L.count; ++i) max_k = std::max(max_k, L.job[i].k);
         const size_t lds = (size_t)cols * ((max_k + 15) & ~15);
         dim3 grid(blocks, std::max(1, L.splits), 1);
         if (cols == 1)
@@ -608,9 +739,7 @@ int launch_gemv(GemvLaunch &L, int cols, hipStream_t stream) {
             hipLaunchKernelGGL(qgemv_int_kernel<2>, grid, dim3(kGemvThreads), lds, stream, L);
         G4_LAUNCHED("qgemv_int_kernel");
     } else {
-        const size_t lds = (size_t)max_k * sizeof(float);
-        dim3 grid(blocks, 1, cols);
-        hipLaunchKernelGGL(qgemv_f32_kernel, grid, dim3(kGemvThreads), lds, stream, L);
+        launch_f32(L, cols, stream);
         G4_LAUNCHED("qgemv_f32_kernel");
     }
     return G4_OK;
