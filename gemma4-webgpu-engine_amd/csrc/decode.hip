@@ -30,6 +30,7 @@ namespace g4 {
 constexpr int kDecThreads = 256;
 constexpr int kAttnChunk = 32;
 constexpr int kAttnMaxHeads = 8;
+typedef float v4f __attribute__((ext_vector_type(4)));  // one lane's 4 MFMA outputs
 // Word 3 of a gfx9 buffer resource for untyped dword loads (DATA_FORMAT 32, no swizzle).
 constexpr int kBufferRsrcWord3 = 0x00020000;
 
@@ -183,10 +184,11 @@ __device__ __forceinline__ void wave_codes_spread(uint32_t word, int (&code)[4])
     }
 }
 
-// Writes the four results of the lane to out[l + 64 k].
+// Hands the four results of the lane to put(l + 64 k, value).
+template <typename Put>
 __device__ __forceinline__ void wave_norm_rope(const int (&code)[4], const float (&gt)[4],
                                                const RopeRow &rope, float scale, bool gain,
-                                               bool rotate, float eps, float *out) {
+                                               bool rotate, float eps, Put put) {
     const int l = threadIdx.x & 63;
     float x[4];
 #pragma unroll
@@ -202,55 +204,68 @@ __device__ __forceinline__ void wave_norm_rope(const int (&code)[4], const float
     }
     if (!rotate) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) out[l + 64 * k] = y[k];
+        for (int k = 0; k < 4; ++k) put(l + 64 * k, y[k]);
         return;
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {  // pair (l + 64 k, l + 64 k + 128)
         const float lo = y[k], hi = y[k + 2];
-        out[l + 64 * k] = __fsub_rn(__fmul_rn(lo, rope.c[k]), __fmul_rn(hi, rope.sn[k]));
-        out[l + 64 * k + 128] = __fadd_rn(__fmul_rn(hi, rope.c[k]), __fmul_rn(lo, rope.sn[k]));
+        put(l + 64 * k, __fsub_rn(__fmul_rn(lo, rope.c[k]), __fmul_rn(hi, rope.sn[k])));
+        put(l + 64 * k + 128, __fadd_rn(__fmul_rn(hi, rope.c[k]), __fmul_rn(lo, rope.sn[k])));
     }
 }
 
-// Grid (max chunks, rows), HALVES x 256 threads (t = the thread's index in its half of 256).
-// Chunk c covers positions lo + 32 c .. min(+32, pos + 1), for every query head of the row at once
-// (heads <= 8 share the one KV head), so each K and V row of the chunk is fetched once per block.
-// HALVES 2 (a grid no wider than the CU count: batch 1): half 0 takes heads 0..3, half 1 heads
-// 4..7, two waves per SIMD with half the dependent chains each; HALVES 1 (wide grids, where the
-// chip is full anyway): every thread takes all heads. Scores: thread t takes eighth t & 7 (32 dims, sequential) of position t >> 3 against its
-// half's heads, and the position's eight lanes combine by the pairwise tree
-// ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)) (an xor butterfly: IEEE addition commutes, so
-// every lane ends with the tree's value). Per head (one 32-lane group of half 0 each): m = max,
-// e = exp(s - m), l = the 32-lane pairwise tree of e. Then thread t accumulates, for its half's
-// heads, sum over positions (ascending) of e * v[t]. Writes (m, l) and o[256] per (row, head,
-// chunk). PRO: q (and on a producer, the position's K and V rows) come from the prologue run here:
-// wave w rebuilds query heads w, w + waves, ...; in the block whose chunk holds the position, waves
-// 0 and 1 also build the new K and V rows, which the block stores and uses in place of the stale
-// rows it loaded.
-// Float4 slot of the chunk's K group (row r, float4 column c4) in the split kernel's LDS copy.
-// Within each 8-slot segment (one lane's 32 dims), slot m moves to (m + seg/2 + 4*(r&1)) mod 8:
-// the 16 lanes of one ds_read_b128 phase (two rows x eight segments, same m) then hit 16
-// distinct 4-bank groups, and 16 consecutive columns of one row (a write phase) stay distinct.
-__device__ __forceinline__ int k_slot(int r, int c4) {
-    const int seg = c4 >> 3;
-    return r * (kDecThreads / 4) + seg * 8 + (((c4 & 7) + (seg >> 1) + 4 * (r & 1)) & 7);
-}
+// Grid (max chunks, rows), HALVES x 256 threads. Chunk c covers positions lo + 32 c .. min(+32,
+// pos + 1), for every query head of the row at once (heads <= 8 share the one KV head), so each K
+// and V row of the chunk is fetched once per block.
+//
+// Both products run on v_mfma_f32_4x4x1 (16 blocks of 4 x 4 x 1, K = 1): one instruction is one
+// f32 fused multiply-add per output, the same bits as __fmaf_rn (subnormals, infinities and NaN
+// included), so a chain of them is the stated sequential sum. It takes both operands from
+// registers (a VALU form reads a query or a weight from LDS for every four multiply-adds of a
+// lane) and does 32 multiply-adds per cycle and SIMD where the VALU does 16.
+//  Scores: lane (b = lane / 4, j = lane % 4) of quarter w holds position 8 w + 4 (b / 8) + j, eighth
+//   b % 8 (32 dims, sequential); the A rows are four heads' values of that eighth. The position's
+//   eight partial dots combine by the pairwise tree ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7))
+//   over lanes 4, 8 and 16 apart.
+//  Per head (one 32-lane group each): m = max, e = exp(s - m), l = the 32-lane pairwise tree of e.
+//  P V: lane l of quarter w holds dim 64 w + l; step u adds e[head][u] * v[u][dim] (ascending).
+// Writes (m, l) and o[256] per (row, head, chunk).
+// HALVES 2 (a grid no wider than the CU count: batch 1): half 0 takes heads 0..3, half 1 heads 4..7;
+// HALVES 1 (wide grids): a wave takes all heads (two accumulator chains).
+// K and V both arrive as whole-row 16-byte loads issued at the head; V waits in registers and goes
+// through the K copy's LDS once the scores are done.
+// PRO: q (and on a producer, the position's K and V rows) come from the prologue run here: wave w
+// rebuilds query heads w, w + waves, ...; in the block whose chunk holds the position, waves 0 and
+// 1 also build the new K and V rows, which the block stores and uses in place of the stale rows
+// it loaded.
+//
+// Rows of 256 floats in LDS: eighths 36 floats apart, rows 304, so the 16 lanes of a score operand
+// read (four eighths x four rows of one float4 index) hit 16 distinct 4-bank groups, every read of
+// a lane is one address plus a constant, and three blocks (52 KB each) fit a CU.
+constexpr int kSegFloats = 36, kRowFloats = 304;
+__device__ __forceinline__ int row_at(int r, int d) { return r * kRowFloats + (d >> 5) * kSegFloats + (d & 31); }
 
-template <bool PRO, int HALVES, bool KST>
-__global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
+constexpr int kEsStride = kAttnChunk + 4;  // floats per head of the weights (bank spread)
+
+template <bool PRO, int HALVES>
+__global__ __launch_bounds__(HALVES * kDecThreads, HALVES == 1 ? 3 : 2) void attn_split_kernel(
     const float *q, const float *k_cache, const float *v_cache, int64_t cache_row_stride, int heads,
     int pos_host, const int32_t *pos_dev, int window, float *part_ml, float *part_o, int max_chunks,
     AttnPrologue pro) {
-    __shared__ __align__(16) float qs[kAttnMaxHeads * kDecThreads];
-    __shared__ __align__(16) float es[kAttnMaxHeads * kAttnChunk];
+    __shared__ __align__(16) float qs[kAttnMaxHeads * kRowFloats];
+    __shared__ __align__(16) float es[kAttnMaxHeads * kEsStride];
     __shared__ __align__(16) float kvnew[PRO ? 2 * kDecThreads : 1];
-    __shared__ __align__(16) float4 ks[KST ? kAttnChunk * kDecThreads / 4 : 1];
-    constexpr int THREADS = HALVES * kDecThreads, WAVES = THREADS / 64;
-    constexpr int HH = kAttnMaxHeads / HALVES;        // heads per thread in scores and PV
+    __shared__ __align__(16) float ks[kAttnChunk * kRowFloats];
+    // K and V of a wide grid are read once: non-temporal (aux bit 1)
+    constexpr int kAux = HALVES == 1 ? 2 : 0;
+    constexpr int WAVES = 4 * HALVES;
+    constexpr int GH = 2 / HALVES;                            // four-head groups per wave
     constexpr int QPW = (kAttnMaxHeads + WAVES - 1) / WAVES;  // query heads per wave (prologue)
+    constexpr int RPW = kAttnChunk / WAVES;                   // K (and V) rows a wave loads
     const int tid = threadIdx.x;
-    const int half = tid >> 8, t = tid & (kDecThreads - 1), w = tid >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int half = w >> 2, w4 = w & 3, t = tid & (kDecThreads - 1);
     const int c = blockIdx.x;
     const int64_t row = blockIdx.y;
     const int pos = step_pos(pos_host, pos_dev);
@@ -259,17 +274,17 @@ __global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
     if (c >= chunks) return;  // whole block
     // the accumulator the merge adds o_proj's per-head partials into starts at zero
     if (PRO && pro.zero && c == 0 && row == 0)
-        for (int i = tid; i < pro.zero_n; i += THREADS) pro.zero[i] = 0;
+        for (int i = tid; i < pro.zero_n; i += HALVES * kDecThreads) pro.zero[i] = 0;
     const int start = lo + c * kAttnChunk;
     const int cnt = min(kAttnChunk, pos + 1 - start);
     float *kb = const_cast<float *>(k_cache) + row * cache_row_stride;
     float *vb = const_cast<float *>(v_cache) + row * cache_row_stride;
     // the producer's new K and V rows belong to the chunk that holds the position (its last)
     const bool store_kv = PRO && pro.k_codes && c == chunks - 1;
-    // the prologue's few operands go out first, then the chunk's K segment and V rows, so the
-    // prologue's arithmetic waits for its own loads only and overlaps the chunk's
+    // the query's (or the prologue's) few operands go out first, then the chunk's K and V rows, so
+    // the prologue's arithmetic waits for its own loads only and overlaps the chunk's
     uint32_t qw[QPW], kvw = 0;
-    float qg[4], kg[4];
+    float qg[4], kg[4], qv[PRO ? 1 : kAttnMaxHeads / HALVES];
     RopeRow rope;
     if (PRO) {
         // heads past the last and the K / V rows of waves that do not build them read valid
@@ -289,15 +304,12 @@ __global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
         wave_gain_load(pro.q_gain, qg);
         wave_gain_load(kv_wave && w == 0 ? pro.k_gain : pro.q_gain, kg);
         rope = wave_rope_row(cos_row, sin_row);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kAttnMaxHeads / HALVES; ++i)  // absent heads read the last one
+            qv[i] = q[(row * heads + min(half + HALVES * i, heads - 1)) * kDecThreads + t];
     }
     __builtin_amdgcn_sched_barrier(0);  // the prologue's loads first, then K, then V
-    const int j = t >> 3, sg = t & 7;
-    float4 kq[8];
-    // KST: the chunk's K rows come in as whole-row float4 runs (one load instruction covers
-    // consecutive 16-byte columns) and reach the lanes' 32-dim segments through LDS; otherwise
-    // each lane reads its own segment (eight loads, each spread over 64 lines)
-    constexpr int KPT = KST ? kAttnChunk * kDecThreads / 4 / THREADS : 1;
-    float4 kl[KPT];
     // The chunk's rows start .. start + cnt - 1 of K and V as buffer resources: a load is the
     // lane's byte offset (one VGPR for every load) plus a scalar row offset, where 64-bit vector
     // addresses per load would hold two VGPRs each until it issues. Every offset stays inside the
@@ -307,41 +319,17 @@ __global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
         kb + (int64_t)start * kDecThreads, (short)0, cnt * kRowBytes, kBufferRsrcWord3);
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
         vb + (int64_t)start * kDecThreads, (short)0, cnt * kRowBytes, kBufferRsrcWord3);
-    // KST, load i: thread f = tid + i * THREADS takes row f / 64 (wave-uniform), float4 column
-    // f % 64, of K and of V
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    if (KST) {
+    float4 kl[RPW];  // row RPW w + i, float4 column `lane`: one load instruction is one whole row
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int r = min(wv + WAVES * i, cnt - 1);
-            kl[i] = __builtin_bit_cast(
-                float4, __builtin_amdgcn_raw_buffer_load_b128(kres, lane * 16, r * kRowBytes, 0));
-        }
-    } else {
-        const float4 *kr = reinterpret_cast<const float4 *>(
-            kb + (int64_t)(start + min(j, cnt - 1)) * kDecThreads + sg * 32);
-#pragma unroll
-        for (int i4 = 0; i4 < 8; ++i4) kq[i4] = kr[i4];
-    }
+    for (int i = 0; i < RPW; ++i)
+        kl[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               kres, lane * 16, min(RPW * w + i, cnt - 1) * kRowBytes, kAux));
     __builtin_amdgcn_sched_barrier(0);  // K ahead of V: the wait for K leaves V in flight
-    // KST: V as whole-row float4 runs too, staged through the K copy's LDS once the scores are
-    // done; otherwise lane t loads dim t of every position
-    float4 vl[KST ? KPT : 1];
-    float vv[KST ? 1 : kAttnChunk];
-    if (KST) {
+    float4 vl[RPW];
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int r = min(wv + WAVES * i, cnt - 1);
-            vl[i] = __builtin_bit_cast(
-                float4, __builtin_amdgcn_raw_buffer_load_b128(vres, lane * 16, r * kRowBytes, 0));
-        }
-    } else {
-#pragma unroll
-        for (int u = 0; u < kAttnChunk; ++u)
-            vv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                  vres, t * 4, min(u, cnt - 1) * kRowBytes, 0));
-    }
+    for (int i = 0; i < RPW; ++i)
+        vl[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               vres, lane * 16, min(RPW * w + i, cnt - 1) * kRowBytes, kAux));
     __builtin_amdgcn_sched_barrier(0);  // every load issued before the prologue's arithmetic
     if (PRO) {
 #pragma unroll
@@ -350,113 +338,87 @@ __global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
             if (h < heads) {
                 int code[4];
                 wave_codes_spread(qw[i], code);
-                wave_norm_rope(code, qg, rope, pro.q_scale, true, true, pro.eps, qs + h * kDecThreads);
+                wave_norm_rope(code, qg, rope, pro.q_scale, true, true, pro.eps, [&](int d, float v) {
+                    qs[row_at(h, d)] = v;
+                });
             }
         }
         if (store_kv && w < 2) {
             int code[4];
             wave_codes_spread(kvw, code);
-            if (w == 0) wave_norm_rope(code, kg, rope, pro.k_scale, true, true, pro.eps, kvnew);
-            else wave_norm_rope(code, kg, rope, pro.v_scale, false, false, pro.eps, kvnew + kDecThreads);
+            if (w == 0)
+                wave_norm_rope(code, kg, rope, pro.k_scale, true, true, pro.eps,
+                               [&](int d, float v) { kvnew[d] = v; });
+            else
+                wave_norm_rope(code, kg, rope, pro.v_scale, false, false, pro.eps,
+                               [&](int d, float v) { kvnew[kDecThreads + d] = v; });
         }
     } else {
-        for (int i = tid; i < heads * kDecThreads; i += THREADS)
-            qs[i] = q[row * heads * kDecThreads + i];
-    }
-    if (KST) {
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int f = tid + i * THREADS;
-            ks[k_slot(f / (kDecThreads / 4), f % (kDecThreads / 4))] = kl[i];
-        }
+        for (int i = 0; i < kAttnMaxHeads / HALVES; ++i)
+            qs[row_at(half + HALVES * i, t)] = qv[i];
     }
-    __syncthreads();
-    if (KST) {
 #pragma unroll
-        for (int i4 = 0; i4 < 8; ++i4) kq[i4] = ks[k_slot(j, sg * 8 + i4)];
-    }
-    if (store_kv) {
+    for (int i = 0; i < RPW; ++i) *reinterpret_cast<float4 *>(ks + row_at(RPW * w + i, 4 * lane)) = kl[i];
+    lds_barrier();  // V stays in flight
+    const int jp = store_kv ? pos - start : -1;
+    if (store_kv && half == 0) {
         // the position's row: the cache gets it, and this block's operands take it in place of the
         // stale row they loaded
-        const int jp = pos - start;
-        if (half == 0) {
-            kb[(int64_t)pos * kDecThreads + t] = kvnew[t];
-            vb[(int64_t)pos * kDecThreads + t] = kvnew[kDecThreads + t];
-        }
-        if (j == jp) {
-#pragma unroll
-            for (int i4 = 0; i4 < 8; ++i4)
-                kq[i4] = *reinterpret_cast<const float4 *>(kvnew + sg * 32 + 4 * i4);
-        }
-        if (!KST) {  // KST: the V row is replaced where the rows go to LDS
-#pragma unroll
-            for (int u = 0; u < kAttnChunk; ++u)
-                if (u == jp) vv[u] = kvnew[kDecThreads + t];
-        }
+        kb[(int64_t)pos * kDecThreads + t] = kvnew[t];
+        vb[(int64_t)pos * kDecThreads + t] = kvnew[kDecThreads + t];
     }
 
-    // scores of this half's heads: eight sequential 32-dim dot products (segment sg) per score, one
-    // fused multiply-add (a single rounding) per element, as the CPU restatement's fmaf;
-    // then the pairwise tree over the segments by DPP within each aligned 8-lane group:
-    // quad_perm(1,0,3,2) and (2,3,0,1) give every lane of a quad ((s0+s1)+(s2+s3)), then
-    // row_half_mirror brings the other quad's sum (a commutative last add). With every head
-    // present the guard-free form lets the eight chains interleave.
-    float sc[HH];
-    auto score = [&](int h) {
-        const float *qh = qs + h * kDecThreads + sg * 32;
-        float a = 0.0f;
+    // scores of this wave's head groups: eight sequential 32-dim dot products (eighth sg) per score
+    const int j = 8 * w4 + 4 * (lane >> 5) + (lane & 3), sg = (lane >> 2) & 7, hq = lane & 3;
+    v4f sc[GH];
 #pragma unroll
-        for (int i4 = 0; i4 < 8; ++i4) {
-            const float4 qv = *reinterpret_cast<const float4 *>(qh + 4 * i4);
-            const float4 kv = kq[i4];
-            a = __fmaf_rn(qv.x, kv.x, a);
-            a = __fmaf_rn(qv.y, kv.y, a);
-            a = __fmaf_rn(qv.z, kv.z, a);
-            a = __fmaf_rn(qv.w, kv.w, a);
+    for (int g = 0; g < GH; ++g) sc[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        float4 kv = *reinterpret_cast<const float4 *>(ks + row_at(j, 32 * sg) + 4 * m);
+        if constexpr (PRO)
+            if (j == jp) kv = *reinterpret_cast<const float4 *>(kvnew + sg * 32 + 4 * m);
+        const float kk[4] = {kv.x, kv.y, kv.z, kv.w};
+        float qq[GH][4];
+#pragma unroll
+        for (int g = 0; g < GH; ++g) {
+            const float4 v = *reinterpret_cast<const float4 *>(qs + row_at((half + g) * 4 + hq, 32 * sg) + 4 * m);
+            qq[g][0] = v.x, qq[g][1] = v.y, qq[g][2] = v.z, qq[g][3] = v.w;
         }
-        return a;
-    };
-    if (heads == kAttnMaxHeads) {
 #pragma unroll
-        for (int hh = 0; hh < HH; ++hh) sc[hh] = score(half * HH + hh);
-    } else {
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int hh = 0; hh < HH; ++hh) sc[hh] = half * HH + hh < heads ? score(half * HH + hh) : 0.0f;
+            for (int g = 0; g < GH; ++g)
+                sc[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(qq[g][e], kk[e], sc[g], 0, 0, 0);
     }
 #pragma unroll
-    for (int hh = 0; hh < HH; ++hh) {
-        float a = __fadd_rn(sc[hh], dpp_f32_b1(sc[hh]));
-        a = __fadd_rn(a, dpp_f32_4e(a));
-        sc[hh] = __fadd_rn(a, dpp_f32_half_mirror(a));
-    }
-    if (sg == 0) {
+    for (int g = 0; g < GH; ++g)
 #pragma unroll
-        for (int hh = 0; hh < HH; ++hh) {
-            const int h = half * HH + hh;
-            if (h < heads) es[h * kAttnChunk + j] = j < cnt ? sc[hh] : -__int_as_float(0x7f800000);
+        for (int i = 0; i < 4; ++i) {  // row i: head 4 (half + g) + i; lanes of eighth 0 get the tree
+            float a = sc[g][i];
+            a = __fadd_rn(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x104, 0xF, 0xF, true)));
+            a = __fadd_rn(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x108, 0xF, 0xF, true)));
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+            a = __fadd_rn(a, __uint_as_float(r[1]));
+            if (sg == 0) es[((half + g) * 4 + i) * kEsStride + j] = j < cnt ? a : -__int_as_float(0x7f800000);
         }
-    }
-    __syncthreads();
-    if (KST) {
-        // the chunk's V rows into the K copy's LDS (every thread read its K operands before the
-        // barrier above), row-major: position u's 256 dims at u * 256 floats; a producer's last
-        // chunk takes the position's new row from kvnew
-        int jp = -1;
-        if constexpr (PRO) jp = store_kv ? pos - start : -1;
+    lds_barrier();
+    // the chunk's V rows into the K copy's LDS (every wave read its K operands before the barrier
+    // above), row-major; a producer's last chunk takes the position's new row from kvnew
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int r = wv + WAVES * i;
-            float4 v = vl[i];
-            if constexpr (PRO)
-                if (r == jp) v = *reinterpret_cast<const float4 *>(kvnew + kDecThreads + 4 * lane);
-            ks[r * (kDecThreads / 4) + lane] = v;
-        }
+    for (int i = 0; i < RPW; ++i) {
+        const int r = RPW * w + i;
+        float4 v = vl[i];
+        if constexpr (PRO)
+            if (r == jp) v = *reinterpret_cast<const float4 *>(kvnew + kDecThreads + 4 * lane);
+        *reinterpret_cast<float4 *>(ks + r * kDecThreads + 4 * lane) = v;
     }
 
     // per head, uniform within its 32-lane group of half 0: max, exp, the pairwise sum
     const int hh = t >> 5, p = t & 31;
     if (half == 0 && hh < heads) {
-        const float x = es[hh * kAttnChunk + p];
+        const float x = es[hh * kEsStride + p];
         float m = x;
         {  // the group's maximum, in every lane of the group
             const float mg = half_wave_max(m);
@@ -467,66 +429,58 @@ __global__ __launch_bounds__(HALVES * kDecThreads) void attn_split_kernel(
         const float e = p < cnt ? d_expf(__fsub_rn(x, m)) : 0.0f;
         float l = e;
         l = half_wave_tree_sum(l);  // lane p = 0 of each 32-lane group holds its head's sum
-        es[hh * kAttnChunk + p] = e;
+        es[hh * kEsStride + p] = e;
         if (p == 0) {
             const int64_t slot = (row * heads + hh) * max_chunks + c;
             part_ml[slot * 2] = m;
             part_ml[slot * 2 + 1] = l;
         }
     }
-    __syncthreads();
+    lds_barrier();
 
-    // o[h][d] = sum over positions (ascending) of e[h][j] * v[j][d] (one fused multiply-add each),
-    // for this half's heads; a whole chunk with every head present takes the guard-free form, whose
-    // chains interleave (each V value read once for all of them)
-    const float *vsf = reinterpret_cast<const float *>(ks);
-    auto vval = [&](int u) { return KST ? vsf[u * kDecThreads + t] : vv[u]; };
-    if (heads == kAttnMaxHeads && cnt == kAttnChunk) {
-        float o[HH];
+    // o[h][d] = sum over positions (ascending) of e[h][j] * v[j][d]; positions past the chunk's end
+    // add nothing (their V row is a stand-in)
+    v4f o[GH];
 #pragma unroll
-        for (int g = 0; g < HH; ++g) o[g] = 0.0f;
+    for (int g = 0; g < GH; ++g) o[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto step4 = [&](int u4, int n) {
+        float e[GH][4], v[4];
 #pragma unroll
-        for (int u4 = 0; u4 < kAttnChunk; u4 += 4) {  // four weights per LDS read
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = vval(u4 + i);
-#pragma unroll
-            for (int g = 0; g < HH; ++g) {
-                const float4 e4 = *reinterpret_cast<const float4 *>(es + (half * HH + g) * kAttnChunk + u4);
-                o[g] = __fmaf_rn(e4.x, v[0], o[g]);
-                o[g] = __fmaf_rn(e4.y, v[1], o[g]);
-                o[g] = __fmaf_rn(e4.z, v[2], o[g]);
-                o[g] = __fmaf_rn(e4.w, v[3], o[g]);
-            }
+        for (int g = 0; g < GH; ++g) {
+            const float4 x = *reinterpret_cast<const float4 *>(es + ((half + g) * 4 + hq) * kEsStride + u4);
+            e[g][0] = x.x, e[g][1] = x.y, e[g][2] = x.z, e[g][3] = x.w;
         }
 #pragma unroll
-        for (int g = 0; g < HH; ++g)
-            part_o[((row * heads + half * HH + g) * max_chunks + c) * kDecThreads + t] = o[g];
+        for (int i = 0; i < 4; ++i) v[i] = ks[(u4 + i) * kDecThreads + t];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i < n)
+#pragma unroll
+                for (int g = 0; g < GH; ++g)
+                    o[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(e[g][i], v[i], o[g], 0, 0, 0);
+    };
+    if (cnt == kAttnChunk) {
+#pragma unroll
+        for (int u4 = 0; u4 < kAttnChunk; u4 += 4) step4(u4, 4);
     } else {
 #pragma unroll
-        for (int g = 0; g < HH; ++g) {
-            const int h = half * HH + g;
-            if (h >= heads) continue;
-            float o = 0.0f;
-#pragma unroll
-            for (int u4 = 0; u4 < kAttnChunk; u4 += 4) {
-                const float4 e4 = *reinterpret_cast<const float4 *>(es + h * kAttnChunk + u4);
-                const float e[4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (u4 + i < cnt) o = __fmaf_rn(e[i], vval(u4 + i), o);
-            }
-            part_o[((row * heads + h) * max_chunks + c) * kDecThreads + t] = o;
-        }
+        for (int u4 = 0; u4 < kAttnChunk; u4 += 4)
+            if (u4 < cnt) step4(u4, cnt - u4);
     }
+#pragma unroll
+    for (int g = 0; g < GH; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int h = (half + g) * 4 + i;
+            if (h < heads) part_o[((row * heads + h) * max_chunks + c) * kDecThreads + t] = o[g][i];
+        }
 }
 
-// The split launch: two halves of four heads while the grid fits the CUs once; the chunk's K
-// staged through LDS while the grid stays resident at that kernel's occupancy (its 44 KB of LDS
-// allows three blocks per CU), else each lane loads its own K segment (11 KB, eight blocks per
-// CU), which measured faster for grids of several rounds (E2B global layers at batch 32: 78.9
-// against 85.3 us; with V staged through LDS as well, the whole batch-32 step 2.872 against
-// 2.887 ms).
+// The split launch: two halves of four heads while the grid fits the CUs once (batch 1: 1.188 ms a
+// step, 1.238 with one half; 1.245 on the VALU products), else one half, three blocks per CU, with
+// non-temporal K and V (32 rows at position 4095, whole attention: 73 us, 80 with cached loads, 98
+// on the VALU products; cached loads stay better for the small grids: 1.188 against 1.209 ms).
+// Blocks of several chunks with the next chunk's loads in flight measured slower (85-91 us).
 template <bool PRO>
 static void launch_split(int chunks, int rows, hipStream_t st, const float *q, const float *k_cache,
                          const float *v_cache, int64_t cache_row_stride, int heads, int pos,
@@ -535,17 +489,13 @@ static void launch_split(int chunks, int rows, hipStream_t st, const float *q, c
     const int64_t blocks = (int64_t)chunks * rows, cus = device_cu_count();
     const dim3 grid(chunks, rows);
     if (blocks <= cus)
-        hipLaunchKernelGGL((attn_split_kernel<PRO, 2, true>), grid, dim3(2 * kDecThreads), 0, st,
-                           q, k_cache, v_cache, cache_row_stride, heads, pos, pos_dev, window,
-                           part_ml, part_o, chunks, pro);
-    else if (blocks <= 3 * cus)
-        hipLaunchKernelGGL((attn_split_kernel<PRO, 1, true>), grid, dim3(kDecThreads), 0, st, q,
-                           k_cache, v_cache, cache_row_stride, heads, pos, pos_dev, window, part_ml,
-                           part_o, chunks, pro);
+        hipLaunchKernelGGL((attn_split_kernel<PRO, 2>), grid, dim3(2 * kDecThreads), 0, st, q, k_cache,
+                           v_cache, cache_row_stride, heads, pos, pos_dev, window, part_ml, part_o,
+                           chunks, pro);
     else
-        hipLaunchKernelGGL((attn_split_kernel<PRO, 1, false>), grid, dim3(kDecThreads), 0, st, q,
-                           k_cache, v_cache, cache_row_stride, heads, pos, pos_dev, window, part_ml,
-                           part_o, chunks, pro);
+        hipLaunchKernelGGL((attn_split_kernel<PRO, 1>), grid, dim3(kDecThreads), 0, st, q, k_cache,
+                           v_cache, cache_row_stride, heads, pos, pos_dev, window, part_ml, part_o,
+                           chunks, pro);
 }
 
 // Thread d merges dim d of head h, row `row`, over the chunks in ascending order: M = max m_c,
