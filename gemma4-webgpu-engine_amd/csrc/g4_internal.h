@@ -439,6 +439,48 @@ __device__ __forceinline__ float gelu_act_value(const GeluAct &a, const void *ga
     return __fmul_rn(d_gelu(g), u);
 }
 
+// The snap of many activations on one scale, without a divide or a branch per value. With r =
+// RN(1 / s), two residual steps q += fma(-q, s, v) * r after q = v * r give the correctly rounded
+// quotient RN(v / s) (Markstein: the first makes q faithful, the second exact; the residuals are
+// exact for the |q| of 0.25 .. 129 that decide a code while 2^-100 <= s <= 2^100, `ok`; other
+// scales divide). The value is clamped first, to where the quotient still rounds to the end
+// codes, so an infinity takes no residual and a NaN lands on -128 (fmaxf drops it). 7 VALU
+// instructions per value; a test for quotients near half integers with a divide behind it was
+// taken by most waves on f16 input, whose exact ties are common (20 x at x = odd / 8).
+struct SrqScale {
+    float s, r, lo, hi;
+    bool ok;
+};
+__device__ __forceinline__ SrqScale srq_scale(float s) {
+    return SrqScale{s, __fdiv_rn(1.0f, s), __fmul_rn(-128.25f, s), __fmul_rn(127.25f, s),
+                    s >= 0x1p-100f && s <= 0x1p100f};
+}
+// v becomes a float within [-128.5, 127.5) that rounds (ties to even) to its code.
+__device__ __forceinline__ void srq_quot8(float (&v)[8], const SrqScale &S) {
+    if (S.ok) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float c = fminf(fmaxf(v[i], S.lo), S.hi);
+            float q = __fmul_rn(c, S.r);
+            q = __fmaf_rn(__fmaf_rn(-q, S.s, c), S.r, q);
+            v[i] = __fmaf_rn(__fmaf_rn(-q, S.s, c), S.r, q);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = srq_code_f(v[i], S.s);
+    }
+}
+
+// Four such values' codes as bytes a, b, c, d of a word: adding 1.5 * 2^23 rounds to the integer,
+// whose two's complement byte is then the sum's low byte.
+__device__ __forceinline__ uint32_t code_bytes(float a, float b, float c, float d) {
+    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(__fadd_rn(b, 12582912.0f)),
+                                              __float_as_uint(__fadd_rn(a, 12582912.0f)), 0x0C0C0400u);
+    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(__fadd_rn(d, 12582912.0f)),
+                                              __float_as_uint(__fadd_rn(c, 12582912.0f)), 0x0C0C0400u);
+    return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
+}
+
 // The closing expression of every quantized linear (qgemv.ts:1168-1172, :680-686), in its order:
 // one f32 multiply folds the input scale into the row scale, one more multiplies the reduced sum.
 __device__ __forceinline__ float linear_epilogue(float in_scale, float row_scale, float sum) {

@@ -38,10 +38,32 @@ int gemv_columns(int bits, const void *wq, const float *scales, const void *x, i
 constexpr int kQuantThreads = 256;
 constexpr int kTileBK = 128;
 
-__device__ __forceinline__ uint32_t pack4b(int a, int b, int c, int d) {
-    return (uint32_t)(a & 0xff) | ((uint32_t)(b & 0xff) << 8) | ((uint32_t)(c & 0xff) << 16) |
-           ((uint32_t)(d & 0xff) << 24);
+// An 8-code group as two words, interleaved [x0 x2 x4 x6 | x1 x3 x5 x7] when PERM.
+template <bool PERM> __device__ __forceinline__ uint2 codes_word2(const float (&c)[8]) {
+    return PERM ? make_uint2(code_bytes(c[0], c[2], c[4], c[6]), code_bytes(c[1], c[3], c[5], c[7]))
+                : make_uint2(code_bytes(c[0], c[1], c[2], c[3]), code_bytes(c[4], c[5], c[6], c[7]));
 }
+
+// Eight activations from one 16-byte load of f16 (widened exactly) or two of f32.
+template <bool F16> __device__ __forceinline__ void widen8(const u32x4 (&raw)[F16 ? 1 : 2], float (&v)[8]) {
+    if constexpr (F16) {
+        const uint32_t h[4] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = __half2float(__ushort_as_half((unsigned short)(h[i] & 0xffff)));
+            v[2 * i + 1] = __half2float(__ushort_as_half((unsigned short)(h[i] >> 16)));
+        }
+    } else {
+        const uint32_t w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
+    }
+}
+
+// q / d for q < 2^16 and a uniform d < 2^16, with m = fast_div_of(d): one multiply, where a
+// division by a run-time value costs about 20 instructions.
+__device__ __forceinline__ uint32_t fast_div_of(uint32_t d) { return 0xFFFFFFFFu / d + 1; }
+__device__ __forceinline__ int fast_div(int q, uint32_t m) { return (int)__umulhi((uint32_t)q, m); }
 
 constexpr int kQuantGroups = 4;  // 8-code groups per thread per pass, all loaded before any snap
 
@@ -52,8 +74,7 @@ constexpr int kQuantGroups = 4;  // 8-code groups per thread per pass, all loade
 template <bool PERM, bool F16>
 __global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(const void *x, int64_t n8,
                                                                       float scale, int8_t *codes) {
-    bool r_ok;
-    const float r = srq_recip(scale, r_ok);
+    const SrqScale S = srq_scale(scale);
     const int64_t stride = (int64_t)gridDim.x * kQuantThreads * kQuantGroups;
     for (int64_t g0 = (int64_t)blockIdx.x * kQuantThreads * kQuantGroups + threadIdx.x; g0 < n8;
          g0 += stride) {
@@ -70,31 +91,9 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(const void
             const int64_t g = g0 + (int64_t)u * kQuantThreads;
             if (g >= n8) break;
             float v[8];
-            if (F16) {
-                const uint32_t h[4] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[2 * i] = __half2float(__ushort_as_half((unsigned short)(h[i] & 0xffff)));
-                    v[2 * i + 1] = __half2float(__ushort_as_half((unsigned short)(h[i] >> 16)));
-                }
-            } else {
-                const uint32_t w[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w,
-                                       raw[u][F16 ? 0 : 1].x, raw[u][F16 ? 0 : 1].y,
-                                       raw[u][F16 ? 0 : 1].z, raw[u][F16 ? 0 : 1].w};
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
-            }
-            int c[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) c[i] = (int)srq_code_fast(v[i], scale, r, r_ok);
-            uint2 out;
-            if (PERM) {
-                out.x = pack4b(c[0], c[2], c[4], c[6]);
-                out.y = pack4b(c[1], c[3], c[5], c[7]);
-            } else {
-                out.x = pack4b(c[0], c[1], c[2], c[3]);
-                out.y = pack4b(c[4], c[5], c[6], c[7]);
-            }
+            widen8<F16>(raw[u], v);
+            srq_quot8(v, S);
+            const uint2 out = codes_word2<PERM>(v);
             reinterpret_cast<uint2 *>(codes)[g] = out;
         }
     }
@@ -153,41 +152,21 @@ __global__ __launch_bounds__(256) void qmatmul8_serial_kernel(
     store_linear_out(dst, (int64_t)col * n + row, out_kind, y, 0, out_scale);
 }
 
-// The B operand of one 16x16x64 step from 8 bytes (16 codes) of weights at `p`.
-template <int BITS>
-__device__ __forceinline__ v4i b_operand(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3,
-                                         int step) {
-    v4i b;
-    if (BITS == 4) {
-        const uint32_t a = step == 0 ? w0 : w2;
-        const uint32_t c = step == 0 ? w1 : w3;
-        b.x = (int)(a & 0x0F0F0F0Fu);
-        b.y = (int)((a >> 4) & 0x0F0F0F0Fu);
-        b.z = (int)(c & 0x0F0F0F0Fu);
-        b.w = (int)((c >> 4) & 0x0F0F0F0Fu);
-    } else {
-        (void)w2;
-        (void)w3;
-        b.x = (int)w0;
-        b.y = (int)w1;
-        b.z = (int)w2;
-        b.w = (int)w3;
-    }
-    return b;
-}
-
-__device__ __forceinline__ void store_tile_out(void *dst, int m, int n, int N, int out_kind,
-                                               int acc, float in_scale, float scale,
-                                               float out_scale) {
-    const float y = linear_epilogue(in_scale, scale, (float)acc);
-    store_linear_out(dst, (int64_t)m * N + n, out_kind, y, acc, out_scale);
-}
+// The two halves of a weight word's eight 4-bit codes, times 16, as signed bytes: with w' = w ^
+// 0x88888888, (w' << 4) & 0xF0F0F0F0 holds the even codes and w' & 0xF0F0F0F0 the odd ones. The
+// accumulator is then 16 * sum(code * x), exact (|sum| <= 2^31 / 16 for K <= 16384), with no
+// zero-point term to take off.
+__device__ __forceinline__ uint32_t nib_even16(uint32_t w) { return ((w ^ 0x88888888u) << 4) & 0xF0F0F0F0u; }
+__device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x88888888u) & 0xF0F0F0F0u; }
 
 // ---- small M: M <= MT token rows, 16 weight rows per block, K split over the block's waves ------
 // The activation snap is fused: the block snaps its MT token rows into LDS as int8 codes (the
 // 4-bit interleave per 8-code group) one K chunk at a time, so a draft-verify or small prefill
-// call is one launch. The 4-bit zero point needs sum(xq) per token row: one more MFMA per step
-// against an all-ones B operand gives it exactly, folded with the partials like the products.
+// call is one launch. 4-bit weights are taken as 16 * code (nib_even16): no zero-point sums, so half
+// the MFMAs and half the partials in the fold of a form with a row-sum product per step. Bound:
+// the chain of launch, codes, MFMAs and fold (int8 codes, us in a graph, before -> now: 16 x 1536 ->
+// 6144 5.6 -> 5.2, 32 x 6144 -> 1536 10.3 -> 9.2, 32 x 1536 -> 256 4.4 -> 3.7; with f16 x snapped
+// here 12 x 1536 -> 2048 5.9 -> 4.5, 32 x 1536 -> 256 10.6 -> 6.6).
 // Lane (j = lane % 16, g = lane / 16) owns weight row n0 + j; per 128-code stage it loads 16 bytes
 // of that row (8-bit: 32), and MFMA half-step s takes codes g*32 + s*16 .. +16 of the stage from
 // both operands. The LDS rows are padded by 16 bytes so the 16 token rows of one A read fall on
@@ -256,7 +235,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     constexpr int XSTR = KC + 16;              // LDS bytes per token row
     constexpr int BATCH = WAVES >= 16 ? 1 : 4;
     constexpr int NP = EPI == 1 ? 2 : 1;             // product sets: the gate's (and the up's)
-    constexpr int NACC = BITS == 4 ? (NP + 1) * TM : NP * TM;  // products, then the row sums
+    constexpr int NACC = NP * TM;
+    constexpr int SHIFT = BITS == 4 ? 4 : 0;         // 4-bit sums are of 16 * code
     // the codes during the K loop, and every wave's partial tiles for the fold: in a region of
     // their own when both fit (two blocks of 4 waves per CU, or one of 16), so the fold needs no
     // barrier for the last reads of the codes; else over the codes' bytes
@@ -292,8 +272,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     const int row_bytes = BITS == 4 ? (K >> 1) : K;
     const uint8_t *wrow = W + (int64_t)n * row_bytes;
     const uint8_t *wrow2 = EPI == 1 ? jobs.w_up + (int64_t)n * row_bytes : wrow;
-    bool r_ok;
-    const float rcp = srq_recip(in_scale, r_ok);
+    const SrqScale S = srq_scale(in_scale);
     // the epilogue's per-output operands (row scales; the paired up rows' scales; the f32 up
     // vector), requested now so the epilogue does not wait a memory round trip for them
     constexpr int EQ = (TM * 256 + THREADS - 1) / THREADS;  // outputs per thread
@@ -311,7 +290,6 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     v4i acc[NACC];
 #pragma unroll
     for (int t = 0; t < NACC; ++t) acc[t] = v4i{0, 0, 0, 0};
-    const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
     // ksplit > 0: block z takes codes [z ksplit, (z + 1) ksplit) of K and stores its int32 partial
     // accumulator (out_kind int32) to dst[z][M][N]; the splits' sum is the exact accumulator
@@ -330,9 +308,10 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
         load_small_weights<BITS, NP, BATCH, WAVES>(bw_first, wrow, wrow2, wave, ksteps, kbase, g);
         lds_barrier();  // the previous chunk's codes are no longer read
         // the snap: each thread issues the loads of SB groups (indices clamped, so every load is
-        // valid) before converting any, so a chunk costs one memory latency per SB groups. Only
-        // the block's real token rows are snapped: a padding row's LDS codes reach only the
-        // products of its own output row, which is never stored.
+        // valid) before converting any, so a chunk costs one memory latency per SB groups; one
+        // loop per input type, since a load in one arm of a branch inside the loop is waited for
+        // there. Only the block's real token rows are snapped: a padding row's LDS codes reach
+        // only the products of its own output row, which is never stored.
         constexpr int SB = 4;
         const int total = min(MT, M - m0) * gpr;
         if (x_kind == G4_KIND_I8) {
@@ -340,12 +319,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
             // once, then a byte permute per 8-code group for 4-bit weights
             constexpr int U16 = (MT * KC / 16 + THREADS - 1) / THREADS;
             const int upr = kcn >> 4, total16 = min(MT, M - m0) * upr;
+            const uint32_t upr_m = fast_div_of(upr);
             u32x4 raw[U16];
             int rr[U16], uu[U16];
 #pragma unroll
             for (int u = 0; u < U16; ++u) {
                 const int q = min(tid + u * THREADS, total16 - 1);
-                rr[u] = q / upr;
+                rr[u] = fast_div(q, upr_m);
                 uu[u] = q - rr[u] * upr;
                 raw[u] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const int8_t *>(x) +
                                                           (int64_t)(m0 + rr[u]) * K + kc0 + uu[u] * 16);
@@ -363,68 +343,34 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
                 *reinterpret_cast<u32x4 *>(&xs[rr[u] * XSTR + uu[u] * 16]) = o;
             }
         }
-        for (int q0 = tid; x_kind != G4_KIND_I8 && q0 < total; q0 += SB * THREADS) {
-            u32x4 raw_a[SB], raw_b[SB];
-            int rr[SB], gg[SB];  // row and group of each load, kept for the stores (one divide)
+        auto snap = [&](auto f16c) {
+            constexpr bool F16 = decltype(f16c)::value;
+            const uint32_t gpr_m = fast_div_of(gpr);
+            for (int q0 = tid; q0 < total; q0 += SB * THREADS) {
+                u32x4 raw[SB][F16 ? 1 : 2];
+                int rr[SB], gg[SB];  // row and group of each load, kept for the stores
 #pragma unroll
-            for (int u = 0; u < SB; ++u) {
-                const int q = min(q0 + u * THREADS, total - 1);
-                const int r = q / gpr, gi = q - r * gpr;
-                rr[u] = r;
-                gg[u] = gi;
-                const int64_t e = (int64_t)(m0 + r) * K + kc0 + gi * 8;
-                if (x_kind == G4_KIND_I8) {
-                    const uint2 v = *reinterpret_cast<const uint2 *>(reinterpret_cast<const int8_t *>(x) + e);
-                    raw_a[u] = u32x4{v.x, v.y, 0u, 0u};
-                    raw_b[u] = u32x4{0u, 0u, 0u, 0u};
-                } else if (x_kind == G4_KIND_F16) {
-                    raw_a[u] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const __half *>(x) + e);
-                    raw_b[u] = u32x4{0u, 0u, 0u, 0u};
-                } else {
-                    const u32x4 *p4 = reinterpret_cast<const u32x4 *>(reinterpret_cast<const float *>(x) + e);
-                    raw_a[u] = p4[0];
-                    raw_b[u] = p4[1];
+                for (int u = 0; u < SB; ++u) {
+                    const int q = min(q0 + u * THREADS, total - 1);
+                    rr[u] = fast_div(q, gpr_m);
+                    gg[u] = q - rr[u] * gpr;
+                    const int64_t e = (int64_t)(m0 + rr[u]) * K + kc0 + gg[u] * 8;
+                    const u32x4 *p4 = reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(x) + e * (F16 ? 2 : 4));
+#pragma unroll
+                    for (int h = 0; h < (F16 ? 1 : 2); ++h) raw[u][h] = p4[h];
+                }
+#pragma unroll
+                for (int u = 0; u < SB; ++u) {
+                    if (q0 + u * THREADS >= total) break;
+                    float v[8];
+                    widen8<F16>(raw[u], v);
+                    srq_quot8(v, S);
+                    *reinterpret_cast<uint2 *>(&xs[rr[u] * XSTR + gg[u] * 8]) = codes_word2<BITS == 4>(v);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < SB; ++u) {
-                if (q0 + u * THREADS >= total) break;
-                const int r = rr[u], gi = gg[u];
-                int c[8];
-                {
-                    if (x_kind == G4_KIND_I8) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            c[i] = (int)(int8_t)((raw_a[u].x >> (8 * i)) & 0xff);
-                            c[4 + i] = (int)(int8_t)((raw_a[u].y >> (8 * i)) & 0xff);
-                        }
-                    } else if (x_kind == G4_KIND_F16) {
-                        const uint32_t h[4] = {raw_a[u].x, raw_a[u].y, raw_a[u].z, raw_a[u].w};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            c[2 * i] = (int)srq_code_fast(
-                                __half2float(__ushort_as_half((unsigned short)(h[i] & 0xffff))), in_scale, rcp, r_ok);
-                            c[2 * i + 1] = (int)srq_code_fast(
-                                __half2float(__ushort_as_half((unsigned short)(h[i] >> 16))), in_scale, rcp, r_ok);
-                        }
-                    } else {
-                        const uint32_t v[8] = {raw_a[u].x, raw_a[u].y, raw_a[u].z, raw_a[u].w,
-                                               raw_b[u].x, raw_b[u].y, raw_b[u].z, raw_b[u].w};
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) c[i] = (int)srq_code_fast(__uint_as_float(v[i]), in_scale, rcp, r_ok);
-                    }
-                }
-                uint2 packed;
-                if (BITS == 4) {
-                    packed.x = pack4b(c[0], c[2], c[4], c[6]);
-                    packed.y = pack4b(c[1], c[3], c[5], c[7]);
-                } else {
-                    packed.x = pack4b(c[0], c[1], c[2], c[3]);
-                    packed.y = pack4b(c[4], c[5], c[6], c[7]);
-                }
-                *reinterpret_cast<uint2 *>(&xs[r * XSTR + gi * 8]) = packed;
-            }
-        }
+        };
+        if (x_kind == G4_KIND_F16) snap(std::true_type{});
+        else if (x_kind != G4_KIND_I8) snap(std::false_type{});
         lds_barrier();
         for (int kb0 = wave; kb0 < ksteps; kb0 += WAVES * BATCH) {
             u32x4 bw[NP][BATCH][BITS == 4 ? 1 : 2];
@@ -460,11 +406,14 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
                         v4i b[NP];
 #pragma unroll
                         for (int p = 0; p < NP; ++p) {
-                            if (BITS == 4)
-                                b[p] = b_operand<4>(bw[p][u][0].x, bw[p][u][0].y, bw[p][u][0].z,
-                                                    bw[p][u][0].w, s);
-                            else
+                            if (BITS == 4) {
+                                const uint32_t wa = s == 0 ? bw[p][u][0].x : bw[p][u][0].z;
+                                const uint32_t wb = s == 0 ? bw[p][u][0].y : bw[p][u][0].w;
+                                b[p] = v4i{(int)nib_even16(wa), (int)nib_odd16(wa), (int)nib_even16(wb),
+                                           (int)nib_odd16(wb)};
+                            } else {
                                 b[p] = __builtin_bit_cast(v4i, bw[p][u][BITS == 4 ? 0 : s]);
+                            }
                         }
 #pragma unroll
                         for (int t = 0; t < TM; ++t) {
@@ -473,9 +422,6 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
                             for (int p = 0; p < NP; ++p)
                                 acc[p * TM + t] =
                                     __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[p], acc[p * TM + t], 0, 0, 0);
-                            if (BITS == 4)  // each code counted once: both halves
-                                acc[NP * TM + t] =
-                                    __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ones, acc[NP * TM + t], 0, 0, 0);
                         }
                     }
                 }
@@ -505,17 +451,14 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
         const int lr = t * 16 + 4 * (ln >> 4) + r;
         const int m = m0 + lr, nn = n0 + (ln & 15);
         if (m >= M || nn >= N) continue;
-        int v = 0, v2 = 0, rsum = 0;
+        int v = 0, v2 = 0;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
             v += reinterpret_cast<const int *>(&red[w][t][ln])[r];
             if (EPI == 1) v2 += reinterpret_cast<const int *>(&red[w][TM + t][ln])[r];
-            if (BITS == 4) rsum += reinterpret_cast<const int *>(&red[w][NP * TM + t][ln])[r];
         }
-        if (BITS == 4) {  // the ones product: sum(xq) of row lr
-            v -= 8 * rsum;
-            v2 -= 8 * rsum;
-        }
+        v >>= SHIFT;
+        v2 >>= SHIFT;
         const float yv = __fmul_rn(__fmul_rn(in_scale, e_scale[e]), (float)v);
         const int64_t o = (int64_t)m * N + nn;
         if (EPI != 0) {  // gelu(gate) * up, snapped for the consumer
@@ -602,8 +545,6 @@ template <int DPS, int L = 0> __device__ __forceinline__ void tile_wait_stages(i
     }
 }
 
-__device__ __forceinline__ uint32_t nib_even16(uint32_t w) { return ((w ^ 0x88888888u) << 4) & 0xF0F0F0F0u; }
-__device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x88888888u) & 0xF0F0F0F0u; }
 // Eight packed codes c0..c7 (one weight word) as 16 x code signed bytes in natural order: the even
 // and odd nibble bytes [c0 c2 c4 c6] and [c1 c3 c5 c7] interleaved by two byte permutes into
 // [c0 c1 c2 c3] and [c4 c5 c6 c7], so the activation codes need no interleave.
@@ -1448,12 +1389,17 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
     return G4_OK;
 }
 
-// The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past about
-// 4 Mi snaps in total (M * K per block times the blocks along N), one snap pass over the M * K
-// activations into a buffer of codes, then the kernel on int8 codes, costs less (config 2: M = 8,
-// K = 1536 over 384 blocks is 4.7 Mi).
+// The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past 48 Ki snaps
+// on the busiest CU (M * K per block, times its blocks there), one snap pass over the M * K
+// activations into a buffer of codes, then the kernel on int8 codes, costs less. Fused against
+// passed, us in a graph: 8 x 1536 -> 6144 (24 Ki) 6.1 / 7.0, 12 x 1536 -> 6144 (36 Ki) 7.1 / 7.4,
+// 24 x 1536 -> 2048 (36 Ki) 5.6 / 6.4, 16 x 1536 -> 6144 (48 Ki) 7.8 / 7.6, 8 x 6144 -> 1536 (48 Ki)
+// 8.1 / 8.0, 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
+// fused (its capture contract: it needs no buffer that an earlier call must have made).
 static bool small_presnap(int m, int n, int k) {
-    return (int64_t)m * k * ((n + 15) / 16) >= ((int64_t)1 << 22);
+    const int64_t cus = device_cu_count();
+    const int64_t blocks = (n + 15) / 16;  // M <= 32: one block row
+    return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && (blocks + cus - 1) / cus * m * k >= 48 * 1024;
 }
 
 // Whether a call snaps f16 / f32 activations into a buffer of M * K codes first (the tile kernels,
