@@ -2,6 +2,7 @@
 // fill kernel and the pure table split planner (src/tableSplit.ts).
 #include "g4_internal.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <mutex>
 #include <vector>
@@ -277,12 +278,71 @@ int captured_node_refusal(hipGraph_t graph) {
 }  // namespace
 
 // The handle of a captured graph: the executable and an event recorded after each launch, so
-// destroy waits for this graph's own replays and nothing else on the device.
+// destroy waits for this graph's own replays and nothing else on the device. A short chain of
+// kernels is replayed as its kernel launches (`chain`, the graph's nodes in order; the arguments
+// live in `graph`): hipGraphLaunch costs 14-15 us of host time whatever it launches, a kernel
+// launch 2.3 us.
 struct G4Graph {
     hipGraphExec_t exec = nullptr;
+    hipGraph_t graph = nullptr;
     hipEvent_t done = nullptr;
     bool launched = false;
+    int device = 0;
+    std::vector<hipKernelNodeParams> chain;
 };
+
+// Where kernel launches stop being cheaper than one graph launch. Us a replay with its event, as
+// launches / as a graph launch: empty kernels, 1: 5.1 / 15.3, 3: 8.5 / 15, 8: 18.5 / 24 (2.3 against
+// 1.7 per further kernel, so even near 16); a layer's seven linears at 8 tokens 37.6 / 45.0, split
+// attention of 32 rows (3 kernels) 64.8 / 72.3 (a graph launch starts about 7 us after the work
+// before it). At 183 and 393 kernels (the decode step) the two differ by under 1% and one graph
+// launch takes less host time.
+constexpr size_t kChainMax = 12;
+
+// One launch is one unit of its stream's order also where several threads launch on it.
+static std::mutex &launch_lock(void *stream) {
+    static std::mutex locks[16];
+    return locks[(reinterpret_cast<uintptr_t>(stream) >> 6) % 16];
+}
+
+// The nodes of `graph` in order when it is one chain of at most kChainMax ordinary kernels (each
+// known to the runtime by its host symbol, launched without attributes), else empty.
+static std::vector<hipKernelNodeParams> kernel_chain(hipGraph_t graph) {
+    const std::vector<hipKernelNodeParams> none;
+    size_t n = 0, ne = 0;
+    if (hipGraphGetNodes(graph, nullptr, &n) != hipSuccess || n == 0 || n > kChainMax) return none;
+    std::vector<hipGraphNode_t> nodes(n);
+    if (hipGraphGetNodes(graph, nodes.data(), &n) != hipSuccess) return none;
+    if (hipGraphGetEdges(graph, nullptr, nullptr, &ne) != hipSuccess || ne != n - 1) return none;
+    std::vector<hipGraphNode_t> from(ne), to(ne);
+    if (ne && hipGraphGetEdges(graph, from.data(), to.data(), &ne) != hipSuccess) return none;
+    // the one node that no edge enters, then along the edges; n - 1 edges that reach all n nodes
+    // in one walk are a chain
+    std::vector<hipKernelNodeParams> chain;
+    hipGraphNode_t at = nullptr;
+    for (hipGraphNode_t c : nodes)
+        if (std::find(to.begin(), to.end(), c) == to.end()) at = c;
+    while (at && chain.size() < n) {
+        hipGraphNodeType type;
+        hipKernelNodeParams kp{};
+        hipFunction_t fn = nullptr;
+        hipKernelNodeAttrValue coop{};
+        if (hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
+            hipGraphKernelNodeGetParams(at, &kp) != hipSuccess || !kp.func || !kp.kernelParams || kp.extra ||
+            hipGetFuncBySymbol(&fn, kp.func) != hipSuccess ||
+            hipGraphKernelNodeGetAttribute(at, hipKernelNodeAttributeCooperative, &coop) != hipSuccess ||
+            coop.cooperative) {
+            (void)hipGetLastError();
+            return none;
+        }
+        chain.push_back(kp);
+        hipGraphNode_t next = nullptr;
+        for (size_t i = 0; i < ne; ++i)
+            if (from[i] == at) next = to[i];
+        at = next;
+    }
+    return chain.size() == n ? chain : none;
+}
 
 int g4_graph_end_capture(void *stream, void **graph_exec) {
     if (!stream || !graph_exec) return set_error(G4_ERR_INVALID, "g4_graph_end_capture: NULL argument");
@@ -301,17 +361,26 @@ int g4_graph_end_capture(void *stream, void **graph_exec) {
     }
     hipGraphExec_t exec = nullptr;
     hipError_t err = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (err != hipSuccess) return hip_status(err, "hipGraphInstantiate");
+    if (err != hipSuccess) {
+        (void)hipGraphDestroy(graph);
+        return hip_status(err, "hipGraphInstantiate");
+    }
+    // The event only tells destroy that the replay is over: no system-scope fence (1 us less on the
+    // device per replay).
     hipEvent_t done = nullptr;
-    err = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+    err = hipEventCreateWithFlags(&done, hipEventDisableTiming | hipEventDisableSystemFence);
     if (err != hipSuccess) {
         (void)hipGraphExecDestroy(exec);
+        (void)hipGraphDestroy(graph);
         return hip_status(err, "hipEventCreateWithFlags");
     }
     G4Graph *g = new G4Graph;
     g->exec = exec;
     g->done = done;
+    g->chain = kernel_chain(graph);
+    if (hipGetDevice(&g->device) != hipSuccess) g->chain.clear();
+    if (g->chain.empty()) (void)hipGraphDestroy(graph);
+    else g->graph = graph;
     *graph_exec = g;
     return G4_OK;
 }
@@ -319,7 +388,23 @@ int g4_graph_end_capture(void *stream, void **graph_exec) {
 int g4_graph_launch(void *graph_exec, void *stream) {
     if (!graph_exec) return set_error(G4_ERR_INVALID, "g4_graph_launch: no graph");
     G4Graph *g = static_cast<G4Graph *>(graph_exec);
-    G4_HIP(hipGraphLaunch(g->exec, as_stream(stream)));
+    bool direct = !g->chain.empty();
+    if (direct) {
+        // on a capturing stream, or with another device current, it stays a graph launch
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        int dev = -1;
+        G4_HIP(hipStreamIsCapturing(as_stream(stream), &st));
+        G4_HIP(hipGetDevice(&dev));
+        direct = st == hipStreamCaptureStatusNone && dev == g->device;
+    }
+    std::lock_guard<std::mutex> lock(launch_lock(stream));
+    if (direct) {
+        for (const hipKernelNodeParams &k : g->chain)
+            G4_HIP(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes,
+                                   as_stream(stream)));
+    } else {
+        G4_HIP(hipGraphLaunch(g->exec, as_stream(stream)));
+    }
     G4_HIP(hipEventRecord(g->done, as_stream(stream)));
     g->launched = true;
     return G4_OK;
@@ -335,6 +420,7 @@ int g4_graph_destroy(void *graph_exec) {
     hipError_t wait = g->launched ? hipEventSynchronize(g->done) : hipSuccess;
     hipError_t d1 = hipGraphExecDestroy(g->exec);
     hipError_t d2 = hipEventDestroy(g->done);
+    if (g->graph) (void)hipGraphDestroy(g->graph);
     delete g;
     if (wait != hipSuccess) return hip_status(wait, "g4_graph_destroy: waiting for the last launch");
     if (d1 != hipSuccess) return hip_status(d1, "hipGraphExecDestroy");

@@ -1,0 +1,52 @@
+"""Graph replays around the length where a chain of kernels stops being replayed as its launches:
+every replay against the eager result with eager work between, and destroy waiting for the last
+replay."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kernels", [1, 2, 11, 12, 13, 40])
+def test_chain_lengths(gpu, kernels):
+    print(f"graph chain of {kernels} kernels", flush=True)
+    st = gpu.Stream()
+    n = 4096
+    x = gpu.DeviceBuffer.from_array(np.linspace(-8, 8, n, dtype=np.float32))
+    outs = [gpu.DeviceBuffer.empty((n,), np.int8) for _ in range(kernels)]
+
+    def record():
+        for i, o in enumerate(outs):
+            gpu.srq_quantize(x, o, n, 0.05 * (i + 1), stream=st.handle)
+
+    g = gpu.Graph(st, record)
+    for rep in range(3):
+        xs = np.linspace(-8 - rep, 8 + rep, n, dtype=np.float32)
+        x.upload(xs)
+        for o in outs:
+            o.fill(0x7B, st.handle)  # eager work between replays
+        g.launch()
+        st.synchronize()
+        for i, o in enumerate(outs):
+            s = np.float32(0.05 * (i + 1))
+            want = np.clip(np.rint(xs / s), -128, 127).astype(np.int8)
+            assert np.array_equal(o.download(), want), (rep, i)
+    g.close()
+    st.close()
+
+
+@pytest.mark.parametrize("kernels", [4, 20])
+def test_destroy_waits_for_the_last_replay(gpu, kernels):
+    print(f"graph of {kernels} fills destroyed right after its launch", flush=True)
+    st, other = gpu.Stream(), gpu.Stream()
+    n = 64 << 20
+    b = gpu.DeviceBuffer.empty((n,), np.uint8)
+    b.fill(0)
+    gpu.synchronize()
+    g = gpu.Graph(st, lambda: [b.fill(i + 1, st.handle) for i in range(kernels)])
+    g.launch()
+    g.close()
+    got = b.download(other.handle)  # another stream: only the destroy's wait orders this read
+    assert np.all(got == kernels)
+    st.close()
+    other.close()
