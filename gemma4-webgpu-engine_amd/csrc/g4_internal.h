@@ -481,6 +481,28 @@ __device__ __forceinline__ uint32_t code_bytes(float a, float b, float c, float 
     return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
 }
 
+// An 8-code group as two words, interleaved [x0 x2 x4 x6 | x1 x3 x5 x7] when PERM.
+template <bool PERM> __device__ __forceinline__ uint2 codes_word2(const float (&c)[8]) {
+    return PERM ? make_uint2(code_bytes(c[0], c[2], c[4], c[6]), code_bytes(c[1], c[3], c[5], c[7]))
+                : make_uint2(code_bytes(c[0], c[1], c[2], c[3]), code_bytes(c[4], c[5], c[6], c[7]));
+}
+
+// Eight activations from one 16-byte load of f16 (widened exactly) or two of f32.
+template <bool F16> __device__ __forceinline__ void widen8(const u32x4 (&raw)[F16 ? 1 : 2], float (&v)[8]) {
+    if constexpr (F16) {
+        const uint32_t h[4] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = __half2float(__ushort_as_half((unsigned short)(h[i] & 0xffff)));
+            v[2 * i + 1] = __half2float(__ushort_as_half((unsigned short)(h[i] >> 16)));
+        }
+    } else {
+        const uint32_t w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
+    }
+}
+
 // The closing expression of every quantized linear (qgemv.ts:1168-1172, :680-686), in its order:
 // one f32 multiply folds the input scale into the row scale, one more multiplies the reduced sum.
 __device__ __forceinline__ float linear_epilogue(float in_scale, float row_scale, float sum) {

@@ -38,28 +38,6 @@ int gemv_columns(int bits, const void *wq, const float *scales, const void *x, i
 constexpr int kQuantThreads = 256;
 constexpr int kTileBK = 128;
 
-// An 8-code group as two words, interleaved [x0 x2 x4 x6 | x1 x3 x5 x7] when PERM.
-template <bool PERM> __device__ __forceinline__ uint2 codes_word2(const float (&c)[8]) {
-    return PERM ? make_uint2(code_bytes(c[0], c[2], c[4], c[6]), code_bytes(c[1], c[3], c[5], c[7]))
-                : make_uint2(code_bytes(c[0], c[1], c[2], c[3]), code_bytes(c[4], c[5], c[6], c[7]));
-}
-
-// Eight activations from one 16-byte load of f16 (widened exactly) or two of f32.
-template <bool F16> __device__ __forceinline__ void widen8(const u32x4 (&raw)[F16 ? 1 : 2], float (&v)[8]) {
-    if constexpr (F16) {
-        const uint32_t h[4] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[2 * i] = __half2float(__ushort_as_half((unsigned short)(h[i] & 0xffff)));
-            v[2 * i + 1] = __half2float(__ushort_as_half((unsigned short)(h[i] >> 16)));
-        }
-    } else {
-        const uint32_t w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i]);
-    }
-}
-
 // q / d for q < 2^16 and a uniform d < 2^16, with m = fast_div_of(d): one multiply, where a
 // division by a run-time value costs about 20 instructions.
 __device__ __forceinline__ uint32_t fast_div_of(uint32_t d) { return 0xFFFFFFFFu / d + 1; }

@@ -159,29 +159,29 @@ __device__ __forceinline__ RawGroup<KIND> load_group(const void *x, int g) {
     return r;
 }
 
+// The group's codes as two words, in the job's layout (interleaved for 4-bit weights).
 template <int KIND>
-__device__ __forceinline__ void group_codes(const RawGroup<KIND> &r, float s, float rcp, bool r_ok,
-                                            int c[8]) {
-    if (KIND == G4_KIND_F32) {
-        const uint32_t v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) c[i] = (int)srq_code_fast(__uint_as_float(v[i]), s, rcp, r_ok);
-    } else if (KIND == G4_KIND_F16) {
-        const uint32_t w[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            c[2 * i] = (int)srq_code_fast(
-                __half2float(__ushort_as_half((unsigned short)(w[i] & 0xffff))), s, rcp, r_ok);
-            c[2 * i + 1] = (int)srq_code_fast(
-                __half2float(__ushort_as_half((unsigned short)(w[i] >> 16))), s, rcp, r_ok);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            c[i] = (int)(int8_t)((r.a.x >> (8 * i)) & 0xff);
-            c[4 + i] = (int)(int8_t)((r.a.y >> (8 * i)) & 0xff);
-        }
+__device__ __forceinline__ uint2 group_codes(const RawGroup<KIND> &r, const SrqScale &S, bool four) {
+    if (KIND == G4_KIND_I8) {
+        return four ? make_uint2(__builtin_amdgcn_perm(r.a.y, r.a.x, 0x06040200u),
+                                 __builtin_amdgcn_perm(r.a.y, r.a.x, 0x07050301u))
+                    : make_uint2(r.a.x, r.a.y);
     }
+    float v[8];
+    if constexpr (KIND == G4_KIND_F16) {
+        const u32x4 raw[1] = {r.a};
+        widen8<true>(raw, v);
+    } else {
+        const u32x4 raw[2] = {r.a, r.b};
+        widen8<false>(raw, v);
+    }
+    srq_quot8(v, S);
+    return four ? codes_word2<true>(v) : codes_word2<false>(v);
+}
+
+// The sum of a group's eight codes.
+__device__ __forceinline__ int word2_sum(uint2 w) {
+    return __builtin_amdgcn_sdot4((int)w.y, 0x01010101, __builtin_amdgcn_sdot4((int)w.x, 0x01010101, 0, false), false);
 }
 
 // The snap body for one activation kind: each thread issues the loads of a batch of groups
@@ -189,9 +189,7 @@ __device__ __forceinline__ void group_codes(const RawGroup<KIND> &r, float s, fl
 // memory latency per batch rather than one per group.
 template <int KIND>
 __device__ __forceinline__ int snap_kind(const StreamJob &J, uint8_t *xs, int tid) {
-    bool r_ok;
-    const float s = J.in_scale;
-    const float rcp = srq_recip(s, r_ok);
+    const SrqScale S = srq_scale(J.in_scale);
     const int groups = J.k >> 3;
     int local = 0;
     constexpr int B = snap_batch<KIND>();
@@ -204,18 +202,9 @@ __device__ __forceinline__ int snap_kind(const StreamJob &J, uint8_t *xs, int ti
         for (int i = 0; i < B; ++i) {
             const int g = g0 + i * kStreamThreads;
             if (g < groups) {
-                int c[8];
-                group_codes<KIND>(raw[i], s, rcp, r_ok, c);
-                uint2 packed;
-                if (J.bits == 4) {
-                    packed.x = pack_bytes(c[0], c[2], c[4], c[6]);
-                    packed.y = pack_bytes(c[1], c[3], c[5], c[7]);
-                } else {
-                    packed.x = pack_bytes(c[0], c[1], c[2], c[3]);
-                    packed.y = pack_bytes(c[4], c[5], c[6], c[7]);
-                }
+                const uint2 packed = group_codes<KIND>(raw[i], S, J.bits == 4);
                 *reinterpret_cast<uint2 *>(xs + g * 8) = packed;
-                local += c[0] + c[1] + c[2] + c[3] + c[4] + c[5] + c[6] + c[7];
+                local += word2_sum(packed);
             }
         }
     }
