@@ -14,11 +14,12 @@
 //
 // Kernels by M (chosen per shape, see pick_kernel):
 //   M <= 2         the GEMV family (qgemv.hip): bit-identical, cheaper than any tile at this M.
-//   3 <= M <= 32   qgemm_small_kernel: one launch with the snap fused (codes in LDS), 16 weight
+//   3 <= M <= 32, and more rows while one block of 32 rows x 16 columns per CU covers the output
+//                  qgemm_small_kernel: one launch with the snap fused (codes in LDS), 16 weight
 //                  rows per block, the block's waves split K (4, or 16 when the grid is no wider
 //                  than the CU count), an LDS fold of the partials; several projections of the
 //                  same x can share one grid (linear_grouped).
-//   M > 32, or over 32768+ rows
+//   larger outputs, or over 32768+ rows
 //                  qgemm_tile_kernel: 64 x 96 output tiles, activation codes and weights streamed
 //                  global -> LDS by direct loads through a 3-4 stage ring, XCD-aware tile order.
 #include "g4_internal.h"
@@ -534,11 +535,13 @@ __device__ __forceinline__ void nib_natural16(uint32_t w, int &lo, int &hi) {
 
 // NAT (4-bit): A holds natural-order codes and B is permuted to match in registers; otherwise A is
 // the per-8 interleaved row the nibble lanes read directly (no permutes).
+// KS: groups of four waves, each with its own ring; group kg takes stages kg, kg + KS, ... and the
+// epilogue adds the groups' sums (int32, exact).
 // BM: 64 tile rows (each wave 32 x 48), or 32 (each wave 16 x 48) for grids that would leave CUs
 // idle at 64: a block keeps about as many bytes in flight as the CU allows, so the launch's
 // bandwidth grows with the number of CUs it occupies.
-template <int BITS, int NS, bool NAT, int BM = kTileBM>
-__global__ __launch_bounds__(256) void qgemm_tile_kernel(
+template <int BITS, int NS, bool NAT, int BM, int KS>
+__global__ __launch_bounds__(256 * KS) void qgemm_tile_kernel(
     const int8_t *__restrict__ A, const uint8_t *__restrict__ W, const float *__restrict__ scales,
     void *dst, int M, int N, int K, float in_scale, float out_scale, int out_kind, int tiles_m,
     int tiles_n) {
@@ -550,9 +553,9 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     constexpr int B_INS = B_BYTES / 1024, B_PW = (B_INS + 3) / 4;
     constexpr int DPS = A_PW + B_PW;
     constexpr int ESTR = kTileEpiStride;
-    static_assert(NS >= 3 && NS * SB <= 160 * 1024, "ring depth");
+    static_assert(NS >= 3 && KS * NS * SB <= 160 * 1024, "ring depth");
     static_assert(NS * SB >= BM * ESTR * 4 + BN * 4, "the epilogue staging fits the ring");
-    __shared__ __align__(1024) uint8_t smem[NS * SB];
+    __shared__ __align__(1024) uint8_t smem_all[KS * NS * SB];
 
     // Blocks go to the 8 XCDs round robin; one XCD gets every M tile of a run of N tiles, so its L2
     // fetches those weight columns once.
@@ -565,7 +568,9 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     // the epilogue's column scale, requested now so the epilogue does not wait a memory round trip
     const float col_scale = tid < BN ? scales[min(n0 + tid, N - 1)] : 0.0f;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;  // in its group
+    const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    uint8_t *smem = smem_all + kg * (NS * SB);  // the group's ring
     const int j = lane & 15, g = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
     const int row_bytes = BITS == 4 ? K >> 1 : K;
@@ -604,9 +609,9 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     auto issue = [&](int st, int buf) {
         const uint32_t base = sbase + buf * SB;
 #pragma unroll
-        for (int i = 0; i < A_PW; ++i) lds_dma16(asrc[i] + st * 128, base + adst[i]);
+        for (int i = 0; i < A_PW; ++i) lds_dma16(asrc[i] + (st * KS + kg) * 128, base + adst[i]);
 #pragma unroll
-        for (int i = 0; i < B_PW; ++i) lds_dma16(bsrc[i] + st * BROW, base + bdst[i]);
+        for (int i = 0; i < B_PW; ++i) lds_dma16(bsrc[i] + (st * KS + kg) * BROW, base + bdst[i]);
     };
     // LDS byte offsets of this lane's operands inside a stage buffer.
     const int sig = (j & 7) ^ ((j >> 3) & 1);
@@ -676,7 +681,7 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     };
 
     // nk >= NS - 1 (the host picks NS). Stages 0 .. NS-2 in flight, then stage 0's operands.
-    const int nk = K >> 7;
+    const int nk = (K >> 7) / KS;  // the group's stages
 #pragma unroll
     for (int st = 0; st < NS - 1; ++st) issue(st, st);
     tile_wait_stages<DPS>(NS - 2);
@@ -718,7 +723,7 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     // columns of one row: one column-scale multiply, the snap, and one store per run.
     tile_wait<0>();  // every wave is done with the ring
     int32_t *sacc = reinterpret_cast<int32_t *>(smem);
-    float *sscale = reinterpret_cast<float *>(smem + BM * ESTR * 4);
+    float *sscale = reinterpret_cast<float *>(smem_all + BM * ESTR * 4);
     if (tid < BN) sscale[tid] = __fmul_rn(in_scale, col_scale);
 #pragma unroll
     for (int t = 0; t < TM; ++t)
@@ -732,12 +737,17 @@ __global__ __launch_bounds__(256) void qgemm_tile_kernel(
     bool r_ok;
     const float rcp = srq_recip(out_scale, r_ok);
     constexpr int RC = BN / 8;
-    for (int q = tid; q < BM * RC; q += 256) {
+    for (int q = tid; q < BM * RC; q += 256 * KS) {
         const int lr = q / RC, c = q - lr * RC;
         const int m = m0 + lr, n = n0 + c * 8;
         if (m >= M || n >= N) continue;
-        const v4i x0 = *reinterpret_cast<const v4i *>(sacc + lr * ESTR + c * 8);
-        const v4i x1 = *reinterpret_cast<const v4i *>(sacc + lr * ESTR + c * 8 + 4);
+        v4i x0 = v4i{0, 0, 0, 0}, x1 = v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const int32_t *p = reinterpret_cast<const int32_t *>(smem_all + s * (NS * SB)) + lr * ESTR + c * 8;
+            x0 += reinterpret_cast<const v4i *>(p)[0];
+            x1 += reinterpret_cast<const v4i *>(p)[1];
+        }
         const int v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
         const int live = min(8, N - n);
         const int64_t o = (int64_t)m * N + n;
@@ -1224,6 +1234,12 @@ static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, b
     if (m <= 16) return K_SKINNY16;
     if (k < 2 * kTileBK) return K_SKINNY32;  // the tile ring needs two K stages
     if (m <= 32) return K_SKINNY32;
+    // few enough outputs for one 16-wave block of 32 rows x 16 columns per CU: every CU then fetches
+    // its own 16 weight rows, where 96-column tiles leave most CUs without work and the others bound
+    // by what one CU can fetch (us in a graph, int8 codes, tile -> small: 64 x 1536 -> 2048 6.7 ->
+    // 4.0, 64 x 6144 -> 1536 15.3 -> 9.2, 256 x 1536 -> 256 6.7 -> 3.9, 512 x 1536 -> 256 6.8 -> 4.9;
+    // at two blocks per CU 128 x 6144 -> 1536 15.3 -> 22.9)
+    if (k >= 4 * kTileBK && (int64_t)((n + 15) / 16) * ((m + 31) / 32) <= device_cu_count()) return K_SKINNY32;
     // the wide tile once its grid fills the device: 4-bit weights, M >= 256, three K stages
     const int64_t wide_blocks = (int64_t)((m + kWideBM - 1) / kWideBM) * ((n + kWideBN - 1) / kWideBN);
     if (bits == 4 && m >= 256 && k >= kWideNS * kTileBK - kTileBK && wide_blocks >= device_cu_count())
@@ -1322,11 +1338,18 @@ static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, cons
     const int nk = k / kTileBK;  // >= 2 (k % 128 == 0 and k >= 256 here)
     // 8-bit weights are natural-order bytes already: their A is natural either way
     const bool nat = BITS == 4 && natural;
-#define G4_TILE(NS_, NAT_, BM_)                                                                   \
-    hipLaunchKernelGGL((qgemm_tile_kernel<BITS, NS_, NAT_, BM_>), dim3(blocks), dim3(256), 0,      \
+#define G4_TILE_K(NS_, NAT_, BM_, KS_)                                                            \
+    hipLaunchKernelGGL((qgemm_tile_kernel<BITS, NS_, NAT_, BM_, KS_>), dim3(blocks), dim3(256 * KS_), 0, \
                        stream, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind,     \
                        tiles_m, tiles_n)
-    if (half) {
+#define G4_TILE(NS_, NAT_, BM_) G4_TILE_K(NS_, NAT_, BM_, 1)
+    // a grid of at most one block per CU splits its K stages over two groups of four waves, twice the
+    // loads in flight per CU (us in a graph: 128 x 6144 -> 1536 15.3 -> 13.6, 128 x 1536 -> 6144 7.1
+    // -> 6.8, 256 x 2048 -> 1536 7.9 -> 7.4, 8-bit 512 x 1536 -> 256 6.2 -> 5.7; four groups 14.0, 7.1)
+    if (half && tiles_m * tiles_n <= device_cu_count() && nk % 2 == 0 && nk >= 6) {
+        if (nat) G4_TILE_K(4, true, 32, 2);
+        else G4_TILE_K(4, false, 32, 2);
+    } else if (half) {
         if (nk >= 3 && nat) G4_TILE(4, true, 32);
         else if (nk >= 3) G4_TILE(4, false, 32);
         else if (nat) G4_TILE(3, true, 32);
@@ -1338,6 +1361,7 @@ static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, cons
         else G4_TILE(3, false, 64);
     }
 #undef G4_TILE
+#undef G4_TILE_K
     G4_LAUNCHED("qgemm_tile_kernel");
     return G4_OK;
 }
@@ -1376,7 +1400,11 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
 static bool small_presnap(int m, int n, int k) {
     const int64_t cus = device_cu_count();
-    const int64_t blocks = (n + 15) / 16;  // M <= 32: one block row
+    const int64_t blocks = (n + 15) / 16;
+    // M > 32: one block per CU (pick_kernel). Up to K = 2048 the call stays one launch, which an eager
+    // caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
+    // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager)
+    if (m > 32) return 32 * k > 64 * 1024;
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && (blocks + cus - 1) / cus * m * k >= 48 * 1024;
 }
 

@@ -1,0 +1,32 @@
+"""The rules that send M > 32 to the small-M kernel (one block of 32 rows x 16 columns per CU) and
+split the tile kernel's K stages over two wave groups, at their edges: ragged rows and columns, K of
+odd and even stage counts, both weight widths, every input and output kind, against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits,m,n,k", [
+    (4, 33, 256, 512), (4, 63, 257, 1536), (4, 64, 2048, 1536), (4, 64, 2049, 1536),   # 256 / 258 blocks
+    (4, 96, 1365, 2048), (4, 97, 1365, 2048), (4, 500, 250, 1536), (4, 64, 40, 2304),
+    (4, 130, 1000, 768), (4, 100, 1500, 1024), (4, 256, 1530, 1280), (4, 40, 6100, 1536),  # tile, 6..12 stages
+    (8, 33, 17, 512), (8, 64, 256, 1536), (8, 128, 999, 896), (8, 300, 700, 1152), (8, 1030, 70, 640),
+])
+def test_routes(gpu, oracle, bits, m, n, k):
+    print(f"routes bits={bits} m={m} n={n} k={k} {gpu.kernel_for_shape(bits, m, n, k)}", flush=True)
+    g = np.random.default_rng(m + n + k)
+    x = g.standard_normal((m, k)).astype(np.float16)
+    w = g.integers(0, 256, (n, k * bits // 8), dtype=np.uint8)
+    s = (g.uniform(0.5, 1.5, n) / (np.sqrt(k) * (4.6 if bits == 4 else 73.6))).astype(np.float32)
+    want, acc, codes = oracle.qgemm(bits, w, s, x.astype(np.float32), n, k, m, 0.05, 0.1)
+    xq = np.clip(np.rint(x.astype(np.float32) / np.float32(0.05)), -128, 127).astype(np.int8)
+    dw, ds = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(s)
+    for xin in (x, x.astype(np.float32), xq):
+        dx = gpu.DeviceBuffer.from_array(xin)
+        for dt, ref in ((np.int32, acc), (np.int8, codes), (np.float32, want)):
+            out = gpu.DeviceBuffer.empty((m, n), dt)
+            out.fill(0x7B)
+            gpu.qgemm(bits, dw, ds, dx, out, k, n, m, 0.05, 0.1)
+            got = out.download()
+            assert np.array_equal(got.view(np.uint8), np.asarray(ref, dt).reshape(m, n).view(np.uint8)), (xin.dtype, dt)
