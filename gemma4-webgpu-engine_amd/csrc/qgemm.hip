@@ -151,10 +151,10 @@ __device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x888888
 // both operands. The LDS rows are padded by 16 bytes so the 16 token rows of one A read fall on
 // distinct banks.
 //
-// WAVES: 4 for wide outputs (many blocks); 16 when the output has too few 16-row blocks to fill
-// the chip (N = 1536 gives 96), so each block walks its K four times faster: a chunk of 128-code
-// steps has one step per wave, and the fold of the 16 partial tiles goes through LDS. The sums are
-// int32 and exact, so the split changes no result.
+// WAVES: 16 while the grid fits the CUs, over CT column tiles of 16 weight rows (small_col_tiles):
+// wave w takes tile w % CT and K part w / CT of 16 / CT, so a block walks its K fast and a CU copies
+// the codes once for all its columns; 4 (CT 1) for wider grids of 16-row blocks. The fold of the
+// partial tiles goes through LDS. The sums are int32 and exact, so the split changes no result.
 //
 // Grouped launches: up to kSmallMaxJobs projections of the same x, K and scales (q, k, v; gate and
 // up) share one grid; block b belongs to the first job whose block_end exceeds it.
@@ -183,8 +183,8 @@ struct SmallJobs {
 // chunks measured a 4.09 ms step, one chunk 4.01 ms).
 template <int MT, int WAVES> constexpr int small_kc() { return (WAVES >= 16 ? 98304 : 49152) / MT; }
 
-// One batch of a lane's weight loads for K steps kb0, kb0 + WAVES, ... (clamped: every load valid).
-template <int BITS, int NP, int BATCH, int WAVES>
+// One batch of a lane's weight loads for K steps kb0, kb0 + STEP, ... (clamped: every load valid).
+template <int BITS, int NP, int BATCH, int STEP>
 __device__ __forceinline__ void load_small_weights(u32x4 (&bw)[NP][BATCH][BITS == 4 ? 1 : 2],
                                                    const uint8_t *wrow, const uint8_t *wrow2, int kb0,
                                                    int ksteps, int kbase, int g) {
@@ -193,7 +193,7 @@ __device__ __forceinline__ void load_small_weights(u32x4 (&bw)[NP][BATCH][BITS =
         const uint8_t *wr = p == 0 ? wrow : wrow2;
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
-            const int kb = min(kb0 + WAVES * u, ksteps - 1);
+            const int kb = min(kb0 + STEP * u, ksteps - 1);
             if (BITS == 4) {
                 bw[p][u][0] = *reinterpret_cast<const u32x4 *>(wr + (kbase + kb) * 64 + g * 16);
             } else {
@@ -204,7 +204,7 @@ __device__ __forceinline__ void load_small_weights(u32x4 (&bw)[NP][BATCH][BITS =
     }
 }
 
-template <int BITS, int MT, int WAVES, int EPI>
+template <int BITS, int MT, int WAVES, int EPI, int CT>
 __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     const void *__restrict__ x, int x_kind, SmallJobs jobs, int M, int K, float in_scale,
     float out_scale, int out_kind, int ksplit) {
@@ -212,7 +212,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     constexpr int TM = MT / 16;
     constexpr int KC = small_kc<MT, WAVES>();  // codes of a row per LDS chunk
     constexpr int XSTR = KC + 16;              // LDS bytes per token row
-    constexpr int BATCH = WAVES >= 16 ? 1 : 4;
+    constexpr int KW = WAVES / CT;             // waves splitting K for one column tile
+    constexpr int BATCH = WAVES >= 16 ? CT : 4;
     constexpr int NP = EPI == 1 ? 2 : 1;             // product sets: the gate's (and the up's)
     constexpr int NACC = NP * TM;
     constexpr int SHIFT = BITS == 4 ? 4 : 0;         // 4-bit sums are of 16 * code
@@ -224,10 +225,11 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
     __shared__ __align__(16) int8_t smem[SEP_RED ? XS_BYTES + RED_BYTES
                                                  : (XS_BYTES > RED_BYTES ? XS_BYTES : RED_BYTES)];
     int8_t *xs = smem;
-    v4i(*red)[NACC][64] = reinterpret_cast<v4i(*)[NACC][64]>(smem + (SEP_RED ? XS_BYTES : 0));
+    v4i(*red)[NACC][64] = reinterpret_cast<v4i(*)[NACC][64]>(smem + (SEP_RED ? XS_BYTES : 0));  // [wave]
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
+    const int ct = CT == 1 ? 0 : wave % CT, kw = wave / CT;  // the wave's column tile and K part
     const int j = lane & 15;
     const int g = lane >> 4;
     // the block's job (uniform selects, no indexed kernel-argument array)
@@ -245,22 +247,23 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
             begin = jobs.block_end[i - 1];
         }
     }
-    const int n0 = ((int)blockIdx.x - begin) * 16;
+    const int n0 = ((int)blockIdx.x - begin) * (16 * CT);
     const int m0 = blockIdx.y * MT;
-    const int n = min(n0 + j, N - 1);
+    const int n = min(n0 + ct * 16 + j, N - 1);
     const int row_bytes = BITS == 4 ? (K >> 1) : K;
     const uint8_t *wrow = W + (int64_t)n * row_bytes;
     const uint8_t *wrow2 = EPI == 1 ? jobs.w_up + (int64_t)n * row_bytes : wrow;
     const SrqScale S = srq_scale(in_scale);
     // the epilogue's per-output operands (row scales; the paired up rows' scales; the f32 up
     // vector), requested now so the epilogue does not wait a memory round trip for them
-    constexpr int EQ = (TM * 256 + THREADS - 1) / THREADS;  // outputs per thread
+    constexpr int OUTS = CT * TM * 256;                     // the block's outputs
+    constexpr int EQ = (OUTS + THREADS - 1) / THREADS;      // outputs per thread
     float e_scale[EQ], e_scale2[EQ], e_aux[EQ];
 #pragma unroll
     for (int e = 0; e < EQ; ++e) {
-        const int q = min(tid + e * THREADS, TM * 256 - 1);
-        const int t = q >> 8, ln = (q >> 2) & 63, r = q & 3;
-        const int nn = min(n0 + (ln & 15), N - 1);
+        const int q = min(tid + e * THREADS, OUTS - 1);
+        const int t = (q >> 8) % TM, ln = (q >> 2) & 63, r = q & 3;
+        const int nn = min(n0 + (q >> 8) / TM * 16 + (ln & 15), N - 1);
         const int m = min(m0 + t * 16 + 4 * (ln >> 4) + r, M - 1);
         e_scale[e] = scales[nn];
         e_scale2[e] = EPI == 1 ? jobs.s_up[nn] : 0.0f;
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
         // first measured slower: every block reads the same few KB of codes, and at the head of
         // the queue those requests pile onto the same L2 lines.
         u32x4 bw_first[NP][BATCH][BITS == 4 ? 1 : 2];
-        load_small_weights<BITS, NP, BATCH, WAVES>(bw_first, wrow, wrow2, wave, ksteps, kbase, g);
+        load_small_weights<BITS, NP, BATCH, KW>(bw_first, wrow, wrow2, kw, ksteps, kbase, g);
         lds_barrier();  // the previous chunk's codes are no longer read
         // the snap: each thread issues the loads of SB groups (indices clamped, so every load is
         // valid) before converting any, so a chunk costs one memory latency per SB groups; one
@@ -351,9 +354,9 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
         if (x_kind == G4_KIND_F16) snap(std::true_type{});
         else if (x_kind != G4_KIND_I8) snap(std::false_type{});
         lds_barrier();
-        for (int kb0 = wave; kb0 < ksteps; kb0 += WAVES * BATCH) {
+        for (int kb0 = kw; kb0 < ksteps; kb0 += KW * BATCH) {
             u32x4 bw[NP][BATCH][BITS == 4 ? 1 : 2];
-            if (kb0 == wave) {
+            if (kb0 == kw) {
 #pragma unroll
                 for (int p = 0; p < NP; ++p)
 #pragma unroll
@@ -361,14 +364,14 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
 #pragma unroll
                         for (int h = 0; h < (BITS == 4 ? 1 : 2); ++h) bw[p][u][h] = bw_first[p][u][h];
             } else {
-                load_small_weights<BITS, NP, BATCH, WAVES>(bw, wrow, wrow2, kb0, ksteps, kbase, g);
+                load_small_weights<BITS, NP, BATCH, KW>(bw, wrow, wrow2, kb0, ksteps, kbase, g);
             }
             // every A operand of the batch read from LDS before the first MFMA, so the reads'
             // latencies overlap (step indices clamped: a step past the end is read, not used)
             v4i av[BATCH][2][TM];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u) {
-                const int kb = min(kb0 + WAVES * u, ksteps - 1);
+                const int kb = min(kb0 + KW * u, ksteps - 1);
 #pragma unroll
                 for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
             }
 #pragma unroll
             for (int u = 0; u < BATCH; ++u) {
-                const int kb = kb0 + WAVES * u;
+                const int kb = kb0 + KW * u;
                 if (kb < ksteps) {
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
@@ -424,17 +427,17 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_small_kernel(
 #pragma unroll
     for (int e = 0; e < EQ; ++e) {
         const int q = tid + e * THREADS;
-        if (q >= TM * 256) break;
+        if (q >= OUTS) break;
         // D layout: lane l, register r -> row 4 (l / 16) + r of A, column l % 16 of B.
-        const int t = q >> 8, ln = (q >> 2) & 63, r = q & 3;
+        const int oc = (q >> 8) / TM, t = (q >> 8) % TM, ln = (q >> 2) & 63, r = q & 3;
         const int lr = t * 16 + 4 * (ln >> 4) + r;
-        const int m = m0 + lr, nn = n0 + (ln & 15);
+        const int m = m0 + lr, nn = n0 + oc * 16 + (ln & 15);
         if (m >= M || nn >= N) continue;
         int v = 0, v2 = 0;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            v += reinterpret_cast<const int *>(&red[w][t][ln])[r];
-            if (EPI == 1) v2 += reinterpret_cast<const int *>(&red[w][TM + t][ln])[r];
+        for (int w = 0; w < KW; ++w) {
+            v += reinterpret_cast<const int *>(&red[w * CT + oc][t][ln])[r];
+            if (EPI == 1) v2 += reinterpret_cast<const int *>(&red[w * CT + oc][TM + t][ln])[r];
         }
         v >>= SHIFT;
         v2 >>= SHIFT;
@@ -1217,6 +1220,24 @@ int workspace_forget_stream(void *stream) {
     return G4_OK;
 }
 
+// The column tiles (16 weight rows each) of a 16-wave small-M block for a grid of `blocks16` single
+// tiles, or 0 for 4-wave blocks of one tile. The fewest whose grid fits the CUs once (1, 2 or 4): a
+// CU then copies the activation codes once for all of its columns (us in a graph, int8 codes, 4-wave
+// -> two tiles: 32 x 1536 -> 6144 7.5 -> 5.3, 8 x 1536 -> 6144 4.5 -> 4.3, 32 x 6144 -> 6144 23.2 -> 11.2;
+// -> four: 32 x 1536 -> 8960 11.7 -> 7.2, 16384 12.8 -> 7.7). Past that, 32-row blocks still take
+// four (32 x 1024 -> 24576 14.9 -> 11.9) and 16-row ones, whose codes are half, the 4-wave blocks
+// (8 x 1024 -> 24576 8.1 / 9.5), which also win up to three tiles per CU while their codes take one
+// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). The paired gate / up form stops
+// at two (its four would spill).
+static int small_col_tiles(int64_t blocks16, int mt, int k, bool paired) {
+    const int64_t cus = device_cu_count();
+    if (blocks16 <= cus) return 1;
+    if (blocks16 <= 2 * cus) return 2;
+    if (paired) return 0;
+    if (mt > 16) return 4;
+    return blocks16 <= 4 * cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
+}
+
 enum KernelChoice { K_GEMV = 0, K_SKINNY16, K_SKINNY32, K_TILE128, K_GEMV_F32, K_GEMV_COLS,
                     K_SERIAL8, K_WIDE };
 
@@ -1234,12 +1255,15 @@ static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, b
     if (m <= 16) return K_SKINNY16;
     if (k < 2 * kTileBK) return K_SKINNY32;  // the tile ring needs two K stages
     if (m <= 32) return K_SKINNY32;
-    // few enough outputs for one 16-wave block of 32 rows x 16 columns per CU: every CU then fetches
-    // its own 16 weight rows, where 96-column tiles leave most CUs without work and the others bound
-    // by what one CU can fetch (us in a graph, int8 codes, tile -> small: 64 x 1536 -> 2048 6.7 ->
-    // 4.0, 64 x 6144 -> 1536 15.3 -> 9.2, 256 x 1536 -> 256 6.7 -> 3.9, 512 x 1536 -> 256 6.8 -> 4.9;
-    // at two blocks per CU 128 x 6144 -> 1536 15.3 -> 22.9)
-    if (k >= 4 * kTileBK && (int64_t)((n + 15) / 16) * ((m + 31) / 32) <= device_cu_count()) return K_SKINNY32;
+    // few enough outputs for one 16-wave small-M block per CU (32 rows x 16 columns; x 32 up to 64
+    // rows or for long K): every CU then fetches its own few weight rows, where 96-column tiles leave
+    // most CUs without work and the others bound by what one CU can fetch (us in a graph, int8 codes,
+    // tile -> small: 64 x 1536 -> 2048 6.7 -> 4.0, 64 x 6144 -> 1536 13.6 -> 9.2, 256 x 1536 -> 256 6.7 ->
+    // 3.9, 64 x 1536 -> 3072 6.3 -> 4.5, 64 x 6144 -> 4096 13.6 -> 11.1, 128 x 6144 -> 1536 13.6 -> 11.0,
+    // 128 x 2048 -> 1536 7.2 -> 5.5; four tiles per block lose: 64 x 1536 -> 6144 6.7 / 7.2)
+    const int64_t small_blocks = (int64_t)((n + 15) / 16) * ((m + 31) / 32);
+    if (k >= 4 * kTileBK && small_blocks <= (m <= 64 || k >= 2048 ? 2 : 1) * (int64_t)device_cu_count())
+        return K_SKINNY32;
     // the wide tile once its grid fills the device: 4-bit weights, M >= 256, three K stages
     const int64_t wide_blocks = (int64_t)((m + kWideBM - 1) / kWideBM) * ((n + kWideBN - 1) / kWideBN);
     if (bits == 4 && m >= 256 && k >= kWideNS * kTileBK - kTileBK && wide_blocks >= device_cu_count())
@@ -1260,21 +1284,30 @@ static const char *choice_name(KernelChoice c, int bits) {
     }
 }
 
-// The small-M kernel over `jobs` (16-row blocks laid end to end): 16 waves per block when the
-// grid has no more blocks than the device has CUs (each block then walks its K four times
-// faster), else 4.
+// The small-M kernel over `jobs` (16-row blocks laid end to end).
 template <int BITS, int MT, int EPI>
 static void launch_small_t(const void *x, int x_kind, const SmallJobs &jobs, int m, int k,
                            float in_scale, float out_scale, int out_kind, hipStream_t stream,
                            int splits = 1) {
     const int ksplit = splits > 1 ? k / splits : 0;
     const dim3 grid(jobs.block_end[jobs.count - 1], (m + MT - 1) / MT, splits);
-    if ((int64_t)grid.x * grid.y * grid.z <= device_cu_count())
-        hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 16, EPI>), grid, dim3(1024), 0, stream, x,
+    const int ct = small_col_tiles((int64_t)grid.x * grid.y * grid.z, MT, k, EPI == 1);
+    if (ct == 0) {
+        hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 4, EPI, 1>), grid, dim3(256), 0, stream, x,
                            x_kind, jobs, m, k, in_scale, out_scale, out_kind, ksplit);
-    else
-        hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 4, EPI>), grid, dim3(256), 0, stream, x,
-                           x_kind, jobs, m, k, in_scale, out_scale, out_kind, ksplit);
+        return;
+    }
+    SmallJobs wide = jobs;
+    int end = 0;
+    for (int i = 0; i < jobs.count; ++i) wide.block_end[i] = end += (jobs.n[i] + 16 * ct - 1) / (16 * ct);
+    const dim3 grid_ct(end, grid.y, grid.z), block(1024);
+#define G4_SMALL_CT(CT_)                                                                            \
+    hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 16, EPI, CT_>), grid_ct, block, 0, stream, x, \
+                       x_kind, wide, m, k, in_scale, out_scale, out_kind, ksplit)
+    if (ct == 1) G4_SMALL_CT(1);
+    else if (ct == 2 || EPI == 1) G4_SMALL_CT(2);
+    else G4_SMALL_CT(EPI == 1 ? 2 : 4);
+#undef G4_SMALL_CT
 }
 
 // epi: 0 plain (any job count), 1 the paired gate/up gelu epilogue (4-bit), 2 the f32-vector one.
@@ -1394,9 +1427,8 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 // The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past 48 Ki snaps
 // on the busiest CU (M * K per block, times its blocks there), one snap pass over the M * K
 // activations into a buffer of codes, then the kernel on int8 codes, costs less. Fused against
-// passed, us in a graph: 8 x 1536 -> 6144 (24 Ki) 6.1 / 7.0, 12 x 1536 -> 6144 (36 Ki) 7.1 / 7.4,
-// 24 x 1536 -> 2048 (36 Ki) 5.6 / 6.4, 16 x 1536 -> 6144 (48 Ki) 7.8 / 7.6, 8 x 6144 -> 1536 (48 Ki)
-// 8.1 / 8.0, 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
+// passed, us in a graph: 24 x 1536 -> 2048 (36 Ki) 5.6 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
+// 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
 static bool small_presnap(int m, int n, int k) {
     const int64_t cus = device_cu_count();
@@ -1405,7 +1437,9 @@ static bool small_presnap(int m, int n, int k) {
     // caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
     // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager)
     if (m > 32) return 32 * k > 64 * 1024;
-    return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && (blocks + cus - 1) / cus * m * k >= 48 * 1024;
+    const int ct = std::max(1, small_col_tiles(blocks, m <= 16 ? 16 : 32, k, false));
+    return (int64_t)m * k * blocks >= ((int64_t)1 << 22) &&
+           ((blocks + ct - 1) / ct + cus - 1) / cus * m * k >= 48 * 1024;
 }
 
 // Whether a call snaps f16 / f32 activations into a buffer of M * K codes first (the tile kernels,

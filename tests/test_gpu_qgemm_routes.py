@@ -14,6 +14,10 @@ pytestmark = pytest.mark.gpu
     (8, 33, 17, 512), (8, 64, 256, 1536), (8, 128, 999, 896), (8, 300, 700, 1152), (8, 1030, 70, 640),
 ])
 def test_routes(gpu, oracle, bits, m, n, k):
+    check_every_kind(gpu, oracle, bits, m, n, k)
+
+
+def check_every_kind(gpu, oracle, bits, m, n, k):
     print(f"routes bits={bits} m={m} n={n} k={k} {gpu.kernel_for_shape(bits, m, n, k)}", flush=True)
     g = np.random.default_rng(m + n + k)
     x = g.standard_normal((m, k)).astype(np.float16)
@@ -30,3 +34,13 @@ def test_routes(gpu, oracle, bits, m, n, k):
             gpu.qgemm(bits, dw, ds, dx, out, k, n, m, 0.05, 0.1)
             got = out.download()
             assert np.array_equal(got.view(np.uint8), np.asarray(ref, dt).reshape(m, n).view(np.uint8)), (xin.dtype, dt)
+
+
+@pytest.mark.parametrize("bits,m,n,k", [
+    (4, 16, 4096, 256), (4, 16, 4097, 512), (4, 5, 8193, 512), (4, 16, 12289, 256), (4, 9, 9001, 3328),
+    (4, 17, 4099, 1536), (4, 32, 8200, 1536), (4, 31, 16500, 256), (8, 32, 4100, 384), (8, 12, 8300, 3200),
+    (8, 20, 17000, 128), (4, 64, 3071, 768), (4, 40, 4096, 2304), (4, 100, 1500, 2048),
+])
+def test_column_tiles(gpu, oracle, bits, m, n, k):
+    # 16-wave blocks of one, two and four column tiles and the 4-wave blocks, either side of each line
+    check_every_kind(gpu, oracle, bits, m, n, k)
