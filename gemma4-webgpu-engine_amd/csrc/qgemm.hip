@@ -21,7 +21,9 @@
 //                  same x can share one grid (linear_grouped).
 //   larger outputs, or over 32768+ rows
 //                  qgemm_tile_kernel: 64 x 96 output tiles, activation codes and weights streamed
-//                  global -> LDS by direct loads through a 3-4 stage ring, XCD-aware tile order.
+//                  global -> LDS by direct loads through a 3-4 stage ring, XCD-aware tile order;
+//                  4-bit outputs that fill the chip take 64 x 192 tiles (qgemm_wide_kernel), and
+//                  256 x 192 ones (qgemm_tall_kernel) when those come in nearly whole rounds of CUs.
 #include "g4_internal.h"
 #include "g4_workspace.h"
 
@@ -971,6 +973,131 @@ __device__ __forceinline__ void wide_k_loop(const uint8_t *const (&src)[NL], con
     wide_wait<0, true>();  // the ring is free for the epilogue
 }
 
+// The epilogue of the 192-column tiles: `sum` are R 16-row tiles x 3 column tiles of 16 x (sums), the
+// wave's rows from row0 and columns from 48 wn; T a code tile of BM rows in LDS that no wave reads
+// any more, S the columns' inScale x scale.
+template <int R, int BM>
+__device__ __forceinline__ void wide_store(const v4i (&sum)[R][3], int row0, uint8_t *T, const float *S, void *dst,
+                                           int m0, int n0, int wn, int M, int N, int out_kind, float out_scale) {
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    bool r_ok;
+    const float rcp = srq_recip(out_scale, r_ok);
+    // A whole tile of int8 outputs (the usual case): the same snap with no row, column or
+    // alignment checks per group of 4. Each group's 4 codes go to a BM x 192 code tile in LDS
+    // (rows 208 bytes apart, so the 64 lanes of a group store hit distinct banks); then each
+    // thread stores 16-byte runs of whole tile rows (192 contiguous bytes per row), in place of
+    // 4-byte stores scattered over 16 rows per instruction. N % 16 == 0 and a 16-byte aligned dst
+    // keep every run aligned.
+    if (out_kind == G4_KIND_I8 && out_scale != 0.0f && m0 + BM <= M && n0 + kWideBN <= N && (N & 15) == 0 &&
+        ((uintptr_t)dst & 15) == 0) {
+#pragma unroll
+        for (int tt = 0; tt < R; ++tt) {
+            uint8_t *trow = T + (row0 + tt * 16 + j) * kWideCodeRow + wn * 48 + 4 * g;
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const float4 s4 = *reinterpret_cast<const float4 *>(S + wn * 48 + u * 16 + 4 * g);
+                const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
+                const int v[4] = {sum[tt][u].x >> 4, sum[tt][u].y >> 4, sum[tt][u].z >> 4, sum[tt][u].w >> 4};
+                float y[4], code[4];
+                float worst = r_ok ? 0.0f : 1.0f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    y[e] = __fmul_rn(sc[e], (float)v[e]);  // the reference's order
+                    const float t = __fmul_rn(y[e], rcp);
+                    code[e] = rintf(t);
+                    worst = fmaxf(worst, fabsf(t - code[e]));
+                }
+                if (worst >= 0.5f - 0x1p-13f) {  // the quotient bound of the generic path below
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) code[e] = rintf(__fdiv_rn(y[e], out_scale));
+                }
+                uint32_t bb[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    bb[e] = __float_as_uint(__fadd_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), 12582912.0f));
+                const uint32_t lo = __builtin_amdgcn_perm(bb[1], bb[0], 0x0C0C0400u);
+                const uint32_t hi = __builtin_amdgcn_perm(bb[3], bb[2], 0x0C0C0400u);
+                *reinterpret_cast<uint32_t *>(trow + u * 16) = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+            }
+        }
+        __syncthreads();
+        for (int c = tid; c < BM * (kWideBN / 16); c += 512) {
+            const int r = c / (kWideBN / 16), cc = c - r * (kWideBN / 16);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(T + r * kWideCodeRow + cc * 16);
+            __builtin_nontemporal_store(
+                v, reinterpret_cast<u32x4 *>(reinterpret_cast<int8_t *>(dst) + (int64_t)(m0 + r) * N + n0 + cc * 16));
+        }
+        return;
+    }
+#pragma unroll
+    for (int tt = 0; tt < R; ++tt) {
+        const int m = m0 + row0 + tt * 16 + j;
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            const int n = n0 + wn * 48 + u * 16 + 4 * g;
+            const int live = min(4, N - n);
+            const bool row_ok = m < M && live > 0;
+            const int64_t o = (int64_t)m * N + n;
+            const int v[4] = {sum[tt][u].x >> 4, sum[tt][u].y >> 4, sum[tt][u].z >> 4, sum[tt][u].w >> 4};
+            if (out_kind == G4_KIND_I32) {
+                if (!row_ok) continue;
+                int32_t *d = reinterpret_cast<int32_t *>(dst) + o;
+                if (live == 4 && (o & 3) == 0) *reinterpret_cast<v4i *>(d) = v4i{v[0], v[1], v[2], v[3]};
+                else for (int e = 0; e < live; ++e) d[e] = v[e];
+                continue;
+            }
+            const float4 s4 = *reinterpret_cast<const float4 *>(S + wn * 48 + u * 16 + 4 * g);
+            const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
+            float y[4], code[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = __fmul_rn(sc[e], (float)v[e]);  // the reference's order
+            if (out_scale == 0.0f) {  // f32 output without an output snap (int8 needs a scale)
+                if (!row_ok) continue;
+                float *d = reinterpret_cast<float *>(dst) + o;
+                if (live == 4 && (o & 3) == 0) *reinterpret_cast<float4 *>(d) = make_float4(y[0], y[1], y[2], y[3]);
+                else for (int e = 0; e < live; ++e) d[e] = y[e];
+                continue;
+            }
+            float worst = r_ok ? 0.0f : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float t = __fmul_rn(y[e], rcp);
+                code[e] = rintf(t);
+                worst = fmaxf(worst, fabsf(t - code[e]));
+            }
+            // |fl(y * fl(1/s)) - fl(y / s)| < 2^-13 while |y / s| <= 256 (beyond, both clamp): a
+            // quotient farther than that from a half integer rounds the same either way.
+            if (worst >= 0.5f - 0x1p-13f) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) code[e] = rintf(__fdiv_rn(y[e], out_scale));
+            }
+            if (!row_ok) continue;
+            if (out_kind == G4_KIND_I8) {
+                // code + 1.5 * 2^23 is exact and its low byte is the code's two's complement byte
+                uint32_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    b[e] = __float_as_uint(__fadd_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), 12582912.0f));
+                int8_t *d = reinterpret_cast<int8_t *>(dst) + o;
+                if (live == 4 && (o & 3) == 0) {
+                    const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0400u);  // b0.0 b1.0
+                    const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0400u);  // b2.0 b3.0
+                    *reinterpret_cast<uint32_t *>(d) = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+                } else {
+                    for (int e = 0; e < live; ++e) d[e] = (int8_t)(b[e] & 0xffu);
+                }
+            } else {  // f32: q * outScale
+                float f[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[e] = __fmul_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), out_scale);
+                float *d = reinterpret_cast<float *>(dst) + o;
+                if (live == 4 && (o & 3) == 0) *reinterpret_cast<float4 *>(d) = make_float4(f[0], f[1], f[2], f[3]);
+                else for (int e = 0; e < live; ++e) d[e] = f[e];
+            }
+        }
+    }
+}
+
 template <bool NAT>
 __global__ __launch_bounds__(512, 4) void qgemm_wide_kernel(
     const int8_t *__restrict__ A, const uint8_t *__restrict__ W, const float *__restrict__ scales,
@@ -1059,123 +1186,149 @@ __global__ __launch_bounds__(512, 4) void qgemm_wide_kernel(
     if (kh == 0) meet(std::integral_constant<int, 0>{});
     else meet(std::integral_constant<int, 1>{});
 
-    bool r_ok;
-    const float rcp = srq_recip(out_scale, r_ok);
-    // A whole tile of int8 outputs (the usual case): the same snap with no row, column or
-    // alignment checks per group of 4. Each group's 4 codes go to a 64 x 192 code tile in LDS
-    // (rows 208 bytes apart, so the 64 lanes of a group store hit distinct banks); then each
-    // thread stores 16-byte runs of whole tile rows (192 contiguous bytes per row), in place of
-    // 4-byte stores scattered over 16 rows per instruction. N % 16 == 0 and a 16-byte aligned dst
-    // keep every run aligned.
-    if (out_kind == G4_KIND_I8 && out_scale != 0.0f && m0 + kWideBM <= M && n0 + kWideBN <= N && (N & 15) == 0 &&
-        ((uintptr_t)dst & 15) == 0) {
-        uint8_t *T = smem + kWideCodeTile;
+    wide_store<2, kWideBM>(sum, 32 * kh, smem + kWideCodeTile, S, dst, m0, n0, wn, M, N, out_kind, out_scale);
+}
+
+// ---- the tall tile: 4-bit weights, 256 x 192 outputs per block of 8 waves ----------------------
+//
+// For outputs of at least one such tile per CU (M = 2048 against 6144 columns: 256 tiles). The K loop
+// of the 64 x 192 tile is bound by LDS (64 KB per stage against 384 MFMA cycles per SIMD); here a
+// stage moves 196 KB (44 KB of direct loads, 152 KB of operand reads) against 1536: each wave owns
+// 128 x 48 outputs (8 x 3 MFMA tiles), so a weight operand is unpacked once for eight MFMAs and an
+// activation operand feeds three. 3-stage ring (132 KB, one block per CU), the operand reads of each
+// half-step in flight under the MFMAs of the one before. Layouts and swizzles are the narrow tile's
+// (a stage buffer is 256 activation rows, then 192 weight columns); the weights are the MFMA's A
+// operand and the epilogue is the wide tile's. Measured: 2048 x 1536 -> 6144 in 22.8 us (1.69 int8
+// POPS; 26.6 on the wide tile), 2048 x 6144 -> 6144 67.0 us (2.31 POPS; 82.2). A stage takes about
+// 2770 cycles, near what a CU's LDS delivers under MFMA load (70-95 bytes per clock); the snap of 96
+// outputs per thread and the fill add about 8 us per tile.
+constexpr int kTallBM = 256, kTallNS = 3;
+constexpr int kTallA = kTallBM * 128, kTallSB = kTallA + kWideBN * 64;
+
+template <bool NAT>
+__global__ __launch_bounds__(512, 2) void qgemm_tall_kernel(
+    const int8_t *__restrict__ A, const uint8_t *__restrict__ W, const float *__restrict__ scales,
+    void *dst, int M, int N, int K, float in_scale, float out_scale, int out_kind, int tiles_m,
+    int tiles_n) {
+    constexpr int NS = kTallNS, NL = 6;  // direct loads per wave and stage: 4 of activations, 2 of weights
+    __shared__ __align__(1024) uint8_t smem[NS * kTallSB];
+    static_assert(1024 + kTallBM * kWideCodeRow <= NS * kTallSB, "the scales and the code tile fit the ring");
+    const int b = blockIdx.x;
+    const int xcd = b & 7, idx = b >> 3;
+    const int tnx = (tiles_n + 7) >> 3;
+    const int tm = idx / tnx;
+    const int tn = (idx % tnx) * 8 + xcd;
+    if (tn >= tiles_n) return;  // whole block, before any barrier
+    const int m0 = tm * kTallBM, n0 = tn * kWideBN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3;
+    const int j = lane & 15, g = lane >> 4;
+    const uint32_t sbase = (uint32_t)(uintptr_t)smem;
+    const int row_bytes = K >> 1;
+    const float col_scale = tid < kWideBN ? scales[min(n0 + tid, N - 1)] : 0.0f;
+    // load q < 32: activation rows 8 q .. 8 q + 7; load 32 + q: weight columns 16 q .. 16 q + 15 (the
+    // last four waves' second one re-loads columns 176 .. 191 to the same bytes)
+    const uint8_t *src[NL];
+    uint32_t dsto[NL];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            uint8_t *trow = T + ((2 * kh + tt) * 16 + j) * kWideCodeRow + wn * 48 + 4 * g;
-#pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const float4 s4 = *reinterpret_cast<const float4 *>(S + wn * 48 + u * 16 + 4 * g);
-                const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
-                const int v[4] = {sum[tt][u].x >> 4, sum[tt][u].y >> 4, sum[tt][u].z >> 4, sum[tt][u].w >> 4};
-                float y[4], code[4];
-                float worst = r_ok ? 0.0f : 1.0f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    y[e] = __fmul_rn(sc[e], (float)v[e]);  // the reference's order
-                    const float t = __fmul_rn(y[e], rcp);
-                    code[e] = rintf(t);
-                    worst = fmaxf(worst, fabsf(t - code[e]));
-                }
-                if (worst >= 0.5f - 0x1p-13f) {  // the quotient bound of the generic path below
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) code[e] = rintf(__fdiv_rn(y[e], out_scale));
-                }
-                uint32_t bb[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    bb[e] = __float_as_uint(__fadd_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), 12582912.0f));
-                const uint32_t lo = __builtin_amdgcn_perm(bb[1], bb[0], 0x0C0C0400u);
-                const uint32_t hi = __builtin_amdgcn_perm(bb[3], bb[2], 0x0C0C0400u);
-                *reinterpret_cast<uint32_t *>(trow + u * 16) = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-            }
-        }
-        __syncthreads();
-        for (int c = tid; c < kWideBM * (kWideBN / 16); c += 512) {
-            const int r = c / (kWideBN / 16), cc = c - r * (kWideBN / 16);
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(T + r * kWideCodeRow + cc * 16);
-            __builtin_nontemporal_store(
-                v, reinterpret_cast<u32x4 *>(reinterpret_cast<int8_t *>(dst) + (int64_t)(m0 + r) * N + n0 + cc * 16));
-        }
-        return;
+    for (int i = 0; i < 4; ++i) {
+        const int q = wave + 8 * i;
+        const int r = 8 * q + (lane >> 3);
+        const int c = (lane & 7) ^ (((lane >> 3) & 7) ^ (q & 1));
+        src[i] = reinterpret_cast<const uint8_t *>(A + (int64_t)min(m0 + r, M - 1) * K + 16 * c);
+        dsto[i] = q * 1024;
     }
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        const int m = m0 + (2 * kh + tt) * 16 + j;
+    for (int i = 4; i < NL; ++i) {
+        const int q = min(wave + 8 * (i - 4), kWideBN / 16 - 1);
+        const int cl = lane >> 2;
+        const int c = (lane & 3) ^ (((cl >> 1) ^ (cl >> 3)) & 3);
+        src[i] = W + (int64_t)min(n0 + 16 * q + cl, N - 1) * row_bytes + 16 * c;
+        dsto[i] = kTallA + q * 1024;
+    }
+    auto issue = [&](int st, int buf) {
+        const uint32_t base = sbase + buf * kTallSB;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) lds_dma16(src[i] + st * (i < 4 ? 128 : 64), base + dsto[i]);
+    };
+    const int sig = (j & 7) ^ ((j >> 3) & 1);
+    uint32_t aoff[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        aoff[h] = (wm * 16 + (j >> 3)) * 1024 + (j & 7) * 128 + 16 * ((2 * g + h) ^ sig);
+    const uint32_t boff = kTallA + (wn * 48 + j) * 64 + 16 * (g ^ (((j >> 1) ^ (j >> 3)) & 3));
+
+    v4i acc[8][3];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) acc[t][u] = v4i{0, 0, 0, 0};
+    v4i ra[2][8];   // the activation operands of the two half-steps
+    u32x4 rb[3];    // the stage's packed weights
+    auto read_a = [&](int buf, int h) {
+        const uint8_t *p = smem + buf * kTallSB + aoff[h];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) ra[h][t] = *reinterpret_cast<const v4i *>(p + t * 2048);
+    };
+    auto unpack = [&](uint32_t w0, uint32_t w1) {
+        if (NAT) {
+            int l0, h0, l1, h1;
+            nib_natural16(w0, l0, h0);
+            nib_natural16(w1, l1, h1);
+            return v4i{l0, h0, l1, h1};
+        }
+        return v4i{(int)nib_even16(w0), (int)nib_odd16(w0), (int)nib_even16(w1), (int)nib_odd16(w1)};
+    };
+    const int nk = K / kTileBK;  // >= NS
+#pragma unroll
+    for (int st = 0; st < NS; ++st) issue(st, st);
+    tile_wait<(NS - 1) * NL>();
+    read_a(0, 0);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) rb[u] = *reinterpret_cast<const u32x4 *>(smem + boff + u * 1024);
+    int cur = 0;
+    for (int st = 0; st < nk; ++st) {
+        read_a(cur, 1);
+        v4i w0[3], w1[3];
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
-            const int n = n0 + wn * 48 + u * 16 + 4 * g;
-            const int live = min(4, N - n);
-            const bool row_ok = m < M && live > 0;
-            const int64_t o = (int64_t)m * N + n;
-            const int v[4] = {sum[tt][u].x >> 4, sum[tt][u].y >> 4, sum[tt][u].z >> 4, sum[tt][u].w >> 4};
-            if (out_kind == G4_KIND_I32) {
-                if (!row_ok) continue;
-                int32_t *d = reinterpret_cast<int32_t *>(dst) + o;
-                if (live == 4 && (o & 3) == 0) *reinterpret_cast<v4i *>(d) = v4i{v[0], v[1], v[2], v[3]};
-                else for (int e = 0; e < live; ++e) d[e] = v[e];
-                continue;
-            }
-            const float4 s4 = *reinterpret_cast<const float4 *>(S + wn * 48 + u * 16 + 4 * g);
-            const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
-            float y[4], code[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = __fmul_rn(sc[e], (float)v[e]);  // the reference's order
-            if (out_scale == 0.0f) {  // f32 output without an output snap (int8 needs a scale)
-                if (!row_ok) continue;
-                float *d = reinterpret_cast<float *>(dst) + o;
-                if (live == 4 && (o & 3) == 0) *reinterpret_cast<float4 *>(d) = make_float4(y[0], y[1], y[2], y[3]);
-                else for (int e = 0; e < live; ++e) d[e] = y[e];
-                continue;
-            }
-            float worst = r_ok ? 0.0f : 1.0f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float t = __fmul_rn(y[e], rcp);
-                code[e] = rintf(t);
-                worst = fmaxf(worst, fabsf(t - code[e]));
-            }
-            // |fl(y * fl(1/s)) - fl(y / s)| < 2^-13 while |y / s| <= 256 (beyond, both clamp): a
-            // quotient farther than that from a half integer rounds the same either way.
-            if (worst >= 0.5f - 0x1p-13f) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) code[e] = rintf(__fdiv_rn(y[e], out_scale));
-            }
-            if (!row_ok) continue;
-            if (out_kind == G4_KIND_I8) {
-                // code + 1.5 * 2^23 is exact and its low byte is the code's two's complement byte
-                uint32_t b[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    b[e] = __float_as_uint(__fadd_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), 12582912.0f));
-                int8_t *d = reinterpret_cast<int8_t *>(dst) + o;
-                if (live == 4 && (o & 3) == 0) {
-                    const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0400u);  // b0.0 b1.0
-                    const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0400u);  // b2.0 b3.0
-                    *reinterpret_cast<uint32_t *>(d) = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-                } else {
-                    for (int e = 0; e < live; ++e) d[e] = (int8_t)(b[e] & 0xffu);
-                }
-            } else {  // f32: q * outScale
-                float f[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) f[e] = __fmul_rn(fminf(fmaxf(code[e], -128.0f), 127.0f), out_scale);
-                float *d = reinterpret_cast<float *>(dst) + o;
-                if (live == 4 && (o & 3) == 0) *reinterpret_cast<float4 *>(d) = make_float4(f[0], f[1], f[2], f[3]);
-                else for (int e = 0; e < live; ++e) d[e] = f[e];
-            }
+            w0[u] = unpack(rb[u].x, rb[u].y);
+            w1[u] = unpack(rb[u].z, rb[u].w);
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                acc[t][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[u], ra[0][t], acc[t][u], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        const int nxt = cur + 1 == NS ? 0 : cur + 1;
+        if (st + 1 < nk) {
+            // stage st + 1 has landed (st + 2 may be in flight) and every wave has read its last
+            // operands of stage st, whose slot takes stage st + 3
+            if (st + 2 < nk) wide_wait<NL, true>();
+            else wide_wait<0, true>();
+            if (st + NS < nk) issue(st + NS, cur);
+            read_a(nxt, 0);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                rb[u] = *reinterpret_cast<const u32x4 *>(smem + nxt * kTallSB + boff + u * 1024);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                acc[t][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[u], ra[1][t], acc[t][u], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
     }
+    wide_wait<0, true>();  // the ring is free
+    float *S = reinterpret_cast<float *>(smem);
+    if (tid < kWideBN) S[tid] = __fmul_rn(in_scale, col_scale);  // f32(inScale * scale[n])
+    __syncthreads();
+    wide_store<8, kTallBM>(acc, 128 * wm, smem + 1024, S, dst, m0, n0, wn, M, N, out_kind, out_scale);
 }
 
 // ---- per-stream workspace for the snapped activation codes ------------------------------------
@@ -1543,6 +1696,24 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     }
     const uint8_t *w = reinterpret_cast<const uint8_t *>(wq);
     if (c == K_WIDE) {
+        // the tall tile where its one block per CU leaves at most a tenth of the CUs without a tile in
+        // the last round: us in a graph, wide -> tall, 2048 x 1536 -> 6144 (256 tiles) 26.6 -> 22.8,
+        // 2048 x 6144 -> 6144 82.2 -> 67.0; 2000 x 2048 -> 5000 (216 tiles) 30.0 / 30.2, 1500 x 1536 ->
+        // 6144 (192) 21.1 / 23.7, 1024 x 1536 -> 6144 (128) 14.5 / 21.9
+        const int tall_m = (m + kTallBM - 1) / kTallBM, tall = tall_m * ((n + kWideBN - 1) / kWideBN);
+        const int cus = device_cu_count(), rounds = (tall + cus - 1) / cus;
+        if (10 * (int64_t)tall >= 9 * (int64_t)rounds * cus && k >= kTallNS * kTileBK) {
+            const int tiles_n = (n + kWideBN - 1) / kWideBN;
+            const dim3 grid(tall_m * ((tiles_n + 7) / 8) * 8);
+            if (natural)
+                hipLaunchKernelGGL(qgemm_tall_kernel<true>, grid, dim3(512), 0, stream, codes, w, scales, dst,
+                                   m, n, k, in_scale, out_scale, out_kind, tall_m, tiles_n);
+            else
+                hipLaunchKernelGGL(qgemm_tall_kernel<false>, grid, dim3(512), 0, stream, codes, w, scales, dst,
+                                   m, n, k, in_scale, out_scale, out_kind, tall_m, tiles_n);
+            G4_LAUNCHED("qgemm_tall_kernel");
+            return G4_OK;
+        }
         const int tiles_m = (m + kWideBM - 1) / kWideBM;
         const int tiles_n = (n + kWideBN - 1) / kWideBN;
         const int blocks = tiles_m * ((tiles_n + 7) / 8) * 8;

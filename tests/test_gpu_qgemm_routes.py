@@ -44,3 +44,29 @@ def check_every_kind(gpu, oracle, bits, m, n, k):
 def test_column_tiles(gpu, oracle, bits, m, n, k):
     # 16-wave blocks of one, two and four column tiles and the 4-wave blocks, either side of each line
     check_every_kind(gpu, oracle, bits, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 6144, 512), (2047, 6137, 768), (1793, 5953, 512), (4096, 6144, 512)])
+@pytest.mark.parametrize("xdt", [np.float16, np.int8])
+def test_tall_tiles(gpu, m, n, k, xdt):
+    # whole rounds of 256 x 192 tiles: full tiles, ragged last rows and columns (odd N: the stores fall
+    # back to single outputs), two rounds; 4 and 6 K stages
+    print(f"tall m={m} n={n} k={k} x={np.dtype(xdt)}", flush=True)
+    g = np.random.default_rng(m + n)
+    w = g.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    s = g.uniform(0.005, 0.02, n).astype(np.float32)
+    x = g.standard_normal((m, k)).astype(np.float16)
+    xq = np.clip(np.rint(x.astype(np.float32) / np.float32(0.05)), -128, 127)
+    wc = np.empty((n, k), np.float32)
+    wc[:, 0::2], wc[:, 1::2] = w & 15, w >> 4
+    # |sum| <= 512 x 8 x 128 x 1.5 < 2^24: float32 products and sums are exact in any order
+    acc = xq.astype(np.float32) @ (wc - 8).T
+    y = (np.float32(0.05) * s)[None, :] * acc
+    q = np.clip(np.rint(y / np.float32(0.1)), -128, 127)
+    dw, ds = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(s)
+    dx = gpu.DeviceBuffer.from_array(x if xdt == np.float16 else xq.astype(np.int8))
+    for dt, ref in ((np.int32, acc), (np.int8, q), (np.float32, q * np.float32(0.1))):
+        out = gpu.DeviceBuffer.empty((m, n), dt)
+        out.fill(0x7B)
+        gpu.qgemm(4, dw, ds, dx, out, k, n, m, 0.05, 0.1)
+        assert np.array_equal(out.download(), ref.astype(dt)), dt
