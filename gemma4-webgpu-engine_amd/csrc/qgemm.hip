@@ -6,7 +6,8 @@
 //     in LDS, each 8-code group interleaved [x0 x2 x4 x6 x1 x3 x5 x7] for 4-bit weights so a weight
 //     word's even and odd nibble lanes line up with the codes). The tile kernel takes an int8
 //     caller's natural-order codes as given (and permutes the 4-bit B to match); f16 / f32 input is
-//     snapped once per row by quantize_rows_kernel into a per-stream workspace, interleaved.
+//     snapped once per row by quantize_rows_kernel into a per-stream workspace, interleaved (for the
+//     strip kernel by quantize_strip_kernel, in the order of its lanes).
 //  2. An MFMA kernel contracts codes x weights with v_mfma_i32_16x16x64_i8 in exact int32. The
 //     int32 sums are exact, so the k order the MFMA uses internally is irrelevant; only the A and
 //     B operands have to agree on it, and they do by construction.
@@ -24,6 +25,8 @@
 //                  global -> LDS by direct loads through a 3-4 stage ring, XCD-aware tile order;
 //                  4-bit outputs that fill the chip take 64 x 192 tiles (qgemm_wide_kernel), and
 //                  256 x 192 ones (qgemm_tall_kernel) when those come in nearly whole rounds of CUs.
+//                  f16 / f32 calls whose output one strip of 64 rows x 32 - 64 columns per CU covers
+//                  take qgemm_strip_kernel: K split over the block's waves, no LDS in its K loop.
 #include "g4_internal.h"
 #include "g4_workspace.h"
 
@@ -78,6 +81,41 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(const void
             reinterpret_cast<uint2 *>(codes)[g] = out;
         }
     }
+}
+
+// The snap pass of the strip kernel: its codes in the order its lanes read them. A tile of 16 rows (the
+// last one of `rows` = M % 16) holds, for each 128-code stage and half-step s, the 16-code chunks of lane
+// group g = 0 .. 3, `rows` rows each: chunk (st, s, g, j) at 16 (((2 st + s) 4 + g) rows + j), M * K bytes
+// in all. The half-step's lane group g takes chunk 2 g + s of the stage (4-bit weights, each 8-code group
+// interleaved) or 4 s + g (8-bit). A wave per (tile, stage, s), so its 64 chunks are one 1 KB store.
+template <int BITS, bool F16>
+__global__ __launch_bounds__(256) void quantize_strip_kernel(const void *x, int m, int k, float scale,
+                                                             int8_t *codes) {
+    const SrqScale S = srq_scale(scale);
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int steps = k / (kTileBK / 2);  // (stage, s) pairs
+    const int wave = (int)blockIdx.x * 4 + (threadIdx.x >> 6);  // strip_cols: M * K <= 2^28
+    const int tile = wave / steps, step = wave - tile * steps;
+    const int rows = min(16, m - 16 * tile);
+    if (j >= rows) return;  // a wave past the last tile too: rows <= 0
+    const int chunk = BITS == 4 ? 2 * g + (step & 1) : 4 * (step & 1) + g;
+    const int64_t e = (int64_t)(16 * tile + j) * k + (step >> 1) * kTileBK + 16 * chunk;
+    const u32x4 *p = reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(x) + e * (F16 ? 2 : 4));
+    u32x4 raw[2][F16 ? 1 : 2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < (F16 ? 1 : 2); ++i) raw[h][i] = p[h * (F16 ? 1 : 2) + i];
+    uint2 out[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float v[8];
+        widen8<F16>(raw[h], v);
+        srq_quot8(v, S);
+        out[h] = codes_word2<BITS == 4>(v);
+    }
+    *reinterpret_cast<u32x4 *>(codes + (int64_t)tile * 16 * k + (((int64_t)step * 4 + g) * rows + j) * 16) =
+        u32x4{out[0].x, out[0].y, out[1].x, out[1].y};
 }
 
 // srqCodes as a kernel (quant.ts:309-334), natural order.
@@ -1331,6 +1369,174 @@ __global__ __launch_bounds__(512, 2) void qgemm_tall_kernel(
     wide_store<8, kTallBM>(acc, 128 * wm, smem + 1024, S, dst, m0, n0, wn, M, N, out_kind, out_scale);
 }
 
+// ---- the strip: 64 x BN outputs per block of 8 waves, operands straight to registers -------------
+//
+// For outputs that one such block per CU covers (512 x 6144 -> 1536: 256 strips of 64 x 48). There the
+// tile kernel is bound by LDS: each 128-code stage of a 32 x 96 tile moves 30 KB through it for 96 MFMA
+// cycles per SIMD, since its waves share operands. Here they share none: a wave takes whole stages (wave,
+// wave + 8, ...) of the whole strip, so an operand goes from memory to the registers of the one wave
+// that needs it and LDS carries only the fold of the eight partial strips. A stage is 8 loads of
+// activations and BN / 16 (8-bit: BN / 8) of weights, D stages in flight per wave (2 x 8 waves x 11 KB).
+// The weights are the MFMA's A operand, so a lane holds 4 adjacent columns of one row.
+//
+// The snap pass leaves the codes in the lanes' order (quantize_strip_kernel), so an activation load is 1 KB
+// in a row; read from rows of K bytes instead (16 rows x 64 bytes a load) 512 x 6144 -> 1536 took 24.9 us, and
+// a caller's own int8 codes, which are such rows, stay with the tile kernel (19.5 / 14.2). Measured, us in a
+// graph with f16 x and its snap, tile -> strip: 512 x 6144 -> 1536 18.4 -> 17.2, 512 x 1536 -> 2048 11.2 ->
+// 9.6, 256 x 6144 -> 1536 15.9 -> 12.8, 1024 x 1536 -> 256 10.5 -> 7.9, 2048 x 1536 -> 256 15.1 -> 8.9,
+// 50 x 6144 -> 6000 14.5 -> 11.3, 8-bit 2048 x 1536 -> 256 16.2 -> 9.9. Bound: the 16-row weight loads and
+// the chain of launch, first stage and fold. Three stages in flight per wave: 17.9, 12.7 -> 13.2.
+//
+// XCD x = blockIdx % 8 takes row group x % xm and column group x / xm of the strips (xm x 8 / xm groups),
+// so that the strips of one XCD share its L2's copy of a few rows and columns.
+template <int BITS, int BN>
+__global__ __launch_bounds__(512, 2) void qgemm_strip_kernel(
+    const int8_t *__restrict__ A, const uint8_t *__restrict__ W, const float *__restrict__ scales,
+    void *dst, int M, int N, int K, float in_scale, float out_scale, int out_kind, int tiles_m,
+    int tiles_n, int xm, int group_m) {
+    constexpr int NT = BN / 16, WH = BITS == 4 ? 1 : 2, WAVES = 8, D = 2;
+    __shared__ __align__(16) v4i red[WAVES][4 * NT][64];
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int group_n = (tiles_n * xm + 7) >> 3;  // ceil(tiles_n / (8 / xm))
+    const int tm = (xcd & (xm - 1)) * group_m + idx % group_m;
+    const int tn = xcd / xm * group_n + idx / group_m;
+    if (tm >= tiles_m || tn >= tiles_n) return;  // whole block, before any barrier
+    const int m0 = tm * 64, n0 = tn * BN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, g = lane >> 4;
+    // byte offsets of this lane's rows and columns (below 2^31: at most 64 x 256 rows, K <= 16384)
+    const int row_bytes = BITS == 4 ? K >> 1 : K;
+    uint32_t ao[4], wo[NT];
+    int as[4];  // bytes from one half-step to the next
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int r0 = min(m0 + 16 * t, (M - 1) & ~15), rows = min(16, M - r0);
+        ao[t] = (uint32_t)r0 * K + (g * rows + min(j, rows - 1)) * 16;
+        as[t] = 64 * rows;
+    }
+#pragma unroll
+    for (int u = 0; u < NT; ++u) wo[u] = (uint32_t)min(n0 + 16 * u + j, N - 1) * row_bytes + 16 * g;
+    const uint8_t *A8 = reinterpret_cast<const uint8_t *>(A);
+
+    v4i acc[4][NT];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[t][u] = v4i{0, 0, 0, 0};
+    v4i ra[D][2][4];
+    u32x4 rw[D][NT][WH];
+    auto load = [&](int d, int st) {
+        const uint8_t *w = W + (int64_t)st * (BITS == 4 ? 64 : 128);
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int h = 0; h < WH; ++h) rw[d][u][h] = *reinterpret_cast<const u32x4 *>(w + wo[u] + 64 * h);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                ra[d][s][t] = *reinterpret_cast<const v4i *>(A8 + (int64_t)(2 * st + s) * as[t] + ao[t]);
+    };
+    auto compute = [&](int d) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            v4i b[NT];
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                if (BITS == 8) {
+                    b[u] = __builtin_bit_cast(v4i, rw[d][u][s & (WH - 1)]);
+                } else {
+                    const uint32_t w0 = s == 0 ? rw[d][u][0].x : rw[d][u][0].z;
+                    const uint32_t w1 = s == 0 ? rw[d][u][0].y : rw[d][u][0].w;
+                    b[u] = v4i{(int)nib_even16(w0), (int)nib_odd16(w0), (int)nib_even16(w1), (int)nib_odd16(w1)};
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[u], ra[d][s][t], acc[t][u], 0, 0, 0);
+        }
+    };
+    const int nk = K / kTileBK;
+    const int cnt = wave < nk ? (nk - wave + WAVES - 1) / WAVES : 0;  // this wave's stages
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < cnt) load(d, wave + WAVES * d);
+    int i = 0;
+    for (; i + 2 * D <= cnt; i += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            compute(d);
+            load(d, wave + WAVES * (i + d + D));
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {  // fewer than 2 D stages left, the first D of them loaded
+        if (i + d < cnt) compute(d);
+        if (i + d + D < cnt) load(d, wave + WAVES * (i + d + D));
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (i + d + D < cnt) compute(d);
+
+    // The fold. Lane (j, g) of tile (t, u) holds row 16 t + j, columns 16 u + 4 g .. + 3; its place in the
+    // tile is (g, j ^ (4 u + g)), so that both the waves' writes (16 places per g) and the reads along a
+    // row (4 g x NT tiles at one j) spread over the banks.
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) red[wave][t * NT + u][16 * g + (j ^ ((4 * u + g) & 15))] = acc[t][u];
+    __syncthreads();
+    bool o_ok;
+    const float orcp = srq_recip(out_scale, o_ok);
+    constexpr int UNITS = 64 * (BN / 4);  // groups of 4 outputs, row by row
+#pragma unroll
+    for (int e = 0; e < (UNITS + 511) / 512; ++e) {
+        const int q = tid + 512 * e;
+        if (UNITS % 512 != 0 && q >= UNITS) break;
+        const int row = q / (BN / 4), c4 = q % (BN / 4);
+        const int u = c4 >> 2, gg = c4 & 3;
+        v4i v{0, 0, 0, 0};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w)
+            v += red[w][(row >> 4) * NT + u][16 * gg + ((row & 15) ^ (c4 & 15))];
+        const int m = m0 + row, n = n0 + 4 * c4;
+        if (m >= M || n >= N) continue;
+        const int live = min(4, N - n);
+        const int64_t o = (int64_t)m * N + n;
+        const bool whole = live == 4 && (o & 3) == 0;
+        if (BITS == 4) v >>= 4;  // the sums are of 16 * code
+        if (out_kind == G4_KIND_I32) {
+            int *d = reinterpret_cast<int *>(dst) + o;
+            for (int c = 0; c < live; ++c) d[c] = v[c];
+            continue;
+        }
+        float y[4], code[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            y[c] = __fmul_rn(__fmul_rn(in_scale, scales[min(n + c, N - 1)]), (float)v[c]);
+            code[c] = out_scale != 0.0f ? srq_code_fast(y[c], out_scale, orcp, o_ok) : 0.0f;
+        }
+        if (out_kind == G4_KIND_I8) {
+            int8_t *d = reinterpret_cast<int8_t *>(dst) + o;
+            uint32_t word = 0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) word |= ((uint32_t)(int)code[c] & 0xffu) << (8 * c);
+            if (whole) *reinterpret_cast<uint32_t *>(d) = word;
+            else for (int c = 0; c < live; ++c) d[c] = (int8_t)(word >> (8 * c));
+        } else {
+            float *d = reinterpret_cast<float *>(dst) + o;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (out_scale != 0.0f) y[c] = __fmul_rn(code[c], out_scale);
+            if (whole) *reinterpret_cast<float4 *>(d) = make_float4(y[0], y[1], y[2], y[3]);
+            else for (int c = 0; c < live; ++c) d[c] = y[c];
+        }
+    }
+}
+
 // ---- per-stream workspace for the snapped activation codes ------------------------------------
 
 namespace {
@@ -1508,6 +1714,44 @@ int linear_split_acc(int bits, const uint8_t *wq, const float *scales, const int
     return G4_OK;
 }
 
+// The strip's columns (32, 48 or 64) for a K_TILE128 call whose activations are snapped here, or 0 for the
+// tile kernel: the fewest whose grid of 64-row strips fits the CUs once (a second round would run on a few
+// CUs). M > 32: below, half of a strip would be padding rows. 8-bit weights (twice the bytes per column)
+// from one stage per wave on: 512 x 1536 -> 1024 tile 9.3, strip 8.4 us; 512 x 256 -> 1536 6.6, 7.4.
+static int strip_cols(int bits, int m, int n, int k) {
+    const int64_t tiles_m = (m + 63) / 64;
+    if (m <= 32 || (bits == 8 && k < 8 * kTileBK)) return 0;
+    for (int bn = 32; bn <= 64; bn += 16)
+        if (tiles_m * ((n + bn - 1) / bn) <= device_cu_count()) return bn;
+    return 0;
+}
+
+template <int BITS>
+static int launch_strip(int bn, const int8_t *codes, const uint8_t *w, const float *scales,
+                        void *dst, int m, int n, int k, float in_scale, float out_scale, int out_kind,
+                        hipStream_t stream) {
+    const int tiles_m = (m + 63) / 64, tiles_n = (n + bn - 1) / bn;
+    // the XCD grouping that reads the fewest bytes per XCD (rows K bytes, columns K BITS / 8)
+    int xm = 1, blocks = 0;
+    int64_t least = INT64_MAX;
+    for (int x = 1; x <= 8; x *= 2) {
+        const int gm = (tiles_m + x - 1) / x, gn = (tiles_n * x + 7) / 8;
+        const int64_t bytes = (int64_t)gm * 64 * 8 + (int64_t)gn * bn * BITS;
+        if (8 * gm * gn <= device_cu_count() + 32 && bytes < least) least = bytes, xm = x, blocks = 8 * gm * gn;
+    }
+    if (blocks == 0) blocks = 8 * tiles_m * ((tiles_n + 7) / 8);
+    const int group_m = (tiles_m + xm - 1) / xm;
+#define G4_STRIP(BN_)                                                                                \
+    hipLaunchKernelGGL((qgemm_strip_kernel<BITS, BN_>), dim3(blocks), dim3(512), 0, stream, codes, w, \
+                       scales, dst, m, n, k, in_scale, out_scale, out_kind, tiles_m, tiles_n, xm, group_m)
+    if (bn == 32) G4_STRIP(32);
+    else if (bn == 48) G4_STRIP(48);
+    else G4_STRIP(64);
+#undef G4_STRIP
+    G4_LAUNCHED("qgemm_strip_kernel");
+    return G4_OK;
+}
+
 template <int BITS>
 static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, const float *scales,
                        void *dst, int m, int n, int k, float in_scale, float out_scale,
@@ -1609,7 +1853,8 @@ static bool needs_codes_buffer(int bits, int m, int n, int k, float in_scale, in
 // The snap pass: M * K f16 / f32 activations (16-byte aligned, K % 128 == 0) into int8 codes in
 // `given` or the stream's workspace, interleaved per 8-code group when perm (the tile kernels'
 // 4-bit layout) or in natural order.
-static int snap_pass(const void *x, int x_kind, int m, int k, float in_scale, bool perm,
+enum CodeOrder { kCodesNatural, kCodesPerm, kCodesStrip4, kCodesStrip8 };
+static int snap_pass(const void *x, int x_kind, int m, int k, float in_scale, CodeOrder order,
                      hipStream_t stream, int8_t *given, const int8_t **codes) {
     void *ws = given;
     if (!ws) {
@@ -1620,21 +1865,29 @@ static int snap_pass(const void *x, int x_kind, int m, int k, float in_scale, bo
     const int64_t per_block = (int64_t)kQuantThreads * kQuantGroups;
     const int qblocks = (int)std::min<int64_t>((n8 + per_block - 1) / per_block, 8 * 1024);
     int8_t *wsc = reinterpret_cast<int8_t *>(ws);
-    if (x_kind == G4_KIND_F16) {
-        if (perm)
-            hipLaunchKernelGGL((quantize_rows_kernel<true, true>), dim3(qblocks), dim3(kQuantThreads), 0,
-                               stream, x, n8, in_scale, wsc);
-        else
-            hipLaunchKernelGGL((quantize_rows_kernel<false, true>), dim3(qblocks), dim3(kQuantThreads), 0,
-                               stream, x, n8, in_scale, wsc);
-    } else {
-        if (perm)
-            hipLaunchKernelGGL((quantize_rows_kernel<true, false>), dim3(qblocks), dim3(kQuantThreads), 0,
-                               stream, x, n8, in_scale, wsc);
-        else
-            hipLaunchKernelGGL((quantize_rows_kernel<false, false>), dim3(qblocks), dim3(kQuantThreads), 0,
-                               stream, x, n8, in_scale, wsc);
+    if (order == kCodesStrip4 || order == kCodesStrip8) {
+        const int64_t waves = (int64_t)((m + 15) / 16) * (k / (kTileBK / 2));
+        const dim3 grid((unsigned)((waves + 3) / 4));
+#define G4_SNAP(BITS_, F16_)                                                                        \
+    hipLaunchKernelGGL((quantize_strip_kernel<BITS_, F16_>), grid, dim3(256), 0, stream, x, m, k, in_scale, wsc)
+        if (order == kCodesStrip4 && x_kind == G4_KIND_F16) G4_SNAP(4, true);
+        else if (order == kCodesStrip4) G4_SNAP(4, false);
+        else if (x_kind == G4_KIND_F16) G4_SNAP(8, true);
+        else G4_SNAP(8, false);
+#undef G4_SNAP
+        G4_LAUNCHED("quantize_strip_kernel");
+        *codes = wsc;
+        return G4_OK;
     }
+    const bool perm = order == kCodesPerm;
+#define G4_SNAP(PERM_, F16_)                                                                        \
+    hipLaunchKernelGGL((quantize_rows_kernel<PERM_, F16_>), dim3(qblocks), dim3(kQuantThreads), 0, \
+                       stream, x, n8, in_scale, wsc)
+    if (perm && x_kind == G4_KIND_F16) G4_SNAP(true, true);
+    else if (perm) G4_SNAP(true, false);
+    else if (x_kind == G4_KIND_F16) G4_SNAP(false, true);
+    else G4_SNAP(false, false);
+#undef G4_SNAP
     G4_LAUNCHED("quantize_rows_kernel");
     *codes = wsc;
     return G4_OK;
@@ -1670,7 +1923,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
         // the snap pass first (natural order: the kernel's int8 path interleaves for 4-bit).
         if (x_kind != G4_KIND_I8 && small_presnap(m, n, k)) {
             const int8_t *codes = nullptr;
-            int rc = snap_pass(x, x_kind, m, k, in_scale, false, stream, given_codes, &codes);
+            int rc = snap_pass(x, x_kind, m, k, in_scale, kCodesNatural, stream, given_codes, &codes);
             if (rc) return rc;
             x = codes;
             x_kind = G4_KIND_I8;
@@ -1690,8 +1943,11 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     // workspace, interleaved for 4-bit weights so the tile kernel needs no permutes.
     const int8_t *codes = reinterpret_cast<const int8_t *>(x);
     const bool natural = x_kind == G4_KIND_I8;
+    const int strip = c == K_TILE128 && !natural ? strip_cols(bits, m, n, k) : 0;
     if (!natural) {
-        int rc = snap_pass(x, x_kind, m, k, in_scale, bits == 4, stream, given_codes, &codes);
+        const CodeOrder order = strip ? (bits == 4 ? kCodesStrip4 : kCodesStrip8)
+                                      : bits == 4 ? kCodesPerm : kCodesNatural;
+        int rc = snap_pass(x, x_kind, m, k, in_scale, order, stream, given_codes, &codes);
         if (rc) return rc;
     }
     const uint8_t *w = reinterpret_cast<const uint8_t *>(wq);
@@ -1726,6 +1982,10 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
         G4_LAUNCHED("qgemm_wide_kernel");
         return G4_OK;
     }
+    if (strip && bits == 4)
+        return launch_strip<4>(strip, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream);
+    if (strip)
+        return launch_strip<8>(strip, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream);
     if (bits == 4)
         return launch_tile<4>(codes, natural, w, scales, dst, m, n, k, in_scale, out_scale, out_kind,
                               stream);

@@ -70,3 +70,14 @@ def test_tall_tiles(gpu, m, n, k, xdt):
         out.fill(0x7B)
         gpu.qgemm(4, dw, ds, dx, out, k, n, m, 0.05, 0.1)
         assert np.array_equal(out.download(), ref.astype(dt)), dt
+
+
+@pytest.mark.parametrize("bits,m,n,k", [
+    # strips of 64 rows x 32, 48 and 64 columns, either side of one per CU; ragged row tiles (M % 16 of 1,
+    # 15 and 0), ragged columns, fewer stages than waves, and 1 .. 6 stages per wave with a remainder
+    (4, 33, 8192, 512), (4, 64, 8193, 256), (4, 65, 6145, 768), (4, 129, 4097, 1280), (4, 513, 1363, 2304),
+    (4, 512, 2049, 1280), (4, 1023, 31, 1536), (4, 1040, 257, 1024), (4, 177, 1535, 5120), (4, 191, 2700, 6144),
+    (8, 1025, 130, 1024), (8, 65, 6145, 1152), (8, 2000, 257, 1024), (8, 143, 1501, 2176),
+])
+def test_strips(gpu, oracle, bits, m, n, k):
+    check_every_kind(gpu, oracle, bits, m, n, k)
