@@ -18,7 +18,7 @@
 //   3 <= M <= 32, and more rows while one block of 32 rows x 16 columns per CU covers the output
 //                  qgemm_small_kernel: one launch with the snap fused (codes in LDS), 16 weight
 //                  rows per block, the block's waves split K (4, or 16 when the grid is no wider
-//                  than the CU count), an LDS fold of the partials; several projections of the
+//                  than the CU count), 16 or 32 rows (small_rows), an LDS fold of the partials; several projections of the
 //                  same x can share one grid (linear_grouped).
 //   larger outputs, or over 32768+ rows
 //                  qgemm_tile_kernel: 64 x 96 output tiles, activation codes and weights streamed
@@ -1597,6 +1597,16 @@ static int small_col_tiles(int64_t blocks16, int mt, int k, bool paired) {
     return blocks16 <= 4 * cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
 }
 
+// The rows of a small-M block: 16, also past 16 rows while the grid of 16-row blocks still fits the CUs once
+// (a block then copies or snaps half of the codes, and twice the CUs work on the call; the weights' second
+// read comes from L2), else 32. Us in a graph, 32 -> 16 rows: 32 x 6144 -> 1536 int8 codes 6.6 -> 5.2, 32 x
+// 1536 -> 256 3.9 -> 3.5; with the snap fused 64 x 1536 -> 256 f32 6.5 -> 4.7, 64 x 2048 -> 1024 f16 7.9 ->
+// 5.5, 24 x 1536 -> 1536 f16 5.9 -> 4.9. Wider grids share one copy of the codes over more columns instead
+// (small_col_tiles).
+static int small_rows(int64_t blocks16, int m) {
+    return m <= 16 || blocks16 * ((m + 15) / 16) <= device_cu_count() ? 16 : 32;
+}
+
 enum KernelChoice { K_GEMV = 0, K_SKINNY16, K_SKINNY32, K_TILE128, K_GEMV_F32, K_GEMV_COLS,
                     K_SERIAL8, K_WIDE };
 
@@ -1670,9 +1680,10 @@ static void launch_small_t(const void *x, int x_kind, const SmallJobs &jobs, int
 }
 
 // epi: 0 plain (any job count), 1 the paired gate/up gelu epilogue (4-bit), 2 the f32-vector one.
-static int launch_small(int bits, int mt, int epi, const void *x, int x_kind, const SmallJobs &jobs,
+static int launch_small(int bits, int epi, const void *x, int x_kind, const SmallJobs &jobs,
                         int m, int k, float in_scale, float out_scale, int out_kind,
                         hipStream_t stream) {
+    const int mt = small_rows(jobs.block_end[jobs.count - 1], m);
 #define G4_SMALL(B, T, E) launch_small_t<B, T, E>(x, x_kind, jobs, m, k, in_scale, out_scale, out_kind, stream)
     if (epi == 1 && mt == 16) G4_SMALL(4, 16, 1);
     else if (epi == 1) G4_SMALL(4, 32, 1);
@@ -1702,11 +1713,12 @@ int linear_split_acc(int bits, const uint8_t *wq, const float *scales, const int
     jobs.n[0] = n;
     jobs.block_end[0] = (n + 15) / 16;
     jobs.count = 1;
-    if (bits == 4 && m <= 16)
+    const int mt = small_rows((int64_t)jobs.block_end[0] * splits, m);
+    if (bits == 4 && mt == 16)
         launch_small_t<4, 16, 0>(x, G4_KIND_I8, jobs, m, k, 1.0f, 0.0f, G4_KIND_I32, stream, splits);
     else if (bits == 4)
         launch_small_t<4, 32, 0>(x, G4_KIND_I8, jobs, m, k, 1.0f, 0.0f, G4_KIND_I32, stream, splits);
-    else if (m <= 16)
+    else if (mt == 16)
         launch_small_t<8, 16, 0>(x, G4_KIND_I8, jobs, m, k, 1.0f, 0.0f, G4_KIND_I32, stream, splits);
     else
         launch_small_t<8, 32, 0>(x, G4_KIND_I8, jobs, m, k, 1.0f, 0.0f, G4_KIND_I32, stream, splits);
@@ -1834,7 +1846,7 @@ static bool small_presnap(int m, int n, int k) {
     // caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
     // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager)
     if (m > 32) return 32 * k > 64 * 1024;
-    const int ct = std::max(1, small_col_tiles(blocks, m <= 16 ? 16 : 32, k, false));
+    const int ct = std::max(1, small_col_tiles(blocks, small_rows(blocks, m), k, false));
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) &&
            ((blocks + ct - 1) / ct + cus - 1) / cus * m * k >= 48 * 1024;
 }
@@ -1935,7 +1947,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
         jobs.n[0] = n;
         jobs.block_end[0] = (n + 15) / 16;
         jobs.count = 1;
-        return launch_small(bits, c == K_SKINNY16 ? 16 : 32, 0, x, x_kind, jobs, m, k, in_scale,
+        return launch_small(bits, 0, x, x_kind, jobs, m, k, in_scale,
                             out_scale, out_kind, stream);
     }
     // An int8 caller's natural-order codes go to the tile kernel as given (one launch; the 4-bit
@@ -2025,7 +2037,7 @@ int linear_grouped(int bits, const void *x, int x_kind, int k, int m, float in_s
         jobs.block_end[i] = blocks;
     }
     jobs.count = count;
-    return launch_small(bits, m <= 16 ? 16 : 32, 0, x, x_kind, jobs, m, k, in_scale, out_scale,
+    return launch_small(bits, 0, x, x_kind, jobs, m, k, in_scale, out_scale,
                         out_kind, as_stream(stream));
 }
 
@@ -2055,7 +2067,7 @@ int linear_gelu(int bits, const void *x, int k, int m, float in_scale, float out
     jobs.aux = up_vec;
     jobs.aux_stride = up_stride;
     jobs.act_scale = act_scale;
-    rc = launch_small(bits, c == K_SKINNY16 ? 16 : 32, w_up ? 1 : 2, x, G4_KIND_I8, jobs, m, k,
+    rc = launch_small(bits, w_up ? 1 : 2, x, G4_KIND_I8, jobs, m, k,
                       in_scale, out_scale, G4_KIND_I8, as_stream(stream));
     if (rc == G4_OK) *launched = true;
     return rc;
