@@ -1,5 +1,6 @@
 // Host runtime of libg4w8a8: the last-error string, device memory, streams and events, the byte
 // fill kernel and the pure table split planner (src/tableSplit.ts).
+#include "g4_graph_replay.h"
 #include "g4_internal.h"
 
 #include <algorithm>
@@ -391,23 +392,30 @@ int g4_graph_launch(void *graph_exec, void *stream) {
     bool direct = !g->chain.empty();
     if (direct) {
         // on a capturing stream, or with another device current, it stays a graph launch
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         int dev = -1;
-        G4_HIP(hipStreamIsCapturing(as_stream(stream), &st));
+        G4_HIP(hipStreamIsCapturing(as_stream(stream), &cap));
         G4_HIP(hipGetDevice(&dev));
-        direct = st == hipStreamCaptureStatusNone && dev == g->device;
+        direct = cap == hipStreamCaptureStatusNone && dev == g->device;
     }
     std::lock_guard<std::mutex> lock(launch_lock(stream));
-    if (direct) {
-        for (const hipKernelNodeParams &k : g->chain)
-            G4_HIP(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes,
-                                   as_stream(stream)));
-    } else {
-        G4_HIP(hipGraphLaunch(g->exec, as_stream(stream)));
-    }
-    G4_HIP(hipEventRecord(g->done, as_stream(stream)));
-    g->launched = true;
-    return G4_OK;
+    const hipStream_t st = as_stream(stream);
+    return replay_chain(
+        direct ? g->chain.size() : 1,
+        [&](size_t i) -> int {
+            if (!direct) {
+                G4_HIP(hipGraphLaunch(g->exec, st));
+                return G4_OK;
+            }
+            const hipKernelNodeParams &k = g->chain[i];
+            G4_HIP(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, st));
+            return G4_OK;
+        },
+        [&]() -> int {
+            G4_HIP(hipEventRecord(g->done, st));
+            return G4_OK;
+        },
+        [&] { return (int)hipStreamSynchronize(st); }, &g->launched);
 }
 
 int g4_graph_destroy(void *graph_exec) {
