@@ -95,8 +95,9 @@ int g4_event_elapsed_ms(float *ms, void *start, void *end);
  * inside a capture is refused with G4_ERR_INVALID. A workspace whose address a capture took is never
  * freed (a graph may be replayed later, on any stream); g4_stream_destroy frees the stream's
  * workspace otherwise. g4_graph_destroy waits for the graph's own last launch (an event recorded
- * after each g4_graph_launch, on the stream it was launched on), not for the whole device, and
- * releases the graph even when that wait fails. Launches of one graph on several streams must be
+ * after each g4_graph_launch, on the stream it was launched on, with a system-scope fence: what the
+ * launch wrote to host memory can be read), not for the whole device, and releases the graph even
+ * when that wait fails. Launches of one graph on several streams must be
  * ordered by the caller (the event marks the most recent launch). g4_graph_end_capture refuses
  * (G4_ERR_INVALID, nothing instantiated, the stream out of capture) a graph holding anything but
  * kernels, device-to-device copies, events and empty nodes: a captured copy to or from host memory

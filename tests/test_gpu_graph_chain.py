@@ -1,6 +1,8 @@
 """Graph replays around the length where a chain of kernels stops being replayed as its launches:
 every replay against the eager result with eager work between, and destroy waiting for the last
 replay."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -50,3 +52,26 @@ def test_destroy_waits_for_the_last_replay(gpu, kernels):
     assert np.all(got == kernels)
     st.close()
     other.close()
+
+
+@pytest.mark.parametrize("kernels", [1, 6, 20])
+def test_destroy_orders_host_memory(gpu, kernels):
+    # the graph writes pinned host memory; after the destroy the host reads it with no other wait
+    print(f"graph of {kernels} fills of host memory destroyed right after its launch", flush=True)
+    st = gpu.Stream()
+    n = 8 << 20
+    host = ctypes.c_void_p()
+    gpu._check(gpu.lib().g4_host_alloc(ctypes.byref(host), n))
+    seen = np.ctypeslib.as_array(ctypes.cast(host, ctypes.POINTER(ctypes.c_uint8)), (n,))
+    try:
+        for rep in range(3):
+            seen[:] = 0
+            g = gpu.Graph(st, lambda: [gpu._check(gpu.lib().g4_fill_u8(host, i + 1, n, st.handle))
+                                       for i in range(kernels)])
+            g.launch()
+            g.close()
+            assert np.all(seen == kernels), rep
+    finally:
+        st.synchronize()
+        gpu.lib().g4_host_free(host)
+        st.close()
