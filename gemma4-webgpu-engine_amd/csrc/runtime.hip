@@ -292,18 +292,32 @@ struct G4Graph {
     std::vector<hipKernelNodeParams> chain;
 };
 
-// Where kernel launches stop being cheaper than one graph launch. Us a replay with its event, as
-// launches / as a graph launch: empty kernels, 1: 5.1 / 15.3, 3: 8.5 / 15, 8: 18.5 / 24 (2.3 against
-// 1.7 per further kernel, so even near 16); a layer's seven linears at 8 tokens 37.6 / 45.0, split
-// attention of 32 rows (3 kernels) 64.8 / 72.3 (a graph launch starts about 7 us after the work
-// before it). At 183 and 393 kernels (the decode step) the two differ by under 1% and one graph
-// launch takes less host time.
-constexpr size_t kChainMax = 12;
+// Where kernel launches stop being cheaper than one graph launch. Us a replay, as launches / as a graph
+// launch. Queued behind each other: empty kernels, 1: 6.6 / 17.7, 3: 10.4 / 19.2, 6: 16.0 / 22.3, 8: 20.3 /
+// 25.9, 10: 25-31 / 29, 12: 30-45 / 32; linears at 8 tokens, 7: 35.9 / 40.8, 9: 40.0 / 44.4, 11: 47.9 / 51.7 (a
+// graph launch starts about 7 us after the work before it).
+constexpr size_t kChainMax = 10;
+// Waited for one by one, a replay of up to 6 kernels is still better as launches (empty, 6: 23 / 32; linears,
+// 6: 37 / 52); past that its commands come to eight with the event, from which on the runtime takes 12 us more
+// to enqueue them and 15 us more to wait (empty, 7: 41 / 32, 8: 43 / 32; linears, 7: 60 / 49). Longer chains are
+// therefore launches only while the replay before is still running, which tells the two uses apart.
+constexpr size_t kChainAlone = 6;
 
 // One launch is one unit of its stream's order also where several threads launch on it.
 static std::mutex &launch_lock(void *stream) {
     static std::mutex locks[16];
     return locks[(reinterpret_cast<uintptr_t>(stream) >> 6) % 16];
+}
+
+// Whether the graph's last replay is still running. The query is one that a capture of this thread (or a
+// global one of another) would not survive, so it is made in the relaxed mode.
+static bool replay_running(const G4Graph *g) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (!g->launched || hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+    const hipError_t state = hipEventQuery(g->done);
+    if (state != hipSuccess) (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return state == hipErrorNotReady;
 }
 
 // The nodes of `graph` in order when it is one chain of at most kChainMax ordinary kernels (each
@@ -399,6 +413,7 @@ int g4_graph_launch(void *graph_exec, void *stream) {
         direct = cap == hipStreamCaptureStatusNone && dev == g->device;
     }
     std::lock_guard<std::mutex> lock(launch_lock(stream));
+    if (direct && g->chain.size() > kChainAlone) direct = replay_running(g);
     const hipStream_t st = as_stream(stream);
     return replay_chain(
         direct ? g->chain.size() : 1,

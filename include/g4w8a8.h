@@ -84,7 +84,7 @@ int g4_event_synchronize(void *event);
 int g4_event_elapsed_ms(float *ms, void *start, void *end);
 
 /* HIP graphs: capture a sequence of enqueues on `stream` once, replay it with one launch (a graph
- * that is one chain of up to 12 kernels is replayed as those kernel launches, which cost less). The
+ * that is one chain of up to 10 kernels is replayed as those kernel launches where they cost less). The
  * decode loop is launch-bound (a launch costs microseconds of host time, more than a small GEMV
  * runs); the reference caches its per-token encode the same way (runtime.ts:702-767). Kernels of
  * this library never allocate or memset inside a capture. g4_qgemm / g4_linear with f16 or f32

@@ -9,7 +9,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kernels", [1, 2, 11, 12, 13, 40])
+@pytest.mark.parametrize("kernels", [1, 2, 6, 7, 10, 11, 12, 13, 40])
 def test_chain_lengths(gpu, kernels):
     print(f"graph chain of {kernels} kernels", flush=True)
     st = gpu.Stream()
@@ -75,3 +75,62 @@ def test_destroy_orders_host_memory(gpu, kernels):
         st.synchronize()
         gpu.lib().g4_host_free(host)
         st.close()
+
+
+@pytest.mark.parametrize("kernels", [6, 7, 10, 11])
+def test_replay_behind_its_own_running_replay(gpu, kernels):
+    # launched again while it runs (as kernel launches), and after it was waited for (as a graph launch)
+    print(f"graph chain of {kernels} kernels, replays in flight", flush=True)
+    st = gpu.Stream()
+    n = 16 << 20
+    b = gpu.DeviceBuffer.empty((n,), np.uint8)
+    outs = [gpu.DeviceBuffer.empty((4096,), np.int8) for _ in range(kernels - 1)]
+    x = gpu.DeviceBuffer.from_array(np.linspace(-8, 8, 4096, dtype=np.float32))
+
+    def record():
+        b.fill(kernels, st.handle)  # long enough that the next launch finds it running
+        for i, o in enumerate(outs):
+            gpu.srq_quantize(x, o, 4096, 0.05 * (i + 1), stream=st.handle)
+
+    g = gpu.Graph(st, record)
+    want = [np.clip(np.rint(np.linspace(-8, 8, 4096, dtype=np.float32) / np.float32(0.05 * (i + 1))), -128, 127)
+            for i in range(kernels - 1)]
+    for rep in range(4):
+        for o in outs + [b]:
+            o.fill(0x7B, st.handle)
+        for _ in range(1 + 3 * (rep % 2)):
+            g.launch()
+        st.synchronize()
+        assert np.all(b.download() == kernels), rep
+        for o, w in zip(outs, want):
+            assert np.array_equal(o.download(), w.astype(np.int8)), rep
+    g.close()
+    st.close()
+
+
+@pytest.mark.parametrize("kernels", [3, 8, 20])
+def test_replay_leaves_a_capture_of_the_thread_alone(gpu, kernels):
+    # a graph launched on another stream while this thread captures: the capture ends as usual
+    print(f"graph of {kernels} kernels launched during a capture", flush=True)
+    st, cap = gpu.Stream(), gpu.Stream()
+    x = gpu.DeviceBuffer.from_array(np.linspace(-8, 8, 4096, dtype=np.float32))
+    outs = [gpu.DeviceBuffer.empty((4096,), np.int8) for _ in range(kernels)]
+    mine = gpu.DeviceBuffer.empty((4096,), np.int8)
+    g = gpu.Graph(st, lambda: [gpu.srq_quantize(x, o, 4096, 0.05, stream=st.handle) for o in outs])
+    g.launch()
+
+    def record():
+        gpu.srq_quantize(x, mine, 4096, 0.1, stream=cap.handle)
+        for _ in range(3):
+            g.launch()
+
+    h = gpu.Graph(cap, record)
+    h.launch()
+    cap.synchronize()
+    st.synchronize()
+    xs = np.linspace(-8, 8, 4096, dtype=np.float32)
+    assert np.array_equal(mine.download(), np.clip(np.rint(xs / np.float32(0.1)), -128, 127).astype(np.int8))
+    for o in outs:
+        assert np.array_equal(o.download(), np.clip(np.rint(xs / np.float32(0.05)), -128, 127).astype(np.int8))
+    for s in (h, g, st, cap):
+        s.close()
