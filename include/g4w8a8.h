@@ -98,7 +98,8 @@ int g4_event_elapsed_ms(float *ms, void *start, void *end);
  * after each g4_graph_launch, on the stream it was launched on, with a system-scope fence: what the
  * launch wrote to host memory can be read), not for the whole device, and releases the graph even
  * when that wait fails. Launches of one graph on several streams must be
- * ordered by the caller (the event marks the most recent launch). g4_graph_end_capture refuses
+ * ordered by the caller (the event marks the most recent launch), and so must other enqueues of
+ * another thread on the stream of a launch: they can run between two of its kernels. g4_graph_end_capture refuses
  * (G4_ERR_INVALID, nothing instantiated, the stream out of capture) a graph holding anything but
  * kernels, device-to-device copies, events and empty nodes: a captured copy to or from host memory
  * would touch that host buffer at every replay, after the enqueuing call returned, and memset
