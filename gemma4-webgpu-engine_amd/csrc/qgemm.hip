@@ -13,7 +13,7 @@
 //     B operands have to agree on it, and they do by construction.
 //  3. The epilogue is the reference's f32(f32(inScale * scale[n]) * f32(acc)) and output snap.
 //
-// Kernels by M (chosen per shape, see pick_kernel):
+// Kernels by M (chosen per call, see route_linear):
 //   M <= 2         the GEMV family (qgemv.hip): bit-identical, cheaper than any tile at this M.
 //   3 <= M <= 32, and more rows while one block of 32 rows x 16 columns per CU covers the output
 //                  qgemm_small_kernel: one launch with the snap fused (codes in LDS), 16 weight
@@ -1608,9 +1608,9 @@ static int small_rows(int64_t blocks16, int m) {
 }
 
 enum KernelChoice { K_GEMV = 0, K_SKINNY16, K_SKINNY32, K_TILE128, K_GEMV_F32, K_GEMV_COLS,
-                    K_SERIAL8, K_WIDE };
+                    K_SERIAL8, K_WIDE, K_STRIP, K_TALL };
 
-// gemm_mode: the caller named qgemm-4bit / qmatmul-8bit (execute.ts matmulKernel in gemm mode).
+// The kernel family of a shape (route_linear goes on to the strip and the tall tile). gemm_mode: the caller named qgemm-4bit / qmatmul-8bit (execute.ts matmulKernel in gemm mode).
 // Uncalibrated qmatmul-8bit then keeps the reference's serial per-output order at any M; the
 // routed g4_linear is gemm mode only above two tokens (a decode step's 8-bit linear is qgemv-8bit,
 // execute.ts:372-375).
@@ -1647,6 +1647,8 @@ static const char *choice_name(KernelChoice c, int bits) {
         case K_SKINNY32: return bits == 4 ? "qgemm-4bit-mfma-small32" : "qmatmul-8bit-mfma-small32";
         case K_TILE128: return bits == 4 ? "qgemm-4bit-mfma-tile" : "qmatmul-8bit-mfma-tile";
         case K_WIDE: return "qgemm-4bit-mfma-wide";
+        case K_TALL: return "qgemm-4bit-mfma-tall";
+        case K_STRIP: return bits == 4 ? "qgemm-4bit-mfma-strip" : "qmatmul-8bit-mfma-strip";
         case K_GEMV_F32: return bits == 4 ? "qgemv-4bit-f32" : "qgemv-8bit-f32";
         case K_SERIAL8: return "qmatmul-8bit-serial";
         default: return bits == 4 ? "qgemv-4bit-columns" : "qgemv-8bit-columns";
@@ -1736,6 +1738,24 @@ static int strip_cols(int bits, int m, int n, int k) {
     for (int bn = 32; bn <= 64; bn += 16)
         if (tiles_m * ((n + bn - 1) / bn) <= device_cu_count()) return bn;
     return 0;
+}
+
+// The tall tile where its one block per CU leaves at most a tenth of the CUs without a tile in the last
+// round: us in a graph, wide -> tall, 2048 x 1536 -> 6144 (256 tiles) 26.6 -> 22.8, 2048 x 6144 -> 6144
+// 82.2 -> 67.0; 2000 x 2048 -> 5000 (216 tiles) 30.0 / 30.2, 1500 x 1536 -> 6144 (192) 21.1 / 23.7, 1024 x
+// 1536 -> 6144 (128) 14.5 / 21.9.
+static bool tall_tiles(int m, int n, int k) {
+    const int64_t tall = (int64_t)((m + kTallBM - 1) / kTallBM) * ((n + kWideBN - 1) / kWideBN);
+    const int64_t cus = device_cu_count(), rounds = (tall + cus - 1) / cus;
+    return k >= kTallNS * kTileBK && 10 * tall >= 9 * rounds * cus;
+}
+
+// The kernel of a call: run_linear launches it and g4_kernel_for_input names it.
+static KernelChoice route_linear(int bits, int m, int n, int k, float in_scale, int x_kind, bool gemm_mode) {
+    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, gemm_mode);
+    if (c == K_TILE128 && x_kind != G4_KIND_I8 && strip_cols(bits, m, n, k)) return K_STRIP;
+    if (c == K_WIDE && tall_tiles(m, n, k)) return K_TALL;
+    return c;
 }
 
 template <int BITS>
@@ -1911,7 +1931,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
                       void *dst, int out_kind, int k, int n, int m, float in_scale,
                       float out_scale, hipStream_t stream, const char *who, bool gemm_mode = true,
                       int8_t *given_codes = nullptr) {
-    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, gemm_mode);
+    const KernelChoice c = route_linear(bits, m, n, k, in_scale, x_kind, gemm_mode);
     if (c == K_SERIAL8) {
         const dim3 grid((n + 255) / 256, m);
         if (x_kind == G4_KIND_F16)
@@ -1955,33 +1975,26 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     // workspace, interleaved for 4-bit weights so the tile kernel needs no permutes.
     const int8_t *codes = reinterpret_cast<const int8_t *>(x);
     const bool natural = x_kind == G4_KIND_I8;
-    const int strip = c == K_TILE128 && !natural ? strip_cols(bits, m, n, k) : 0;
     if (!natural) {
-        const CodeOrder order = strip ? (bits == 4 ? kCodesStrip4 : kCodesStrip8)
-                                      : bits == 4 ? kCodesPerm : kCodesNatural;
+        const CodeOrder order = c == K_STRIP ? (bits == 4 ? kCodesStrip4 : kCodesStrip8)
+                                             : bits == 4 ? kCodesPerm : kCodesNatural;
         int rc = snap_pass(x, x_kind, m, k, in_scale, order, stream, given_codes, &codes);
         if (rc) return rc;
     }
     const uint8_t *w = reinterpret_cast<const uint8_t *>(wq);
+    if (c == K_TALL) {
+        const int tiles_m = (m + kTallBM - 1) / kTallBM, tiles_n = (n + kWideBN - 1) / kWideBN;
+        const dim3 grid(tiles_m * ((tiles_n + 7) / 8) * 8);
+        if (natural)
+            hipLaunchKernelGGL(qgemm_tall_kernel<true>, grid, dim3(512), 0, stream, codes, w, scales, dst,
+                               m, n, k, in_scale, out_scale, out_kind, tiles_m, tiles_n);
+        else
+            hipLaunchKernelGGL(qgemm_tall_kernel<false>, grid, dim3(512), 0, stream, codes, w, scales, dst,
+                               m, n, k, in_scale, out_scale, out_kind, tiles_m, tiles_n);
+        G4_LAUNCHED("qgemm_tall_kernel");
+        return G4_OK;
+    }
     if (c == K_WIDE) {
-        // the tall tile where its one block per CU leaves at most a tenth of the CUs without a tile in
-        // the last round: us in a graph, wide -> tall, 2048 x 1536 -> 6144 (256 tiles) 26.6 -> 22.8,
-        // 2048 x 6144 -> 6144 82.2 -> 67.0; 2000 x 2048 -> 5000 (216 tiles) 30.0 / 30.2, 1500 x 1536 ->
-        // 6144 (192) 21.1 / 23.7, 1024 x 1536 -> 6144 (128) 14.5 / 21.9
-        const int tall_m = (m + kTallBM - 1) / kTallBM, tall = tall_m * ((n + kWideBN - 1) / kWideBN);
-        const int cus = device_cu_count(), rounds = (tall + cus - 1) / cus;
-        if (10 * (int64_t)tall >= 9 * (int64_t)rounds * cus && k >= kTallNS * kTileBK) {
-            const int tiles_n = (n + kWideBN - 1) / kWideBN;
-            const dim3 grid(tall_m * ((tiles_n + 7) / 8) * 8);
-            if (natural)
-                hipLaunchKernelGGL(qgemm_tall_kernel<true>, grid, dim3(512), 0, stream, codes, w, scales, dst,
-                                   m, n, k, in_scale, out_scale, out_kind, tall_m, tiles_n);
-            else
-                hipLaunchKernelGGL(qgemm_tall_kernel<false>, grid, dim3(512), 0, stream, codes, w, scales, dst,
-                                   m, n, k, in_scale, out_scale, out_kind, tall_m, tiles_n);
-            G4_LAUNCHED("qgemm_tall_kernel");
-            return G4_OK;
-        }
         const int tiles_m = (m + kWideBM - 1) / kWideBM;
         const int tiles_n = (n + kWideBN - 1) / kWideBN;
         const int blocks = tiles_m * ((tiles_n + 7) / 8) * 8;
@@ -1994,10 +2007,12 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
         G4_LAUNCHED("qgemm_wide_kernel");
         return G4_OK;
     }
-    if (strip && bits == 4)
-        return launch_strip<4>(strip, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream);
-    if (strip)
-        return launch_strip<8>(strip, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream);
+    if (c == K_STRIP) {
+        const int bn = strip_cols(bits, m, n, k);
+        return bits == 4
+                   ? launch_strip<4>(bn, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream)
+                   : launch_strip<8>(bn, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind, stream);
+    }
     if (bits == 4)
         return launch_tile<4>(codes, natural, w, scales, dst, m, n, k, in_scale, out_scale, out_kind,
                               stream);
@@ -2158,14 +2173,18 @@ int g4_linear(int bits, const void *wq, const float *scales, const void *x, int 
                       m_cols > 2);
 }
 
-int g4_kernel_for_shape(int bits, int m_cols, int num_rows, int k, char *buf, size_t buf_len) {
+int g4_kernel_for_input(int bits, int m_cols, int num_rows, int k, int x_kind, char *buf, size_t buf_len) {
     if (!buf || buf_len == 0) return set_error(G4_ERR_INVALID, "g4_kernel_for_shape: no buffer");
-    const KernelChoice c = pick_kernel(bits, m_cols, num_rows, k, 1.0f, true);
+    const KernelChoice c = route_linear(bits, m_cols, num_rows, k, 1.0f, x_kind, true);
     const char *name = choice_name(c, bits);
     if (c == K_GEMV && m_cols == 1 && stream_class_for(bits, k) >= 0)
         name = bits == 4 ? "qgemv-4bit-stream" : "qgemv-8bit-stream";
     snprintf(buf, buf_len, "%s", name);
     return G4_OK;
+}
+
+int g4_kernel_for_shape(int bits, int m_cols, int num_rows, int k, char *buf, size_t buf_len) {
+    return g4_kernel_for_input(bits, m_cols, num_rows, k, G4_KIND_I8, buf, buf_len);
 }
 
 int g4_srq_quantize(const void *x, int x_kind, int8_t *codes, int64_t n, float scale,

@@ -159,6 +159,8 @@ SIGNATURES = {
     "g4_qgemm_noalloc": (_c_int, [_c_int, _vp, _vp, _vp, _c_int, _vp, _c_int, _c_int, _c_int,
                                   _c_int, _c_float, _c_float, _vp]),
     "g4_qgemm_noalloc_max_codes": (ctypes.c_size_t, []),
+    "g4_kernel_for_input": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, ctypes.c_char_p,
+                                     ctypes.c_size_t]),
     "g4_kernel_for_shape": (_c_int, [_c_int, _c_int, _c_int, _c_int, ctypes.c_char_p,
                                      ctypes.c_size_t]),
     "g4_projection_batch": (_c_int, [_c_int, _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp,
@@ -472,9 +474,9 @@ def linear(bits, wq, scales, x, dst, k, num_rows, m_cols, in_scale=0.0, out_scal
         _check(st)
 
 
-def kernel_for_shape(bits, m_cols, num_rows, k) -> str:
+def kernel_for_shape(bits, m_cols, num_rows, k, x_kind=KIND_I8) -> str:
     buf = ctypes.create_string_buffer(64)
-    _check(lib().g4_kernel_for_shape(bits, m_cols, num_rows, k, buf, 64))
+    _check(lib().g4_kernel_for_input(bits, m_cols, num_rows, k, x_kind, buf, 64))
     return buf.value.decode()
 
 

@@ -232,9 +232,10 @@ napi_value Linear(napi_env env, napi_callback_info info) {
 }
 
 napi_value KernelForShape(napi_env env, napi_callback_info info) {
-    Args a(env, info, 4);
+    Args a(env, info, 5);
     char buf[64];
-    if (throw_status(env, g4_kernel_for_shape(a.i32(0), a.i32(1), a.i32(2), a.i32(3), buf, 64)))
+    if (throw_status(env, g4_kernel_for_input(a.i32(0), a.i32(1), a.i32(2), a.i32(3),
+                                              a.i32(4, G4_KIND_I8), buf, 64)))
         return nullptr;
     napi_value s;
     napi_create_string_utf8(env, buf, strlen(buf), &s);

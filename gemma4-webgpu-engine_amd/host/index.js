@@ -1032,7 +1032,7 @@ module.exports = {
   sliceForRow,
   slicedGatherDispatches,
   GemvPlan,
-  kernelForShape: (bits, m, n, k) => g4().kernelForShape(bits, m, n, k),
+  kernelForShape: (bits, m, n, k, xKind) => g4().kernelForShape(bits, m, n, k, xKind),
   deviceCount: () => g4().deviceCount(),
   setDevice: d => g4().setDevice(d),
   synchronize: () => g4().synchronize(),

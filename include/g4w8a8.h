@@ -161,7 +161,11 @@ int g4_qgemm_noalloc(int bits, const void *wq, const float *scales, const void *
                      float out_scale, void *stream);
 size_t g4_qgemm_noalloc_max_codes(void);
 
-/* Name of the kernel g4_linear picks for a shape, written into buf (NUL terminated). */
+/* Name of the kernel a calibrated g4_qgemm picks for a shape and activation kind, written into buf (NUL
+ * terminated); g4_kernel_for_shape: for int8 codes. The small-M names give the class of M (small16 up
+ * to 16 tokens), not the block's rows. */
+int g4_kernel_for_input(int bits, int m_cols, int num_rows, int k, int x_kind, char *buf,
+                        size_t buf_len);
 int g4_kernel_for_shape(int bits, int m_cols, int num_rows, int k, char *buf, size_t buf_len);
 
 /*

@@ -131,6 +131,21 @@ def test_kernel_choice_per_shape(g4):
     assert g4.kernel_for_shape(4, 3, 262144, 1536) == "qgemm-4bit-mfma-tile"
 
 
+def test_kernel_choice_per_call(g4):
+    """The kernels that the grid's fill (tall tiles) or the activations' kind (strips) decide."""
+    assert g4.kernel_for_shape(4, 2048, 6144, 1536) == "qgemm-4bit-mfma-tall"
+    assert g4.kernel_for_shape(4, 2048, 6144, 1536, g4.KIND_F16) == "qgemm-4bit-mfma-tall"
+    assert g4.kernel_for_shape(4, 2048, 6144, 256) == "qgemm-4bit-mfma-tile"  # two K stages
+    for kind in (g4.KIND_F16, g4.KIND_F32):
+        assert g4.kernel_for_shape(4, 512, 1536, 6144, kind) == "qgemm-4bit-mfma-strip"
+        assert g4.kernel_for_shape(8, 2048, 256, 1536, kind) == "qmatmul-8bit-mfma-strip"
+        assert g4.kernel_for_shape(8, 512, 1536, 256, kind) == "qmatmul-8bit-mfma-tile"
+        assert g4.kernel_for_shape(4, 200, 6144, 1536, kind) == "qgemm-4bit-mfma-tile"
+    # a caller's own codes are in rows, which the strip does not read
+    assert g4.kernel_for_shape(4, 512, 1536, 6144, g4.KIND_I8) == "qgemm-4bit-mfma-tile"
+    assert g4.kernel_for_shape(8, 2048, 256, 1536, g4.KIND_I8) == "qmatmul-8bit-mfma-tile"
+
+
 class _Fake:
     ptr = 0x1000
     kind = 2
