@@ -1740,14 +1740,25 @@ static int strip_cols(int bits, int m, int n, int k) {
     return 0;
 }
 
-// The tall tile where its one block per CU leaves at most a tenth of the CUs without a tile in the last
-// round: us in a graph, wide -> tall, 2048 x 1536 -> 6144 (256 tiles) 26.6 -> 22.8, 2048 x 6144 -> 6144
-// 82.2 -> 67.0; 2000 x 2048 -> 5000 (216 tiles) 30.0 / 30.2, 1500 x 1536 -> 6144 (192) 21.1 / 23.7, 1024 x
-// 1536 -> 6144 (128) 14.5 / 21.9.
+// The tall tile where its rounds of one block per CU are nearly full of tiles. Rounds are those of the
+// busiest XCD (column tiles go to the 8 XCDs in turn), and what fills them is counted in the wide kernel's 64-row
+// tiles, so that rows past M count as empty. One round pays from about three quarters on; several only when
+// nearly full (more so at the K whose wide loop is unrolled), since the wide kernel's blocks, two per CU, follow
+// each other without a gap. Us in a graph, int8 codes, wide / tall at the share of the rounds that is filled:
+// one round, 2048 x 1536 -> 6144 (1.00) 23.9 / 22.6, 400 x 1536 -> 24576 (0.88) 23.0 / 23.6 and K = 6144 73.8 /
+// 66.5, 800 x 1536 -> 12288 (0.81) 23.3 / 21.5, 1500 x 1536 -> 6144 (0.75) 21.1 / 23.7, 281 x 1536 -> 24576 (0.62)
+// 18.8 / 21.3; two, 1024 x 1536 -> 24576 (1.00) 44.5 / 43.1, 904 x 2816 -> 22825 (0.88) 89.9 / 85.8, 876 x 4096 -> 23141 (0.88) 110.1 / 115.5, 800 x 1536 ->
+// 24576 (0.81) 38.7 / 41.9, 513 x 1536 -> 16128 (0.39) 22.4 / 39.4; three, 1500 x 2048 -> 24576 (1.00) 82.5 / 78.9,
+// 1782 x 3840 -> 18964 (0.95) 149.5 / 136.1, 1500 x 1536 -> 16128 (0.69) 48.7 / 61.7.
 static bool tall_tiles(int m, int n, int k) {
-    const int64_t tall = (int64_t)((m + kTallBM - 1) / kTallBM) * ((n + kWideBN - 1) / kWideBN);
-    const int64_t cus = device_cu_count(), rounds = (tall + cus - 1) / cus;
-    return k >= kTallNS * kTileBK && 10 * tall >= 9 * rounds * cus;
+    const int64_t cus = device_cu_count(), per_xcd = cus / 8;
+    const int64_t tiles_n = (n + kWideBN - 1) / kWideBN, xcd_n = (tiles_n + 7) / 8;
+    const int64_t tall_m = (m + kTallBM - 1) / kTallBM, wide_m = (m + kWideBM - 1) / kWideBM;
+    const int64_t rounds = (xcd_n * tall_m + per_xcd - 1) / per_xcd;
+    const int64_t filled = xcd_n * wide_m, room = rounds * per_xcd * (kTallBM / kWideBM);
+    const bool wide_unrolled = k == 12 * kTileBK || k == 16 * kTileBK;  // wide_k_loop's two lengths
+    return k >= kTallNS * kTileBK && 10 * tiles_n * tall_m >= 9 * rounds * cus &&
+           100 * filled >= (rounds == 1 ? 78 : wide_unrolled ? 95 : 92) * room;
 }
 
 // The kernel of a call: run_linear launches it and g4_kernel_for_input names it.

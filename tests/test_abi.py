@@ -141,6 +141,12 @@ def test_kernel_choice_per_call(g4):
         assert g4.kernel_for_shape(8, 2048, 256, 1536, kind) == "qmatmul-8bit-mfma-strip"
         assert g4.kernel_for_shape(8, 512, 1536, 256, kind) == "qmatmul-8bit-mfma-tile"
         assert g4.kernel_for_shape(4, 200, 6144, 1536, kind) == "qgemm-4bit-mfma-tile"
+    # tall tiles need nearly full rounds: of the busiest XCD (16128 columns are 84 tiles, 11 on some XCDs),
+    # and of real rows
+    for m, n in ((281, 24576), (513, 16128), (1500, 16128), (800, 24576), (1576, 6626), (1500, 6144)):
+        assert g4.kernel_for_shape(4, m, n, 1536) == "qgemm-4bit-mfma-wide", (m, n)
+    for m, n in ((400, 24576), (800, 12288), (1024, 24576), (1500, 24576), (1793, 5953)):
+        assert g4.kernel_for_shape(4, m, n, 1536) == "qgemm-4bit-mfma-tall", (m, n)
     # a caller's own codes are in rows, which the strip does not read
     assert g4.kernel_for_shape(4, 512, 1536, 6144, g4.KIND_I8) == "qgemm-4bit-mfma-tile"
     assert g4.kernel_for_shape(8, 2048, 256, 1536, g4.KIND_I8) == "qmatmul-8bit-mfma-tile"
