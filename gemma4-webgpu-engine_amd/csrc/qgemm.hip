@@ -28,6 +28,7 @@
 //                  f16 / f32 calls whose output one strip of 64 rows x 32 - 64 columns per CU covers
 //                  take qgemm_strip_kernel: K split over the block's waves, no LDS in its K loop.
 #include "g4_internal.h"
+#include "g4_strip_grid.h"
 #include "g4_workspace.h"
 
 #include <algorithm>
@@ -1386,9 +1387,7 @@ __global__ __launch_bounds__(512, 2) void qgemm_tall_kernel(
 // 9.6, 256 x 6144 -> 1536 15.9 -> 12.8, 1024 x 1536 -> 256 10.5 -> 7.9, 2048 x 1536 -> 256 15.1 -> 8.9,
 // 50 x 6144 -> 6000 14.5 -> 11.3, 8-bit 2048 x 1536 -> 256 16.2 -> 9.9. Bound: the 16-row weight loads and
 // the chain of launch, first stage and fold. Three stages in flight per wave: 17.9, 12.7 -> 13.2.
-//
-// XCD x = blockIdx % 8 takes row group x % xm and column group x / xm of the strips (xm x 8 / xm groups),
-// so that the strips of one XCD share its L2's copy of a few rows and columns.
+// Blocks and strips: g4_strip_grid.h.
 template <int BITS, int BN>
 __global__ __launch_bounds__(512, 2) void qgemm_strip_kernel(
     const int8_t *__restrict__ A, const uint8_t *__restrict__ W, const float *__restrict__ scales,
@@ -1396,11 +1395,8 @@ __global__ __launch_bounds__(512, 2) void qgemm_strip_kernel(
     int tiles_n, int xm, int group_m) {
     constexpr int NT = BN / 16, WH = BITS == 4 ? 1 : 2, WAVES = 8, D = 2;
     __shared__ __align__(16) v4i red[WAVES][4 * NT][64];
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int group_n = (tiles_n * xm + 7) >> 3;  // ceil(tiles_n / (8 / xm))
-    const int tm = (xcd & (xm - 1)) * group_m + idx % group_m;
-    const int tn = xcd / xm * group_n + idx / group_m;
-    if (tm >= tiles_m || tn >= tiles_n) return;  // whole block, before any barrier
+    int tm = 0, tn = 0;
+    if (!strip_tile(blockIdx.x, tiles_m, tiles_n, xm, group_m, tm, tn)) return;  // whole block, before any barrier
     const int m0 = tm * 64, n0 = tn * BN;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1733,10 +1729,9 @@ int linear_split_acc(int bits, const uint8_t *wq, const float *scales, const int
 // CUs). M > 32: below, half of a strip would be padding rows. 8-bit weights (twice the bytes per column)
 // from one stage per wave on: 512 x 1536 -> 1024 tile 9.3, strip 8.4 us; 512 x 256 -> 1536 6.6, 7.4.
 static int strip_cols(int bits, int m, int n, int k) {
-    const int64_t tiles_m = (m + 63) / 64;
     if (m <= 32 || (bits == 8 && k < 8 * kTileBK)) return 0;
     for (int bn = 32; bn <= 64; bn += 16)
-        if (tiles_m * ((n + bn - 1) / bn) <= device_cu_count()) return bn;
+        if ((int64_t)((m + 63) / 64) * ((n + bn - 1) / bn) <= device_cu_count()) return bn;
     return 0;
 }
 
@@ -1773,20 +1768,10 @@ template <int BITS>
 static int launch_strip(int bn, const int8_t *codes, const uint8_t *w, const float *scales,
                         void *dst, int m, int n, int k, float in_scale, float out_scale, int out_kind,
                         hipStream_t stream) {
-    const int tiles_m = (m + 63) / 64, tiles_n = (n + bn - 1) / bn;
-    // the XCD grouping that reads the fewest bytes per XCD (rows K bytes, columns K BITS / 8)
-    int xm = 1, blocks = 0;
-    int64_t least = INT64_MAX;
-    for (int x = 1; x <= 8; x *= 2) {
-        const int gm = (tiles_m + x - 1) / x, gn = (tiles_n * x + 7) / 8;
-        const int64_t bytes = (int64_t)gm * 64 * 8 + (int64_t)gn * bn * BITS;
-        if (8 * gm * gn <= device_cu_count() + 32 && bytes < least) least = bytes, xm = x, blocks = 8 * gm * gn;
-    }
-    if (blocks == 0) blocks = 8 * tiles_m * ((tiles_n + 7) / 8);
-    const int group_m = (tiles_m + xm - 1) / xm;
+    const StripGrid G = strip_grid(BITS, m, n, bn, device_cu_count());
 #define G4_STRIP(BN_)                                                                                \
-    hipLaunchKernelGGL((qgemm_strip_kernel<BITS, BN_>), dim3(blocks), dim3(512), 0, stream, codes, w, \
-                       scales, dst, m, n, k, in_scale, out_scale, out_kind, tiles_m, tiles_n, xm, group_m)
+    hipLaunchKernelGGL((qgemm_strip_kernel<BITS, BN_>), dim3(G.blocks), dim3(512), 0, stream, codes, w, \
+                       scales, dst, m, n, k, in_scale, out_scale, out_kind, G.tiles_m, G.tiles_n, G.xm, G.group_m)
     if (bn == 32) G4_STRIP(32);
     else if (bn == 48) G4_STRIP(48);
     else G4_STRIP(64);

@@ -78,6 +78,8 @@ def test_tall_tiles(gpu, m, n, k, xdt):
     (4, 33, 8192, 512), (4, 64, 8193, 256), (4, 65, 6145, 768), (4, 129, 4097, 1280), (4, 513, 1363, 2304),
     (4, 512, 2049, 1280), (4, 1023, 31, 1536), (4, 1040, 257, 1024), (4, 177, 1535, 5120), (4, 191, 2700, 6144),
     (8, 1025, 130, 1024), (8, 65, 6145, 1152), (8, 2000, 257, 1024), (8, 143, 1501, 2176),
+    # row groups on every second and fourth XCD, and strips in turn
+    (4, 281, 2048, 256), (4, 513, 1024, 512), (4, 1132, 884, 512), (8, 1100, 850, 1024),
 ])
 def test_strips(gpu, oracle, bits, m, n, k):
     check_every_kind(gpu, oracle, bits, m, n, k)
