@@ -1803,8 +1803,13 @@ static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, cons
 #define G4_TILE(NS_, NAT_, BM_) G4_TILE_K(NS_, NAT_, BM_, 1)
     // a grid of at most one block per CU splits its K stages over two groups of four waves, twice the
     // loads in flight per CU (us in a graph: 128 x 6144 -> 1536 15.3 -> 13.6, 128 x 1536 -> 6144 7.1
-    // -> 6.8, 256 x 2048 -> 1536 7.9 -> 7.4, 8-bit 512 x 1536 -> 256 6.2 -> 5.7; four groups 14.0, 7.1)
-    if (half && tiles_m * tiles_n <= device_cu_count() && nk % 2 == 0 && nk >= 6) {
+    // -> 6.8, 256 x 2048 -> 1536 7.9 -> 7.4, 8-bit 512 x 1536 -> 256 6.2 -> 5.7; four groups 14.0, 7.1).
+    // 8-bit rings take 128 KB (4-bit 80, two blocks per CU), so there one block per CU also has to hold on
+    // the XCD with the most column tiles: 513 x 1536 -> 1024 (34 blocks) 7.2 us without the split, 9.3 with
+    // it. 4-bit 1098 x 3072 -> 402 (35 blocks) 15.1, 14.3.
+    const bool one_per_cu = BITS == 4 ? (int64_t)tiles_m * tiles_n <= device_cu_count()
+                                      : (int64_t)tiles_m * ((tiles_n + 7) / 8) <= device_cu_count() / 8;
+    if (half && one_per_cu && nk % 2 == 0 && nk >= 6) {
         if (nat) G4_TILE_K(4, true, 32, 2);
         else G4_TILE_K(4, false, 32, 2);
     } else if (half) {

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
     (4, 96, 1365, 2048), (4, 97, 1365, 2048), (4, 500, 250, 1536), (4, 64, 40, 2304),
     (4, 130, 1000, 768), (4, 100, 1500, 1024), (4, 256, 1530, 1280), (4, 40, 6100, 1536),  # tile, 6..12 stages
     (8, 33, 17, 512), (8, 64, 256, 1536), (8, 128, 999, 896), (8, 300, 700, 1152), (8, 1030, 70, 640),
+    (8, 512, 1024, 1536), (8, 513, 1024, 768),  # 32 and 34 blocks on one XCD
 ])
 def test_routes(gpu, oracle, bits, m, n, k):
     check_every_kind(gpu, oracle, bits, m, n, k)
