@@ -1582,14 +1582,16 @@ int workspace_forget_stream(void *stream) {
 // -> four: 32 x 1536 -> 8960 11.7 -> 7.2, 16384 12.8 -> 7.7). Past that, 32-row blocks still take
 // four (32 x 1024 -> 24576 14.9 -> 11.9) and 16-row ones, whose codes are half, the 4-wave blocks
 // (8 x 1024 -> 24576 8.1 / 9.5), which also win up to three tiles per CU while their codes take one
-// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). The paired gate / up form stops
+// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). At K = 128 a block has one K step, so a second
+// round of four-tile blocks that is at most half full costs more than it saves (8-bit, 4-wave / four tiles:
+// 683 x 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5). The paired gate / up form stops
 // at two (its four would spill).
 static int small_col_tiles(int64_t blocks16, int mt, int k, bool paired) {
     const int64_t cus = device_cu_count();
     if (blocks16 <= cus) return 1;
     if (blocks16 <= 2 * cus) return 2;
     if (paired) return 0;
-    if (mt > 16) return 4;
+    if (mt > 16) return k == kTileBK && blocks16 > 4 * cus && blocks16 <= 6 * cus ? 0 : 4;
     return blocks16 <= 4 * cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
 }
 
@@ -1863,9 +1865,10 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 static bool small_presnap(int m, int n, int k) {
     const int64_t cus = device_cu_count();
     const int64_t blocks = (n + 15) / 16;
-    // M > 32: one block per CU (pick_kernel). Up to K = 2048 the call stays one launch, which an eager
-    // caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
-    // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager)
+    // M > 32: few blocks per CU, or K = 128 (pick_kernel). Up to K = 2048 the call stays one launch, which an
+    // eager caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
+    // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager). At K = 128 four column tiles share each snap: 8-bit f16 2048 x
+    // 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
     if (m > 32) return 32 * k > 64 * 1024;
     const int ct = std::max(1, small_col_tiles(blocks, small_rows(blocks, m), k, false));
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) &&
