@@ -1575,7 +1575,7 @@ int workspace_forget_stream(void *stream) {
     return G4_OK;
 }
 
-// The column tiles (16 weight rows each) of a 16-wave small-M block for a grid of `blocks16` single
+// The column tiles (16 weight rows each) of a 16-wave small-M block for `rows` block rows of n16 single
 // tiles, or 0 for 4-wave blocks of one tile. The fewest whose grid fits the CUs once (1, 2 or 4): a
 // CU then copies the activation codes once for all of its columns (us in a graph, int8 codes, 4-wave
 // -> two tiles: 32 x 1536 -> 6144 7.5 -> 5.3, 8 x 1536 -> 6144 4.5 -> 4.3, 32 x 6144 -> 6144 23.2 -> 11.2;
@@ -1584,15 +1584,17 @@ int workspace_forget_stream(void *stream) {
 // (8 x 1024 -> 24576 8.1 / 9.5), which also win up to three tiles per CU while their codes take one
 // LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). At K = 128 a block has one K step, so a second
 // round of four-tile blocks that is at most half full costs more than it saves (8-bit, 4-wave / four tiles:
-// 683 x 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5). The paired gate / up form stops
+// 683 x 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5), and so
+// does a grid that two tiles would have fitted but for the odd one (f16 697 x 128 -> 366 5.8 / 7.4). The paired gate / up form stops
 // at two (its four would spill).
-static int small_col_tiles(int64_t blocks16, int mt, int k, bool paired) {
-    const int64_t cus = device_cu_count();
+static int small_col_tiles(int64_t n16, int64_t rows, int mt, int k, bool paired) {
+    const int64_t cus = device_cu_count(), blocks16 = n16 * rows;
     if (blocks16 <= cus) return 1;
-    if (blocks16 <= 2 * cus) return 2;
+    if ((n16 + 1) / 2 * rows <= cus) return 2;
     if (paired) return 0;
-    if (mt > 16) return k == kTileBK && blocks16 > 4 * cus && blocks16 <= 6 * cus ? 0 : 4;
-    return blocks16 <= 4 * cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
+    if (k == kTileBK && mt > 16 && (blocks16 <= 2 * cus || (blocks16 > 4 * cus && blocks16 <= 6 * cus))) return 0;
+    if (mt > 16) return 4;
+    return (n16 + 3) / 4 * rows <= cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
 }
 
 // The rows of a small-M block: 16, also past 16 rows while the grid of 16-row blocks still fits the CUs once
@@ -1612,7 +1614,7 @@ enum KernelChoice { K_GEMV = 0, K_SKINNY16, K_SKINNY32, K_TILE128, K_GEMV_F32, K
 // Uncalibrated qmatmul-8bit then keeps the reference's serial per-output order at any M; the
 // routed g4_linear is gemm mode only above two tokens (a decode step's 8-bit linear is qgemv-8bit,
 // execute.ts:372-375).
-static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, bool gemm_mode) {
+static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, int x_kind, bool gemm_mode) {
     if (in_scale == 0.0f) return bits == 8 && gemm_mode ? K_SERIAL8 : K_GEMV_F32;
     if (m <= 2) return K_GEMV;
     if (k % kTileBK != 0) return K_GEMV_COLS;
@@ -1627,10 +1629,18 @@ static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, b
     // most CUs without work and the others bound by what one CU can fetch (us in a graph, int8 codes,
     // tile -> small: 64 x 1536 -> 2048 6.7 -> 4.0, 64 x 6144 -> 1536 13.6 -> 9.2, 256 x 1536 -> 256 6.7 ->
     // 3.9, 64 x 1536 -> 3072 6.3 -> 4.5, 64 x 6144 -> 4096 13.6 -> 11.1, 128 x 6144 -> 1536 13.6 -> 11.0,
-    // 128 x 2048 -> 1536 7.2 -> 5.5; four tiles per block lose: 64 x 1536 -> 6144 6.7 / 7.2)
-    const int64_t small_blocks = (int64_t)((n + 15) / 16) * ((m + 31) / 32);
-    if (k >= 4 * kTileBK && small_blocks <= (m <= 64 || k >= 2048 ? 2 : 1) * (int64_t)device_cu_count())
-        return K_SKINNY32;
+    // 128 x 2048 -> 1536 7.2 -> 5.5; four tiles per block lose: 64 x 1536 -> 6144 6.7 / 7.2). A grid past the
+    // CUs by a few blocks takes a second round: 8-bit 696 x 3840 -> 360 (264 blocks) 16.3, tile 8.1; 4-bit f16
+    // 1380 x 3328 -> 165 21.8, strip 12.3.
+    const int ct = m <= 64 || k >= 16 * kTileBK ? 2 : 1;
+    const int64_t cus = device_cu_count(), rows = (m + 31) / 32, n16 = (n + 15) / 16;
+    if (k >= 4 * kTileBK && (n16 + ct - 1) / ct * rows <= cus) return K_SKINNY32;
+    // int8 codes on up to three column tiles of the tile kernel, which go to as many of the 8 XCDs: the small-M
+    // kernel still wins with four tiles per block (4-bit, 1652 x 2560 -> 135 14.2 / 7.9, 928 x 8448 -> 257 18.7 /
+    // 21.6, 12 calls of up to 288 columns 0.74 of the tile's time on average; 8-bit 1700 x 2560 -> 140 13.4 / 10.5,
+    // even at K = 3456 and slower on more columns)
+    const bool narrow = bits == 4 ? n <= 3 * kTileBN : n <= 2 * kTileBN && k < 24 * kTileBK;
+    if (x_kind == G4_KIND_I8 && narrow && k >= 16 * kTileBK && n16 * rows <= 2 * cus) return K_SKINNY32;
     // the wide tile once its grid fills the device: 4-bit weights, M >= 256, three K stages
     const int64_t wide_blocks = (int64_t)((m + kWideBM - 1) / kWideBM) * ((n + kWideBN - 1) / kWideBN);
     if (bits == 4 && m >= 256 && k >= kWideNS * kTileBK - kTileBK && wide_blocks >= device_cu_count())
@@ -1660,7 +1670,7 @@ static void launch_small_t(const void *x, int x_kind, const SmallJobs &jobs, int
                            int splits = 1) {
     const int ksplit = splits > 1 ? k / splits : 0;
     const dim3 grid(jobs.block_end[jobs.count - 1], (m + MT - 1) / MT, splits);
-    const int ct = small_col_tiles((int64_t)grid.x * grid.y * grid.z, MT, k, EPI == 1);
+    const int ct = small_col_tiles(grid.x, (int64_t)grid.y * grid.z, MT, k, EPI == 1);
     if (ct == 0) {
         hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 4, EPI, 1>), grid, dim3(256), 0, stream, x,
                            x_kind, jobs, m, k, in_scale, out_scale, out_kind, ksplit);
@@ -1760,7 +1770,7 @@ static bool tall_tiles(int m, int n, int k) {
 
 // The kernel of a call: run_linear launches it and g4_kernel_for_input names it.
 static KernelChoice route_linear(int bits, int m, int n, int k, float in_scale, int x_kind, bool gemm_mode) {
-    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, gemm_mode);
+    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, x_kind, gemm_mode);
     if (c == K_TILE128 && x_kind != G4_KIND_I8 && strip_cols(bits, m, n, k)) return K_STRIP;
     if (c == K_WIDE && tall_tiles(m, n, k)) return K_TALL;
     return c;
@@ -1870,7 +1880,7 @@ static bool small_presnap(int m, int n, int k) {
     // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager). At K = 128 four column tiles share each snap: 8-bit f16 2048 x
     // 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
     if (m > 32) return 32 * k > 64 * 1024;
-    const int ct = std::max(1, small_col_tiles(blocks, small_rows(blocks, m), k, false));
+    const int ct = std::max(1, small_col_tiles(blocks, 1, small_rows(blocks, m), k, false));
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) &&
            ((blocks + ct - 1) / ct + cus - 1) / cus * m * k >= 48 * 1024;
 }
@@ -1880,7 +1890,7 @@ static bool small_presnap(int m, int n, int k) {
 // their operands.
 static bool needs_codes_buffer(int bits, int m, int n, int k, float in_scale, int x_kind,
                                bool gemm_mode) {
-    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, gemm_mode);
+    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, x_kind, gemm_mode);
     if (x_kind == G4_KIND_I8) return false;
     if (c == K_TILE128 || c == K_WIDE) return true;
     return (c == K_SKINNY16 || c == K_SKINNY32) && small_presnap(m, n, k);
@@ -2034,7 +2044,7 @@ int linear_grouped(int bits, const void *x, int x_kind, int k, int m, float in_s
         int rc = check_linear(bits, o.wq, o.scales, x, x_kind, o.dst, out_kind, k, o.n, m, in_scale,
                               out_scale, who);
         if (rc) return rc;
-        const KernelChoice c = pick_kernel(bits, m, o.n, k, in_scale, false);
+        const KernelChoice c = pick_kernel(bits, m, o.n, k, in_scale, x_kind, false);
         small &= c == K_SKINNY16 || c == K_SKINNY32;
     }
     if (!small) {  // one call each, through the library's routing
@@ -2069,7 +2079,7 @@ int linear_gelu(int bits, const void *x, int k, int m, float in_scale, float out
     int rc = check_linear(bits, w_gate, s_gate, x, G4_KIND_I8, act, G4_KIND_I8, k, n, m, in_scale,
                           out_scale, who);
     if (rc) return rc;
-    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, false);
+    const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, G4_KIND_I8, false);
     if ((c != K_SKINNY16 && c != K_SKINNY32) || k > 16384 || act_scale == 0.0f) return G4_OK;
     if (w_up ? (bits != 4 || !s_up || (reinterpret_cast<uintptr_t>(w_up) & 15)) : (!up_vec || up_stride < n))
         return set_error(G4_ERR_INVALID, "gelu linear: the up operand (4-bit paired rows with scales, "
