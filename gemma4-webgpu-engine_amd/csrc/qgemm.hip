@@ -1867,9 +1867,9 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 }
 
 // The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past 48 Ki snaps
-// on the busiest CU (M * K per block, times its blocks there), one snap pass over the M * K
+// on the busiest CU (its rows * K per block, times its blocks there), one snap pass over the M * K
 // activations into a buffer of codes, then the kernel on int8 codes, costs less. Fused against
-// passed, us in a graph: 24 x 1536 -> 2048 (36 Ki) 5.6 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
+// passed, us in a graph: 32 x 1536 -> 2048 (16-row blocks, 24 Ki) 5.2 / 6.3, 24 x 2048 -> 2048 (32 Ki) 5.7 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
 // 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
 static bool small_presnap(int m, int n, int k) {
@@ -1880,9 +1880,10 @@ static bool small_presnap(int m, int n, int k) {
     // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager). At K = 128 four column tiles share each snap: 8-bit f16 2048 x
     // 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
     if (m > 32) return 32 * k > 64 * 1024;
-    const int ct = std::max(1, small_col_tiles(blocks, 1, small_rows(blocks, m), k, false));
-    return (int64_t)m * k * blocks >= ((int64_t)1 << 22) &&
-           ((blocks + ct - 1) / ct + cus - 1) / cus * m * k >= 48 * 1024;
+    const int mt = small_rows(blocks, m), rows = (m + mt - 1) / mt;
+    const int ct = std::max(1, small_col_tiles(blocks, rows, mt, k, false));
+    const int64_t per_cu = ((blocks + ct - 1) / ct * rows + cus - 1) / cus;
+    return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && per_cu * std::min(m, mt) * k >= 48 * 1024;
 }
 
 // Whether a call snaps f16 / f32 activations into a buffer of M * K codes first (the tile kernels,

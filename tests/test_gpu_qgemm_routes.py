@@ -95,3 +95,24 @@ def test_strips(gpu, oracle, bits, m, n, k):
 ])
 def test_sixteen_row_blocks(gpu, oracle, bits, m, n, k):
     check_every_kind(gpu, oracle, bits, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(32, 2048, 1536), (17, 1536, 2048), (28, 2048, 2048)])
+def test_sixteen_row_blocks_snap_in_place(gpu, m, n, k):
+    # fewer than 48 Ki snaps on a CU: one launch with no codes buffer, so a stream's first call can be captured
+    print(f"fused snap m={m} n={n} k={k}", flush=True)
+    g = np.random.default_rng(m)
+    x = gpu.DeviceBuffer.from_array(g.standard_normal((m, k)).astype(np.float16))
+    w = gpu.DeviceBuffer.from_array(g.integers(0, 256, (n, k // 2), dtype=np.uint8))
+    s = gpu.DeviceBuffer.from_array(g.uniform(0.005, 0.02, n).astype(np.float32))
+    out, want = (gpu.DeviceBuffer.empty((m, n), np.int32) for _ in range(2))
+    st = gpu.Stream()
+    graph = gpu.Graph(st, lambda: gpu.qgemm(4, w, s, x, out, k, n, m, 0.05, 0.1, stream=st.handle))
+    gpu.qgemm(4, w, s, x, want, k, n, m, 0.05, 0.1)
+    for _ in range(3):
+        out.fill(0x7B, st.handle)
+        graph.launch()
+        st.synchronize()
+        assert np.array_equal(out.download(), want.download())
+    graph.close()
+    st.close()
