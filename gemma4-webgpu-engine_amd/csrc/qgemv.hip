@@ -393,6 +393,7 @@ __global__ __launch_bounds__(kGemvThreads, f32_blocks_per_cu<COLS>()) void qgemv
     const int nch = k / CPC;
     const int slabs = (nch + SLAB - 1) / SLAB;
     const int64_t row_bytes = BITS == 4 ? (k >> 1) : k;
+    const int col0 = COLS == 1 ? blockIdx.y : 0;
     const int per = J.passes;  // row groups per wave (block uniform)
     const int groups = (J.rows + 3) >> 2;
     const int g_beg = ((blockIdx.x - J.wg_begin) * 4 + wave) * per;
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(kGemvThreads, f32_blocks_per_cu<COLS>()) void qgemv
                     const int kk = ch0 * CPC + e;
                     float v = 0.0f;  // past K: zero times a clamped chunk's finite codes
                     if (kk < k) {
-                        const int64_t at = (int64_t)c * k + kk;
+                        const int64_t at = (int64_t)(col0 + c) * k + kk;
                         v = J.act.up ? gelu_act_value(J.act, J.x, J.x_kind, at) : load_act(J.x, J.x_kind, at);
                     }
                     xs[c][(e / CPC) * XSTR + e % CPC] = v;
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(kGemvThreads, f32_blocks_per_cu<COLS>()) void qgemv
             const float scale = J.scales[row];
 #pragma unroll
             for (int c = 0; c < COLS; ++c)
-                store_linear_out(J.dst, (int64_t)c * J.rows + row, J.out_kind,
+                store_linear_out(J.dst, (int64_t)(col0 + c) * J.rows + row, J.out_kind,
                                  linear_epilogue(1.0f, scale, tot[c]), 0, J.out_scale);
         }
     }
@@ -682,15 +683,15 @@ static int total_blocks(const GemvLaunch &L) {
 }
 
 // Lays the uncalibrated jobs out (one K and width per launch: a single linear, or a batch over one x)
-// and launches the f32 kernel of their slab shape.
-template <int BITS, int COLS> static void launch_f32_t(GemvLaunch &L, hipStream_t stream) {
+// and launches the f32 kernel of their slab shape, `grid_cols` x COLS columns.
+template <int BITS, int COLS> static void launch_f32_t(GemvLaunch &L, int grid_cols, hipStream_t stream) {
     constexpr int MAX = f32_max_cpl<BITS>();
     const int nch = L.job[0].k / (BITS == 4 ? 32 : 16);
     const int slabs = (nch + 16 * MAX - 1) / (16 * MAX);
     const int cpl = (nch + 16 * slabs - 1) / (16 * slabs);
     int64_t groups = 0;
     for (int i = 0; i < L.count; ++i) groups += (L.job[i].rows + 3) / 4;
-    const int64_t waves = 4LL * f32_blocks_per_cu<COLS>() * device_cu_count();
+    const int64_t waves = 4LL * f32_blocks_per_cu<COLS>() * device_cu_count() / grid_cols;
     const int per = (int)std::max<int64_t>(1, (groups + waves - 1) / waves);
     int wg = 0;
     for (int i = 0; i < L.count; ++i) {
@@ -698,16 +699,23 @@ template <int BITS, int COLS> static void launch_f32_t(GemvLaunch &L, hipStream_
         L.job[i].wg_begin = wg;
         wg += ((L.job[i].rows + 3) / 4 + 4 * per - 1) / (4 * per);
     }
-    const dim3 grid(wg), block(kGemvThreads);
+    const dim3 grid(wg, grid_cols), block(kGemvThreads);
     if (cpl == 1) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 1, COLS>), grid, block, 0, stream, L);
     else if (cpl == 2) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 2, COLS>), grid, block, 0, stream, L);
     else if (cpl == 3) hipLaunchKernelGGL((qgemv_f32_kernel<BITS, 3, COLS>), grid, block, 0, stream, L);
     else hipLaunchKernelGGL((qgemv_f32_kernel<BITS, MAX, COLS>), grid, block, 0, stream, L);
 }
 
+// Two columns share one weight stream, or, while a wave then has at most two row groups, run as blocks of one
+// column each: the weights then come from L2 the second time, and the x of one column per lane is half the staging
+// and half the chain. Us, together / apart: 8-bit 1536 x 2048 7.6 / 6.0, 16384 x 1536 51.4 / 34.2, 1536 x 12288
+// 10.6 / 10.4, 1536 x 32768 15.2 / 19.6; 4-bit 1536 x 1536 6.5 / 4.9, 1536 x 12288 9.4 / 8.3, 1536 x 32768 12.5 / 15.6.
 static void launch_f32(GemvLaunch &L, int cols, hipStream_t stream) {
-    if (L.job[0].bits == 4) cols == 1 ? launch_f32_t<4, 1>(L, stream) : launch_f32_t<4, 2>(L, stream);
-    else cols == 1 ? launch_f32_t<8, 1>(L, stream) : launch_f32_t<8, 2>(L, stream);
+    int64_t groups = 0;
+    for (int i = 0; i < L.count; ++i) groups += (L.job[i].rows + 3) / 4;
+    const bool together = cols == 2 && groups > 4LL * f32_blocks_per_cu<1>() * device_cu_count();
+    if (L.job[0].bits == 4) together ? launch_f32_t<4, 2>(L, 1, stream) : launch_f32_t<4, 1>(L, cols, stream);
+    else together ? launch_f32_t<8, 2>(L, 1, stream) : launch_f32_t<8, 1>(L, cols, stream);
 }
 
 // Launches the integer or f32 GEMV over L.count jobs with `cols` token columns (1 or 2).

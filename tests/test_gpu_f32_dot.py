@@ -23,6 +23,7 @@ def out_buf(g4, shape):
 @pytest.mark.parametrize("bits,k,n", [
     (4, 256, 1), (4, 512, 3), (4, 768, 67), (4, 1536, 5), (4, 1792, 64), (4, 16384, 21),
     (8, 128, 2), (8, 1024, 66), (8, 1152, 9), (8, 1536, 130), (8, 16384, 7),
+    (4, 256, 12288), (8, 128, 12289),  # the last that runs its columns apart, the first together (256 CUs)
     (4, 1536, 13000),   # two groups per wave
     (4, 256, 200003),   # more than one 16-group run per wave
 ])
