@@ -1582,18 +1582,24 @@ int workspace_forget_stream(void *stream) {
 // -> four: 32 x 1536 -> 8960 11.7 -> 7.2, 16384 12.8 -> 7.7). Past that, 32-row blocks still take
 // four (32 x 1024 -> 24576 14.9 -> 11.9) and 16-row ones, whose codes are half, the 4-wave blocks
 // (8 x 1024 -> 24576 8.1 / 9.5), which also win up to three tiles per CU while their codes take one
-// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). At K = 128 a block has one K step, so a second
-// round of four-tile blocks that is at most half full costs more than it saves (8-bit, 4-wave / four tiles:
-// 683 x 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5), and so
-// does a grid that two tiles would have fitted but for the odd one (f16 697 x 128 -> 366 5.8 / 7.4). The paired gate / up form stops
+// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). 8-bit blocks of one to three K steps have
+// little to gain from a second round of four-tile blocks that is at most half full (4-wave / four tiles: 683 x
+// 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5; 20 x 256 ->
+// 16729, 1046 tiles, 10.5 / 12.2; 29 x 384 -> 18920 11.5 / 12.8), with one step also from the start of a third (513 x
+// 128 -> 2048 15.4 / 17.1) and from a grid that two tiles would have fitted but for the odd one (f16 697 x 128 ->
+// 366 5.8 / 7.4). The paired gate / up form stops
 // at two (its four would spill).
-static int small_col_tiles(int64_t n16, int64_t rows, int mt, int k, bool paired) {
+static int small_col_tiles(int bits, int64_t n16, int64_t rows, int mt, int k, bool paired) {
     const int64_t cus = device_cu_count(), blocks16 = n16 * rows;
     if (blocks16 <= cus) return 1;
     if ((n16 + 1) / 2 * rows <= cus) return 2;
     if (paired) return 0;
-    if (k == kTileBK && mt > 16 && (blocks16 <= 2 * cus || (blocks16 > 4 * cus && blocks16 <= 6 * cus))) return 0;
-    if (mt > 16) return 4;
+    if (mt > 16) {
+        const int64_t blocks = (n16 + 3) / 4 * rows, full = blocks / cus, left = blocks % cus;
+        const bool short_k = bits == 8 && k <= 3 * kTileBK, one_step = k == kTileBK;
+        if (one_step && (blocks16 <= 2 * cus || (full == 2 && left > 0 && 5 * left <= 2 * cus))) return 0;
+        return short_k && full == 1 && left > 0 && 2 * left <= cus ? 0 : 4;
+    }
     return (n16 + 3) / 4 * rows <= cus && (blocks16 > 3 * cus || k > 3072) ? 4 : 0;
 }
 
@@ -1632,7 +1638,10 @@ static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, i
     // 128 x 2048 -> 1536 7.2 -> 5.5; four tiles per block lose: 64 x 1536 -> 6144 6.7 / 7.2). A grid past the
     // CUs by a few blocks takes a second round: 8-bit 696 x 3840 -> 360 (264 blocks) 16.3, tile 8.1; 4-bit f16
     // 1380 x 3328 -> 165 21.8, strip 12.3.
-    const int ct = m <= 64 || k >= 16 * kTileBK ? 2 : 1;
+    // 8-bit codes past one LDS chunk (K = 3072) lose with two tiles: 52 x 4224 -> 3696 8.8 / 10.7, 124 x 4736 ->
+    // 1984 9.4 / 13.1.
+    const bool two_chunks = bits == 8 && x_kind == G4_KIND_I8 && k > 24 * kTileBK && n > 2 * kTileBN;
+    const int ct = (m <= 64 || k >= 16 * kTileBK) && !two_chunks ? 2 : 1;
     const int64_t cus = device_cu_count(), rows = (m + 31) / 32, n16 = (n + 15) / 16;
     if (k >= 4 * kTileBK && (n16 + ct - 1) / ct * rows <= cus) return K_SKINNY32;
     // int8 codes on up to three column tiles of the tile kernel, which go to as many of the 8 XCDs: the small-M
@@ -1670,7 +1679,7 @@ static void launch_small_t(const void *x, int x_kind, const SmallJobs &jobs, int
                            int splits = 1) {
     const int ksplit = splits > 1 ? k / splits : 0;
     const dim3 grid(jobs.block_end[jobs.count - 1], (m + MT - 1) / MT, splits);
-    const int ct = small_col_tiles(grid.x, (int64_t)grid.y * grid.z, MT, k, EPI == 1);
+    const int ct = small_col_tiles(BITS, grid.x, (int64_t)grid.y * grid.z, MT, k, EPI == 1);
     if (ct == 0) {
         hipLaunchKernelGGL((qgemm_small_kernel<BITS, MT, 4, EPI, 1>), grid, dim3(256), 0, stream, x,
                            x_kind, jobs, m, k, in_scale, out_scale, out_kind, ksplit);
@@ -1872,7 +1881,7 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 // passed, us in a graph: 32 x 1536 -> 2048 (16-row blocks, 24 Ki) 5.2 / 6.3, 24 x 2048 -> 2048 (32 Ki) 5.7 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
 // 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
-static bool small_presnap(int m, int n, int k) {
+static bool small_presnap(int bits, int m, int n, int k) {
     const int64_t cus = device_cu_count();
     const int64_t blocks = (n + 15) / 16;
     // M > 32: few blocks per CU, or K = 128 (pick_kernel). Up to K = 2048 the call stays one launch, which an
@@ -1881,7 +1890,7 @@ static bool small_presnap(int m, int n, int k) {
     // 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
     if (m > 32) return 32 * k > 64 * 1024;
     const int mt = small_rows(blocks, m), rows = (m + mt - 1) / mt;
-    const int ct = std::max(1, small_col_tiles(blocks, rows, mt, k, false));
+    const int ct = std::max(1, small_col_tiles(bits, blocks, rows, mt, k, false));
     const int64_t per_cu = ((blocks + ct - 1) / ct * rows + cus - 1) / cus;
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && per_cu * std::min(m, mt) * k >= 48 * 1024;
 }
@@ -1894,7 +1903,7 @@ static bool needs_codes_buffer(int bits, int m, int n, int k, float in_scale, in
     const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, x_kind, gemm_mode);
     if (x_kind == G4_KIND_I8) return false;
     if (c == K_TILE128 || c == K_WIDE) return true;
-    return (c == K_SKINNY16 || c == K_SKINNY32) && small_presnap(m, n, k);
+    return (c == K_SKINNY16 || c == K_SKINNY32) && small_presnap(bits, m, n, k);
 }
 
 // The snap pass: M * K f16 / f32 activations (16-byte aligned, K % 128 == 0) into int8 codes in
@@ -1968,7 +1977,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     if (c == K_SKINNY16 || c == K_SKINNY32) {
         // One launch, the activation snap fused into the small-M kernel; or, past small_presnap,
         // the snap pass first (natural order: the kernel's int8 path interleaves for 4-bit).
-        if (x_kind != G4_KIND_I8 && small_presnap(m, n, k)) {
+        if (x_kind != G4_KIND_I8 && small_presnap(bits, m, n, k)) {
             const int8_t *codes = nullptr;
             int rc = snap_pass(x, x_kind, m, k, in_scale, kCodesNatural, stream, given_codes, &codes);
             if (rc) return rc;

@@ -190,9 +190,12 @@ def test_kernel_choice_of_ragged_small_grids(g4):
     """Rows by column tiles that pass the CUs by a few blocks leave the small-M kernel (a second round for the
     whole call), but for int8 codes on a few columns."""
     for kind in (g4.KIND_I8, g4.KIND_F16):
-        assert g4.kernel_for_shape(8, 704, 352, 3840, kind) == "qmatmul-8bit-mfma-small32"  # 11 x 22 blocks
-        assert "small" not in g4.kernel_for_shape(8, 704, 353, 3840, kind)                  # 12 x 22
+        assert g4.kernel_for_shape(8, 704, 352, 2816, kind) == "qmatmul-8bit-mfma-small32"  # 11 x 22 blocks
+        assert "small" not in g4.kernel_for_shape(8, 704, 353, 2816, kind)                  # 12 x 22
     assert "small" not in g4.kernel_for_shape(4, 1380, 165, 3328, g4.KIND_F16)
+    # two column tiles of 8-bit codes: up to one LDS chunk of K
+    assert g4.kernel_for_shape(8, 124, 1984, 3072, g4.KIND_I8) == "qmatmul-8bit-mfma-small32"
+    assert g4.kernel_for_shape(8, 124, 1984, 3200, g4.KIND_I8) == "qmatmul-8bit-mfma-tile"
     assert g4.kernel_for_shape(4, 1380, 165, 3328, g4.KIND_I8) == "qgemm-4bit-mfma-small32"
     assert g4.kernel_for_shape(8, 1700, 140, 2560, g4.KIND_I8) == "qmatmul-8bit-mfma-small32"
     assert g4.kernel_for_shape(8, 1700, 140, 3840, g4.KIND_I8) == "qmatmul-8bit-mfma-tile"

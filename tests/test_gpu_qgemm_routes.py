@@ -42,6 +42,7 @@ def check_every_kind(gpu, oracle, bits, m, n, k):
     (4, 17, 4099, 1536), (4, 32, 8200, 1536), (4, 31, 16500, 256), (8, 32, 4100, 384), (8, 12, 8300, 3200),
     # 23 column tiles by 22 block rows: two tiles per block would be 264 blocks
     (8, 697, 366, 128), (4, 700, 360, 2048), (8, 697, 361, 2176), (4, 1640, 140, 2048), (8, 1700, 140, 2048),
+    (8, 20, 16729, 256), (8, 29, 18921, 384), (8, 513, 2048, 128), (8, 52, 3697, 3200), (8, 52, 3697, 3072),
     (8, 20, 17000, 128), (8, 512, 1537, 128), (8, 513, 1600, 128), (8, 31, 16385, 128), (4, 64, 3071, 768), (4, 40, 4096, 2304), (4, 100, 1500, 2048),
 ])
 def test_column_tiles(gpu, oracle, bits, m, n, k):
