@@ -1821,7 +1821,16 @@ static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, cons
     hipLaunchKernelGGL((qgemm_tile_kernel<BITS, NS_, NAT_, BM_, KS_>), dim3(blocks), dim3(256 * KS_), 0, \
                        stream, codes, w, scales, dst, m, n, k, in_scale, out_scale, out_kind,     \
                        tiles_m, tiles_n)
-#define G4_TILE(NS_, NAT_, BM_) G4_TILE_K(NS_, NAT_, BM_, 1)
+    // natural order only exists for 4-bit weights
+#define G4_TILE(NS_, BM_)                                      \
+    do {                                                       \
+        if constexpr (BITS == 4) {                             \
+            if (nat) G4_TILE_K(NS_, true, BM_, 1);             \
+            else G4_TILE_K(NS_, false, BM_, 1);                \
+        } else {                                               \
+            G4_TILE_K(NS_, false, BM_, 1);                     \
+        }                                                      \
+    } while (0)
     // a grid of at most one block per CU splits its K stages over two groups of four waves, twice the
     // loads in flight per CU (us in a graph: 128 x 6144 -> 1536 15.3 -> 13.6, 128 x 1536 -> 6144 7.1
     // -> 6.8, 256 x 2048 -> 1536 7.9 -> 7.4, 8-bit 512 x 1536 -> 256 6.2 -> 5.7; four groups 14.0, 7.1).
@@ -1830,20 +1839,12 @@ static int launch_tile(const int8_t *codes, bool natural, const uint8_t *w, cons
     // it. 4-bit 1098 x 3072 -> 402 (35 blocks) 15.1, 14.3.
     const bool one_per_cu = BITS == 4 ? (int64_t)tiles_m * tiles_n <= device_cu_count()
                                       : (int64_t)tiles_m * ((tiles_n + 7) / 8) <= device_cu_count() / 8;
-    if (half && one_per_cu && nk % 2 == 0 && nk >= 6) {
-        if (nat) G4_TILE_K(4, true, 32, 2);
-        else G4_TILE_K(4, false, 32, 2);
-    } else if (half) {
-        if (nk >= 3 && nat) G4_TILE(4, true, 32);
-        else if (nk >= 3) G4_TILE(4, false, 32);
-        else if (nat) G4_TILE(3, true, 32);
-        else G4_TILE(3, false, 32);
-    } else {
-        if (nk >= 3 && nat) G4_TILE(4, true, 64);
-        else if (nk >= 3) G4_TILE(4, false, 64);
-        else if (nat) G4_TILE(3, true, 64);
-        else G4_TILE(3, false, 64);
-    }
+    // 4-bit f16 / f32 calls of so few tiles are strips (strip_cols), so interleaved 4-bit codes need no split.
+    if (half && one_per_cu && nk % 2 == 0 && nk >= 6 && (BITS == 8 || nat)) G4_TILE_K(4, BITS == 4, 32, 2);
+    else if (half && nk >= 3) G4_TILE(4, 32);
+    else if (half) G4_TILE(3, 32);
+    else if (nk >= 3) G4_TILE(4, 64);
+    else G4_TILE(3, 64);
 #undef G4_TILE
 #undef G4_TILE_K
     G4_LAUNCHED("qgemm_tile_kernel");

@@ -50,7 +50,7 @@ def gate(gpu):
     return n, k, w, s, dev(gpu, w), dev(gpu, s)
 
 
-@pytest.mark.parametrize("m", [3, 4, 8, 16, 17, 32, 33, 128, 512])
+@pytest.mark.parametrize("m", [3, 4, 8, 16, 17, 32, 33, 128, 200, 512])
 def test_config2_gate_full_compare(gpu, oracle, gate, m):
     n, k, w, s, wb, sb = gate
     x = syn.activations("c2", f"x{m}", m, k, outlier_frac=0.01)
@@ -73,11 +73,13 @@ def test_config2_gate_full_compare(gpu, oracle, gate, m):
 @pytest.mark.parametrize("x_kind", ["f16", "i8"])
 def test_config2_gate_m2048_full(gpu, oracle, gate, x_kind):
     """Every output of the M = 2048 gate call against the oracle: f16 activations (the snap pass,
-    then the wide kernel on interleaved codes) and int8 codes (the wide kernel's NAT instantiation
+    then the tall kernel on interleaved codes) and int8 codes (the tall kernel's NAT instantiation
     reading the caller's codes in place); int8 codes and int32 accumulators. As a size-independent
     property, a few columns also equal the GEMV kernel's answer for that column alone."""
     n, k, w, s, wb, sb = gate
     m = 2048
+    kind = gpu.KIND_F16 if x_kind == "f16" else gpu.KIND_I8
+    assert gpu.kernel_for_shape(4, m, n, k, kind) == "qgemm-4bit-mfma-tall"
     x = syn.activations("c2", "x2048", m, k, outlier_frac=0.01)
     print(f"config2 m=2048 x={x_kind} kernel={gpu.kernel_for_shape(4, m, n, k)}", flush=True)
     _, acc, codes = oracle.qgemm(4, w, s, x.astype(np.float32), n, k, m, syn.IN_SCALE,
@@ -111,7 +113,7 @@ def test_qmatmul8_shapes(gpu, oracle, m, n, k):
     assert f32_equal(of.download(), want)
 
 
-@pytest.mark.parametrize("m,n", [(37, 1000), (129, 2047), (64, 128)])
+@pytest.mark.parametrize("m,n", [(37, 1000), (129, 2047), (64, 128), (201, 6200)])  # the last on the tile kernel
 def test_int4_partial_tiles(gpu, oracle, m, n):
     k = 2048
     w = syn.int4_weights("tiles", f"{m}x{n}", n, k)
@@ -136,12 +138,13 @@ def test_uncalibrated_gemm_grid_exact(gpu, oracle):
 
 
 @pytest.mark.parametrize("out_kind", ["f32", "i8", "i32"])
-def test_tile_epilogue_kinds_m96(gpu, oracle, gate, out_kind):
-    # The tile kernel's epilogue for every output kind, over a ragged last M tile (96 = 64 + 32)
-    # and every column of the gate shape.
+@pytest.mark.parametrize("m,kernel", [(96, "strip"), (200, "tile")])
+def test_tile_epilogue_kinds_m96(gpu, oracle, gate, out_kind, m, kernel):
+    # The strip's and the tile kernel's epilogue for every output kind, over a ragged last M tile
+    # (96 = 64 + 32, 200 = 3 x 64 + 8) and every column of the gate shape.
     n, k, w, s, wb, sb = gate
-    m = 96
-    x = syn.activations("c2", "epi96", m, k, outlier_frac=0.01)
+    assert kernel in gpu.kernel_for_shape(4, m, n, k, gpu.KIND_F16)
+    x = syn.activations("c2", f"epi{m}", m, k, outlier_frac=0.01)
     want, acc, codes = oracle.qgemm(4, w, s, x.astype(np.float32), n, k, m, syn.IN_SCALE,
                                     syn.OUT_SCALE)
     dt = {"f32": np.float32, "i8": np.int8, "i32": np.int32}[out_kind]

@@ -1,6 +1,7 @@
-"""The rules that send M > 32 to the small-M kernel (one block of 32 rows x 16 columns per CU) and
-split the tile kernel's K stages over two wave groups, at their edges: ragged rows and columns, K of
-odd and even stage counts, both weight widths, every input and output kind, against the oracle."""
+"""The kernels of M > 2 and the rules between them, at their edges: the small-M kernel's block rows and
+column tiles, the strips, the tile kernel's 32- and 64-row forms, rings and K split, and the tall tiles.
+Ragged rows and columns, K of odd and even stage counts, both weight widths, every input and output kind,
+against the oracle; each test asserts the kernel it is about."""
 import numpy as np
 import pytest
 
@@ -53,6 +54,8 @@ def test_column_tiles(gpu, oracle, bits, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(2048, 6144, 512), (2047, 6137, 768), (1793, 5953, 512), (4096, 6144, 512)])
 @pytest.mark.parametrize("xdt", [np.float16, np.int8])
 def test_tall_tiles(gpu, m, n, k, xdt):
+    kind = gpu.KIND_F16 if xdt == np.float16 else gpu.KIND_I8
+    assert gpu.kernel_for_shape(4, m, n, k, kind) == "qgemm-4bit-mfma-tall"
     # whole rounds of 256 x 192 tiles: full tiles, ragged last rows and columns (odd N: the stores fall
     # back to single outputs), two rounds; 4 and 6 K stages
     print(f"tall m={m} n={n} k={k} x={np.dtype(xdt)}", flush=True)
@@ -80,12 +83,27 @@ def test_tall_tiles(gpu, m, n, k, xdt):
     # strips of 64 rows x 32, 48 and 64 columns, either side of one per CU; ragged row tiles (M % 16 of 1,
     # 15 and 0), ragged columns, fewer stages than waves, and 1 .. 6 stages per wave with a remainder
     (4, 33, 8192, 512), (4, 64, 8193, 256), (4, 65, 6145, 768), (4, 129, 4097, 1280), (4, 513, 1363, 2304),
-    (4, 512, 2049, 1280), (4, 1023, 31, 1536), (4, 1040, 257, 1024), (4, 177, 1535, 5120), (4, 191, 2700, 6144),
-    (8, 1025, 130, 1024), (8, 65, 6145, 1152), (8, 2000, 257, 1024), (8, 143, 1501, 2176),
+    (4, 1023, 31, 256), (4, 1040, 257, 1024), (4, 177, 1535, 5120), (4, 191, 2700, 6144),
+    (8, 1025, 130, 1024), (8, 65, 6145, 1152), (8, 2000, 257, 1024), (8, 143, 1801, 2176),
     # row groups on every second and fourth XCD, and strips in turn
     (4, 281, 2048, 256), (4, 513, 1024, 512), (4, 1132, 884, 512), (8, 1100, 850, 1024),
 ])
 def test_strips(gpu, oracle, bits, m, n, k):
+    for kind in (gpu.KIND_F32, gpu.KIND_F16):
+        assert gpu.kernel_for_shape(bits, m, n, k, kind).endswith("mfma-strip")
+    check_every_kind(gpu, oracle, bits, m, n, k)
+
+
+@pytest.mark.parametrize("bits,m,n,k", [
+    # 64-row tiles on rings of 4 and 3 stages (K of 4 and more stages, and 2), 4-bit codes interleaved by the
+    # snap (f16 / f32) and in natural order (int8), 8-bit; ragged last rows and columns
+    (4, 200, 6145, 512), (4, 200, 6145, 256), (4, 512, 4001, 768), (8, 512, 6143, 640), (8, 2048, 1537, 256),
+    # 32-row tiles that are no strips: one more column than 256 strips of 64
+    (4, 512, 2049, 256), (4, 512, 2049, 1280), (8, 513, 1024, 256), (8, 500, 2100, 1152),
+])
+def test_tiles(gpu, oracle, bits, m, n, k):
+    for kind in (gpu.KIND_F32, gpu.KIND_F16, gpu.KIND_I8):
+        assert gpu.kernel_for_shape(bits, m, n, k, kind).endswith("mfma-tile")
     check_every_kind(gpu, oracle, bits, m, n, k)
 
 
@@ -95,6 +113,7 @@ def test_strips(gpu, oracle, bits, m, n, k):
     (4, 250, 255, 1536), (4, 257, 240, 2304), (8, 18, 1536, 128), (8, 32, 257, 1536), (8, 100, 500, 6400),
 ])
 def test_sixteen_row_blocks(gpu, oracle, bits, m, n, k):
+    assert "small" in gpu.kernel_for_shape(bits, m, n, k, gpu.KIND_F16)
     check_every_kind(gpu, oracle, bits, m, n, k)
 
 

@@ -123,12 +123,14 @@ def test_small_m_snap(gpu, oracle, bits, m, n, mode):
 
 @pytest.mark.parametrize("mode", ["adv", "ka"])
 @pytest.mark.parametrize("bits", [4, 8])
-def test_tile_snap(gpu, oracle, bits, mode):
-    """M > 32: quantize_rows (f32 in) and the tile kernel's epilogue snap; int8 codes in take the
-    natural-order tile kernel with the same epilogue."""
-    m, n, k = 96, 1536, 1536
+@pytest.mark.parametrize("m,n,f32_kernel", [(96, 1536, "strip"), (200, 6144, "tile")])
+def test_tile_snap(gpu, oracle, bits, mode, m, n, f32_kernel):
+    """M > 32: f32 in, the snap passes of the strip and the tile kernel and their epilogue snaps; int8
+    codes in take the natural-order tile kernel."""
+    k = 1536
     w, s, x, sin, sout, want = case(oracle, bits, m, n, k, mode, 41 + bits)
     assert "tile" in gpu.kernel_for_shape(bits, m, n, k)
+    assert f32_kernel in gpu.kernel_for_shape(bits, m, n, k, gpu.KIND_F32)
     dw, ds = dev(gpu, w), dev(gpu, s)
     codes = oracle.srq_codes(x.reshape(-1), sin).reshape(m, k)
     for src_name, src in (("f32", dev(gpu, x)), ("i8", dev(gpu, codes))):
