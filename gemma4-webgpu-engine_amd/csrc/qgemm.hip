@@ -1882,14 +1882,18 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
 // passed, us in a graph: 32 x 1536 -> 2048 (16-row blocks, 24 Ki) 5.2 / 6.3, 24 x 2048 -> 2048 (32 Ki) 5.7 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
 // 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
-static bool small_presnap(int bits, int m, int n, int k) {
+static bool small_presnap(int bits, int m, int n, int k, int x_kind) {
     const int64_t cus = device_cu_count();
     const int64_t blocks = (n + 15) / 16;
     // M > 32: few blocks per CU, or K = 128 (pick_kernel). Up to K = 2048 the call stays one launch, which an
     // eager caller's host time is bound by (64 x 2048 -> 1536 eager 7.5 us fused, 9.1 passed; 7.8 / 7.2 in a
-    // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager). At K = 128 four column tiles share each snap: 8-bit f16 2048 x
-    // 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
-    if (m > 32) return 32 * k > 64 * 1024;
+    // graph; 64 x 6144 -> 1536 18.0 / 11.2 eager), unless 32-row blocks read 6 MiB of f32 or more (fused / passed:
+    // 1024 x 2048 -> 256 14.1 / 10.8 us in a graph, 13.6 / 10.4 eager, 1024 x 1536 -> 128 11.4 / 9.3; f16 9.4 / 11.1 at
+    // 2048 x 2048 -> 128, 2048 x 1024 -> 64 6.3 / 8.2). At K = 128 four column tiles share each snap: 8-bit f16 2048
+    // x 128 -> 1536 35.4 us in a graph, 41.5 with a pass and 4-wave blocks.
+    if (m > 32)
+        return 32 * k > 64 * 1024 || (x_kind == G4_KIND_F32 && k >= 12 * kTileBK &&
+                                      (int64_t)m * k * 4 >= (6 << 20) && small_rows(blocks, m) == 32);
     const int mt = small_rows(blocks, m), rows = (m + mt - 1) / mt;
     const int ct = std::max(1, small_col_tiles(bits, blocks, rows, mt, k, false));
     const int64_t per_cu = ((blocks + ct - 1) / ct * rows + cus - 1) / cus;
@@ -1904,7 +1908,7 @@ static bool needs_codes_buffer(int bits, int m, int n, int k, float in_scale, in
     const KernelChoice c = pick_kernel(bits, m, n, k, in_scale, x_kind, gemm_mode);
     if (x_kind == G4_KIND_I8) return false;
     if (c == K_TILE128 || c == K_WIDE) return true;
-    return (c == K_SKINNY16 || c == K_SKINNY32) && small_presnap(bits, m, n, k);
+    return (c == K_SKINNY16 || c == K_SKINNY32) && small_presnap(bits, m, n, k, x_kind);
 }
 
 // The snap pass: M * K f16 / f32 activations (16-byte aligned, K % 128 == 0) into int8 codes in
@@ -1978,7 +1982,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     if (c == K_SKINNY16 || c == K_SKINNY32) {
         // One launch, the activation snap fused into the small-M kernel; or, past small_presnap,
         // the snap pass first (natural order: the kernel's int8 path interleaves for 4-bit).
-        if (x_kind != G4_KIND_I8 && small_presnap(bits, m, n, k)) {
+        if (x_kind != G4_KIND_I8 && small_presnap(bits, m, n, k, x_kind)) {
             const int8_t *codes = nullptr;
             int rc = snap_pass(x, x_kind, m, k, in_scale, kCodesNatural, stream, given_codes, &codes);
             if (rc) return rc;

@@ -108,9 +108,10 @@ def test_tiles(gpu, oracle, bits, m, n, k):
 
 
 @pytest.mark.parametrize("bits,m,n,k", [
-    # 16-row blocks past 16 rows, either side of one block per CU; ragged last rows and columns
+    # 16-row blocks past 16 rows, either side of one block per CU; ragged last rows and columns; f32 that is
+    # snapped in a pass of its own (1024 x 1536)
     (4, 17, 2048, 512), (4, 17, 2049, 256), (4, 31, 1536, 6400), (4, 33, 1361, 1536), (4, 49, 1024, 768),
-    (4, 250, 255, 1536), (4, 257, 240, 2304), (8, 18, 1536, 128), (8, 32, 257, 1536), (8, 100, 500, 6400),
+    (4, 250, 255, 1536), (4, 257, 240, 2304), (4, 1024, 121, 1536), (8, 18, 1536, 128), (8, 32, 257, 1536), (8, 100, 500, 6400),
 ])
 def test_sixteen_row_blocks(gpu, oracle, bits, m, n, k):
     assert "small" in gpu.kernel_for_shape(bits, m, n, k, gpu.KIND_F16)
