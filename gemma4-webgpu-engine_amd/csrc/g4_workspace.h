@@ -1,7 +1,7 @@
 // The per-stream activation workspace of the tile GEMM: the lifetime rules, host code only.
 //
-// A g4_qgemm call with f16 / f32 activations at M > 32 snaps them into a device buffer that the
-// tile kernel then reads. The buffer belongs to (device, stream), so calls ordered on one stream
+// A g4_qgemm call whose f16 / f32 activations are snapped in a pass of their own (needs_codes_buffer)
+// keeps the codes in a device buffer that its matrix kernel then reads. The buffer belongs to (device, stream), so calls ordered on one stream
 // share it. The rules:
 //  - A call that fits the current buffer uses it. If the stream is capturing a graph, the buffer
 //    is marked captured: the graph's nodes now hold its address.

@@ -2,12 +2,12 @@
 // qmatmul-8bit (src/kernels/pleMatmul.ts), plus the shape routing of src/execute.ts:372-430.
 //
 // Pipeline of one call (calibrated path):
-//  1. The activation snap (the SRQ input prologue): M <= 32 fuses it into the small kernel (codes
-//     in LDS, each 8-code group interleaved [x0 x2 x4 x6 x1 x3 x5 x7] for 4-bit weights so a weight
-//     word's even and odd nibble lanes line up with the codes). The tile kernel takes an int8
-//     caller's natural-order codes as given (and permutes the 4-bit B to match); f16 / f32 input is
-//     snapped once per row by quantize_rows_kernel into a per-stream workspace, interleaved (for the
-//     strip kernel by quantize_strip_kernel, in the order of its lanes).
+//  1. The activation snap (the SRQ input prologue): the small-M kernel fuses it while few of its blocks
+//     share a row (small_presnap; codes in LDS, each 8-code group interleaved [x0 x2 x4 x6 x1 x3 x5 x7]
+//     for 4-bit weights so a weight word's even and odd nibble lanes line up with the codes). The
+//     other kernels take an int8 caller's natural-order codes as given (and permute the 4-bit B to
+//     match); f16 / f32 input is snapped once per row by quantize_rows_kernel into a per-stream
+//     workspace, interleaved (for the strip kernel by quantize_strip_kernel, in the order of its lanes).
 //  2. An MFMA kernel contracts codes x weights with v_mfma_i32_16x16x64_i8 in exact int32. The
 //     int32 sums are exact, so the k order the MFMA uses internally is irrelevant; only the A and
 //     B operands have to agree on it, and they do by construction.
@@ -15,16 +15,18 @@
 //
 // Kernels by M (chosen per call, see route_linear):
 //   M <= 2         the GEMV family (qgemv.hip): bit-identical, cheaper than any tile at this M.
-//   3 <= M <= 32, and more rows while one block of 32 rows x 16 columns per CU covers the output
-//                  qgemm_small_kernel: one launch with the snap fused (codes in LDS), 16 weight
-//                  rows per block, the block's waves split K (4, or 16 when the grid is no wider
-//                  than the CU count), 16 or 32 rows (small_rows), an LDS fold of the partials; several projections of the
+//   3 <= M <= 32, more rows while 16-wave blocks of 32 rows x 16 (or 32) columns cover the output
+//   with one per CU, and any M at K = 128 (pick_kernel)
+//                  qgemm_small_kernel: blocks of 16 or 32 rows (small_rows) by 1, 2 or 4 tiles of 16
+//                  weight rows (small_col_tiles), the block's waves split K (16 waves, or 4 on wide
+//                  grids of single tiles), an LDS fold of the partials; several projections of the
 //                  same x can share one grid (linear_grouped).
 //   larger outputs, or over 32768+ rows
 //                  qgemm_tile_kernel: 64 x 96 output tiles, activation codes and weights streamed
 //                  global -> LDS by direct loads through a 3-4 stage ring, XCD-aware tile order;
 //                  4-bit outputs that fill the chip take 64 x 192 tiles (qgemm_wide_kernel), and
-//                  256 x 192 ones (qgemm_tall_kernel) when those come in nearly whole rounds of CUs.
+//                  256 x 192 ones (qgemm_tall_kernel) when those come in nearly whole rounds of CUs
+//                  (tall_tiles).
 //                  f16 / f32 calls whose output one strip of 64 rows x 32 - 64 columns per CU covers
 //                  take qgemm_strip_kernel: K split over the block's waves, no LDS in its K loop.
 #include "g4_internal.h"
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(256) void qmatmul8_serial_kernel(
 __device__ __forceinline__ uint32_t nib_even16(uint32_t w) { return ((w ^ 0x88888888u) << 4) & 0xF0F0F0F0u; }
 __device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x88888888u) & 0xF0F0F0F0u; }
 
-// ---- small M: M <= MT token rows, 16 weight rows per block, K split over the block's waves ------
+// ---- small M: MT token rows and CT tiles of 16 weight rows per block, K split over its waves ------
 // The activation snap is fused: the block snaps its MT token rows into LDS as int8 codes (the
 // 4-bit interleave per 8-code group) one K chunk at a time, so a draft-verify or small prefill
 // call is one launch. 4-bit weights are taken as 16 * code (nib_even16): no zero-point sums, so half
@@ -192,7 +194,7 @@ __device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x888888
 // both operands. The LDS rows are padded by 16 bytes so the 16 token rows of one A read fall on
 // distinct banks.
 //
-// WAVES: 16 while the grid fits the CUs, over CT column tiles of 16 weight rows (small_col_tiles):
+// WAVES: 16, over CT column tiles of 16 weight rows (small_col_tiles: one block per CU and round):
 // wave w takes tile w % CT and K part w / CT of 16 / CT, so a block walks its K fast and a CU copies
 // the codes once for all its columns; 4 (CT 1) for wider grids of 16-row blocks. The fold of the
 // partial tiles goes through LDS. The sums are int32 and exact, so the split changes no result.

@@ -2,8 +2,8 @@
 // capture, tight serving loops, harnesses that forbid hipMalloc). It has no counterpart in the
 // reference.
 //
-// The only memory g4_qgemm needs beyond its operands is the buffer of snapped activation codes on
-// the tile path (f16 / f32 activations at M > 32: M * K bytes). Here that buffer is `scratch`, a
+// The only memory g4_qgemm needs beyond its operands is the buffer of activation codes on the paths
+// that snap f16 / f32 activations in a pass of their own (needs_codes_buffer: M * K bytes). Here that buffer is `scratch`, a
 // file-scope device array of kScratchBytes that every GPU holds for the life of the process. The
 // host never uses the array's name as an address: at the first call on a device (that device
 // current) hipGetSymbolAddress gives that device's copy, kept per device and passed to the kernels.

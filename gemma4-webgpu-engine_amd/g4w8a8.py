@@ -432,8 +432,8 @@ def synchronize():
 # ---- the entry points ---------------------------------------------------------------------------
 #
 # The per-token calls go from the loaded library to the status test with nothing between: host time
-# is what a single small launch is bound by (g4.linear 3.9 -> 3.0 us of Python per call; 1536 x 1536
-# at one token 5.7 -> 5.0 us).
+# is what a single small launch is bound by (g4.linear 3.95 -> 3.2 us of Python per call; 1536 x 1536
+# at one token 5.95 -> 5.7 us, near what two runs differ by).
 
 def qgemv(bits, wq, scales, x, dst, k, num_rows, cols=1, in_scale=0.0, out_scale=0.0,
           x_kind=None, out_kind=None, stream=None):

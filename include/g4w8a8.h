@@ -88,8 +88,8 @@ int g4_event_elapsed_ms(float *ms, void *start, void *end);
  * decode loop is launch-bound (a launch costs microseconds of host time, more than a small GEMV
  * runs); the reference caches its per-token encode the same way (runtime.ts:702-767). Kernels of
  * this library never allocate or memset inside a capture. g4_qgemm / g4_linear with f16 or f32
- * activations at M > 32 (and at M >= 3 for some shapes once M * K * ceil(N / 16) reaches 4 Mi, where
- * one snap pass beats the small-M kernel snapping in every block) snap them into a per-stream workspace: it must
+ * activations at M > 32 (not every shape), and at M >= 3 for some shapes once M * K * ceil(N / 16) reaches
+ * 4 Mi, snap them in one pass into a per-stream workspace: it must
  * already be large enough when
  * the capture starts (run the same shape once on the stream first); a call that would grow it
  * inside a capture is refused with G4_ERR_INVALID. A workspace whose address a capture took is never
