@@ -186,9 +186,9 @@ __device__ __forceinline__ uint32_t nib_odd16(uint32_t w) { return (w ^ 0x888888
 // 4-bit interleave per 8-code group) one K chunk at a time, so a draft-verify or small prefill
 // call is one launch. 4-bit weights are taken as 16 * code (nib_even16): no zero-point sums, so half
 // the MFMAs and half the partials in the fold of a form with a row-sum product per step. Bound:
-// the chain of launch, codes, MFMAs and fold (int8 codes, us in a graph, before -> now: 16 x 1536 ->
-// 6144 5.6 -> 5.2, 32 x 6144 -> 1536 10.3 -> 9.2, 32 x 1536 -> 256 4.4 -> 3.7; with f16 x snapped
-// here 12 x 1536 -> 2048 5.9 -> 4.5, 32 x 1536 -> 256 10.6 -> 6.6).
+// the chain of launch, codes, MFMAs and fold (int8 codes, us in a graph, with row sums on 4-wave blocks of 32
+// rows -> now: 16 x 1536 -> 6144 5.1 -> 4.3, 32 x 6144 -> 1536 8.7 -> 5.5, 32 x 1536 -> 256 4.8 -> 3.7; with f16 x
+// snapped here 32 x 1536 -> 256 10.9 -> 5.0).
 // Lane (j = lane % 16, g = lane / 16) owns weight row n0 + j; per 128-code stage it loads 16 bytes
 // of that row (8-bit: 32), and MFMA half-step s takes codes g*32 + s*16 .. +16 of the stage from
 // both operands. The LDS rows are padded by 16 bytes so the 16 token rows of one A read fall on
@@ -1239,10 +1239,11 @@ __global__ __launch_bounds__(512, 4) void qgemm_wide_kernel(
 // activation operand feeds three. 3-stage ring (132 KB, one block per CU), the operand reads of each
 // half-step in flight under the MFMAs of the one before. Layouts and swizzles are the narrow tile's
 // (a stage buffer is 256 activation rows, then 192 weight columns); the weights are the MFMA's A
-// operand and the epilogue is the wide tile's. Measured: 2048 x 1536 -> 6144 in 22.8 us (1.69 int8
-// POPS; 26.6 on the wide tile), 2048 x 6144 -> 6144 67.0 us (2.31 POPS; 82.2). A stage takes about
-// 2770 cycles, near what a CU's LDS delivers under MFMA load (70-95 bytes per clock); the snap of 96
-// outputs per thread and the fill add about 8 us per tile.
+// operand and the epilogue is the wide tile's. Measured against the wide tile, alternated:
+// 2048 x 1536 -> 6144 24.7 -> 22.5 us (1.72 int8 POPS), 2048 x 6144 -> 6144 76.6 -> 66.4 us (2.33 POPS). Over the
+// first the MFMA units are busy 7.7 us and the LDS pipes about 4.3; a stage takes about 2770 cycles, its barrier
+// and first operand reads exposed with one block per CU, and the snap of 96 outputs per thread and the fill
+// add about 8 us per tile.
 constexpr int kTallBM = 256, kTallNS = 3;
 constexpr int kTallA = kTallBM * 128, kTallSB = kTallA + kWideBN * 64;
 
