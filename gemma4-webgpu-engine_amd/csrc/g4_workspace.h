@@ -1,8 +1,8 @@
 // The per-stream activation workspace of the tile GEMM: the lifetime rules, host code only.
 //
 // A g4_qgemm call whose f16 / f32 activations are snapped in a pass of their own (needs_codes_buffer)
-// keeps the codes in a device buffer that its matrix kernel then reads. The buffer belongs to (device, stream), so calls ordered on one stream
-// share it. The rules:
+// keeps the codes in a device buffer that its matrix kernel then reads. The buffer belongs to (device,
+// stream), so calls ordered on one stream share it. The rules:
 //  - A call that fits the current buffer uses it. If the stream is capturing a graph, the buffer
 //    is marked captured: the graph's nodes now hold its address.
 //  - A call that needs a larger buffer while the stream captures is refused (allocating is not

@@ -1579,19 +1579,18 @@ int workspace_forget_stream(void *stream) {
 }
 
 // The column tiles (16 weight rows each) of a 16-wave small-M block for `rows` block rows of n16 single
-// tiles, or 0 for 4-wave blocks of one tile. The fewest whose grid fits the CUs once (1, 2 or 4): a
-// CU then copies the activation codes once for all of its columns (us in a graph, int8 codes, 4-wave
-// -> two tiles: 32 x 1536 -> 6144 7.5 -> 5.3, 8 x 1536 -> 6144 4.5 -> 4.3, 32 x 6144 -> 6144 23.2 -> 11.2;
-// -> four: 32 x 1536 -> 8960 11.7 -> 7.2, 16384 12.8 -> 7.7). Past that, 32-row blocks still take
-// four (32 x 1024 -> 24576 14.9 -> 11.9) and 16-row ones, whose codes are half, the 4-wave blocks
-// (8 x 1024 -> 24576 8.1 / 9.5), which also win up to three tiles per CU while their codes take one
-// LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 -> 9000 9.8 / 8.1). 8-bit blocks of one to three K steps have
-// little to gain from a second round of four-tile blocks that is at most half full (4-wave / four tiles: 683 x
-// 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128 -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5; 20 x 256 ->
-// 16729, 1046 tiles, 10.5 / 12.2; 29 x 384 -> 18920 11.5 / 12.8), with one step also from the start of a third (513 x
-// 128 -> 2048 15.4 / 17.1) and from a grid that two tiles would have fitted but for the odd one (f16 697 x 128 ->
-// 366 5.8 / 7.4). The paired gate / up form stops
-// at two (its four would spill).
+// tiles, or 0 for 4-wave blocks of one tile. The fewest whose grid fits the CUs once (1, 2 or 4): a CU then
+// copies the activation codes once for all of its columns (us in a graph, int8 codes, 4-wave -> two tiles: 32
+// x 1536 -> 6144 7.5 -> 5.3, 8 x 1536 -> 6144 4.5 -> 4.3, 32 x 6144 -> 6144 23.2 -> 11.2; -> four: 32 x 1536
+// -> 8960 11.7 -> 7.2, 16384 12.8 -> 7.7). Past that, 32-row blocks still take four (32 x 1024 -> 24576 14.9
+// -> 11.9) and 16-row ones, whose codes are half, the 4-wave blocks (8 x 1024 -> 24576 8.1 / 9.5), which also
+// win up to three tiles per CU while their codes take one LDS chunk (8 x 1536 -> 8960 5.3 / 5.7; 8 x 4096 ->
+// 9000 9.8 / 8.1). 8-bit blocks of one to three K steps have little to gain from a second round of four-tile
+// blocks that is at most half full (4-wave / four tiles: 683 x 128 -> 749, 1034 tiles, 9.2 / 11.9; 512 x 128
+// -> 1536, 1536 tiles, 11.0 / 12.1; 1840 tiles 14.1 / 12.5; 20 x 256 -> 16729, 1046 tiles, 10.5 / 12.2; 29 x
+// 384 -> 18920 11.5 / 12.8), with one step also from the start of a third (513 x 128 -> 2048 15.4 / 17.1) and
+// from a grid that two tiles would have fitted but for the odd one (f16 697 x 128 -> 366 5.8 / 7.4). The
+// paired gate / up form stops at two (its four would spill).
 static int small_col_tiles(int bits, int64_t n16, int64_t rows, int mt, int k, bool paired) {
     const int64_t cus = device_cu_count(), blocks16 = n16 * rows;
     if (blocks16 <= cus) return 1;
@@ -1619,10 +1618,10 @@ static int small_rows(int64_t blocks16, int m) {
 enum KernelChoice { K_GEMV = 0, K_SKINNY16, K_SKINNY32, K_TILE128, K_GEMV_F32, K_GEMV_COLS,
                     K_SERIAL8, K_WIDE, K_STRIP, K_TALL };
 
-// The kernel family of a shape (route_linear goes on to the strip and the tall tile). gemm_mode: the caller named qgemm-4bit / qmatmul-8bit (execute.ts matmulKernel in gemm mode).
-// Uncalibrated qmatmul-8bit then keeps the reference's serial per-output order at any M; the
-// routed g4_linear is gemm mode only above two tokens (a decode step's 8-bit linear is qgemv-8bit,
-// execute.ts:372-375).
+// The kernel family of a shape (route_linear goes on to the strip and the tall tile). gemm_mode: the caller
+// named qgemm-4bit / qmatmul-8bit (execute.ts matmulKernel in gemm mode). Uncalibrated qmatmul-8bit then
+// keeps the reference's serial per-output order at any M; the routed g4_linear is gemm mode only above two
+// tokens (a decode step's 8-bit linear is qgemv-8bit, execute.ts:372-375).
 static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, int x_kind, bool gemm_mode) {
     if (in_scale == 0.0f) return bits == 8 && gemm_mode ? K_SERIAL8 : K_GEMV_F32;
     if (m <= 2) return K_GEMV;
@@ -1760,15 +1759,16 @@ static int strip_cols(int bits, int m, int n, int k) {
 }
 
 // The tall tile where its rounds of one block per CU are nearly full of tiles. Rounds are those of the
-// busiest XCD (column tiles go to the 8 XCDs in turn), and what fills them is counted in the wide kernel's 64-row
-// tiles, so that rows past M count as empty. One round pays from about three quarters on; several only when
-// nearly full (more so at the K whose wide loop is unrolled), since the wide kernel's blocks, two per CU, follow
-// each other without a gap. Us in a graph, int8 codes, wide / tall at the share of the rounds that is filled:
-// one round, 2048 x 1536 -> 6144 (1.00) 23.9 / 22.6, 400 x 1536 -> 24576 (0.88) 23.0 / 23.6 and K = 6144 73.8 /
-// 66.5, 800 x 1536 -> 12288 (0.81) 23.3 / 21.5, 1500 x 1536 -> 6144 (0.75) 21.1 / 23.7, 281 x 1536 -> 24576 (0.62)
-// 18.8 / 21.3; two, 1024 x 1536 -> 24576 (1.00) 44.5 / 43.1, 904 x 2816 -> 22825 (0.88) 89.9 / 85.8, 876 x 4096 -> 23141 (0.88) 110.1 / 115.5, 800 x 1536 ->
-// 24576 (0.81) 38.7 / 41.9, 513 x 1536 -> 16128 (0.39) 22.4 / 39.4; three, 1500 x 2048 -> 24576 (1.00) 82.5 / 78.9,
-// 1782 x 3840 -> 18964 (0.95) 149.5 / 136.1, 1500 x 1536 -> 16128 (0.69) 48.7 / 61.7.
+// busiest XCD (column tiles go to the 8 XCDs in turn), and what fills them is counted in the wide kernel's
+// 64-row tiles, so that rows past M count as empty. One round pays from about three quarters on; several only
+// when nearly full (more so at the K whose wide loop is unrolled), since the wide kernel's blocks, two per
+// CU, follow each other without a gap. Us in a graph, int8 codes, wide / tall at the share of the rounds that
+// is filled: one round, 2048 x 1536 -> 6144 (1.00) 23.9 / 22.6, 400 x 1536 -> 24576 (0.88) 23.0 / 23.6 and K
+// = 6144 73.8 / 66.5, 800 x 1536 -> 12288 (0.81) 23.3 / 21.5, 1500 x 1536 -> 6144 (0.75) 21.1 / 23.7, 281 x
+// 1536 -> 24576 (0.62) 18.8 / 21.3; two, 1024 x 1536 -> 24576 (1.00) 44.5 / 43.1, 904 x 2816 -> 22825 (0.88)
+// 89.9 / 85.8, 876 x 4096 -> 23141 (0.88) 110.1 / 115.5, 800 x 1536 -> 24576 (0.81) 38.7 / 41.9, 513 x 1536
+// -> 16128 (0.39) 22.4 / 39.4; three, 1500 x 2048 -> 24576 (1.00) 82.5 / 78.9, 1782 x 3840 -> 18964 (0.95)
+// 149.5 / 136.1, 1500 x 1536 -> 16128 (0.69) 48.7 / 61.7.
 static bool tall_tiles(int m, int n, int k) {
     const int64_t cus = device_cu_count(), per_xcd = cus / 8;
     const int64_t tiles_n = (n + kWideBN - 1) / kWideBN, xcd_n = (tiles_n + 7) / 8;
@@ -1879,11 +1879,11 @@ static int check_linear(int bits, const void *wq, const float *scales, const voi
     return G4_OK;
 }
 
-// The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past 48 Ki snaps
-// on the busiest CU (its rows * K per block, times its blocks there), one snap pass over the M * K
-// activations into a buffer of codes, then the kernel on int8 codes, costs less. Fused against
-// passed, us in a graph: 32 x 1536 -> 2048 (16-row blocks, 24 Ki) 5.2 / 6.3, 24 x 2048 -> 2048 (32 Ki) 5.7 / 6.4, 8 x 6144 -> 1536 (48 Ki) 8.1 / 8.0,
-// 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
+// The small-M kernel snaps f16 / f32 activations itself, in every one of its blocks: past 48 Ki snaps on the
+// busiest CU (its rows * K per block, times its blocks there), one snap pass over the M * K activations into
+// a buffer of codes, then the kernel on int8 codes, costs less. Fused against passed, us in a graph: 32 x
+// 1536 -> 2048 (16-row blocks, 24 Ki) 5.2 / 6.3, 24 x 2048 -> 2048 (32 Ki) 5.7 / 6.4, 8 x 6144 -> 1536 (48
+// Ki) 8.1 / 8.0, 12 x 6144 -> 1536 (72 Ki) 9.7 / 8.6. Below 4 Mi snaps over the whole grid the call stays
 // fused (its capture contract: it needs no buffer that an earlier call must have made).
 static bool small_presnap(int bits, int m, int n, int k, int x_kind) {
     const int64_t cus = device_cu_count();
