@@ -1898,9 +1898,18 @@ static bool small_presnap(int bits, int m, int n, int k, int x_kind) {
         return 32 * k > 64 * 1024 || (x_kind == G4_KIND_F32 && k >= 12 * kTileBK &&
                                       (int64_t)m * k * 4 >= (6 << 20) && small_rows(blocks, m) == 32);
     const int mt = small_rows(blocks, m), rows = (m + mt - 1) / mt;
-    const int ct = std::max(1, small_col_tiles(bits, blocks, rows, mt, k, false));
+    const int tiles = small_col_tiles(bits, blocks, rows, mt, k, false);
+    const int ct = tiles ? tiles : mt > 16 ? 4 : 1;  // short K on 4-wave blocks is charged as on four tiles
     const int64_t per_cu = ((blocks + ct - 1) / ct * rows + cus - 1) / cus;
     return (int64_t)m * k * blocks >= ((int64_t)1 << 22) && per_cu * std::min(m, mt) * k >= 48 * 1024;
+}
+
+// Whether the small-M kernel also serves a call of more than 32 rows in one launch: used where the call would
+// rather snap in a pass of its own and there is no buffer for the codes (a first call inside a capture).
+static bool fused_without_codes(int m, int n, int k, int x_kind) {
+    const int64_t grid16 = (int64_t)((n + 15) / 16) * ((m + 31) / 32);
+    return x_kind != G4_KIND_I8 && m > 32 && k % kTileBK == 0 && k >= 4 * kTileBK && k <= 16 * kTileBK &&
+           grid16 <= (m <= 64 || k == 16 * kTileBK ? 2 : 1) * (int64_t)device_cu_count();
 }
 
 // Whether a call snaps f16 / f32 activations into a buffer of M * K codes first (the tile kernels,
@@ -1962,8 +1971,14 @@ static int snap_pass(const void *x, int x_kind, int m, int k, float in_scale, Co
 static int run_linear(int bits, const void *wq, const float *scales, const void *x, int x_kind,
                       void *dst, int out_kind, int k, int n, int m, float in_scale,
                       float out_scale, hipStream_t stream, const char *who, bool gemm_mode = true,
-                      int8_t *given_codes = nullptr) {
-    const KernelChoice c = route_linear(bits, m, n, k, in_scale, x_kind, gemm_mode);
+                      int8_t *given_codes = nullptr, bool fused = false) {
+    const KernelChoice c = fused ? K_SKINNY32 : route_linear(bits, m, n, k, in_scale, x_kind, gemm_mode);
+    auto without_codes = [&](int rc) {
+        if (rc != G4_ERR_INVALID || !fused_without_codes(m, n, k, x_kind)) return rc;
+        clear_error();
+        return run_linear(bits, wq, scales, x, x_kind, dst, out_kind, k, n, m, in_scale, out_scale, stream,
+                          who, gemm_mode, nullptr, true);
+    };
     if (c == K_SERIAL8) {
         const dim3 grid((n + 255) / 256, m);
         if (x_kind == G4_KIND_F16)
@@ -1985,10 +2000,10 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
     if (c == K_SKINNY16 || c == K_SKINNY32) {
         // One launch, the activation snap fused into the small-M kernel; or, past small_presnap,
         // the snap pass first (natural order: the kernel's int8 path interleaves for 4-bit).
-        if (x_kind != G4_KIND_I8 && small_presnap(bits, m, n, k, x_kind)) {
+        if (x_kind != G4_KIND_I8 && !fused && small_presnap(bits, m, n, k, x_kind)) {
             const int8_t *codes = nullptr;
             int rc = snap_pass(x, x_kind, m, k, in_scale, kCodesNatural, stream, given_codes, &codes);
-            if (rc) return rc;
+            if (rc) return without_codes(rc);
             x = codes;
             x_kind = G4_KIND_I8;
         }
@@ -2011,7 +2026,7 @@ static int run_linear(int bits, const void *wq, const float *scales, const void 
         const CodeOrder order = c == K_STRIP ? (bits == 4 ? kCodesStrip4 : kCodesStrip8)
                                              : bits == 4 ? kCodesPerm : kCodesNatural;
         int rc = snap_pass(x, x_kind, m, k, in_scale, order, stream, given_codes, &codes);
-        if (rc) return rc;
+        if (rc) return without_codes(rc);
     }
     const uint8_t *w = reinterpret_cast<const uint8_t *>(wq);
     if (c == K_TALL) {
@@ -2160,8 +2175,10 @@ int qgemm_given_codes(int bits, const void *wq, const float *scales, const void 
                          out_scale);
     if (rc) return rc;
     int8_t *codes = nullptr;
-    if (needs_codes_buffer(bits, m_cols, num_rows, k, in_scale, x_kind, true)) {
-        const size_t need = (size_t)m_cols * (size_t)k;
+    const size_t need = (size_t)m_cols * (size_t)k;
+    const bool codes_first = needs_codes_buffer(bits, m_cols, num_rows, k, in_scale, x_kind, true);
+    const bool fused = codes_first && need > codes_bytes && fused_without_codes(m_cols, num_rows, k, x_kind);
+    if (codes_first && !fused) {
         if (need > codes_bytes)
             return set_error(G4_ERR_INVALID,
                              "%s: M * K = %zu activation codes exceed the %zu-byte scratch buffer "
@@ -2172,7 +2189,7 @@ int qgemm_given_codes(int bits, const void *wq, const float *scales, const void 
     }
     return run_linear(bits, wq, scales, x, x_kind, dst, out_kind, k, num_rows, m_cols, in_scale,
                       out_scale, as_stream(stream), bits == 4 ? "qgemm-4bit" : "qmatmul-8bit", true,
-                      codes);
+                      codes, fused);
 }
 
 }  // namespace g4

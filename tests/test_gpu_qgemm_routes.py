@@ -118,18 +118,23 @@ def test_sixteen_row_blocks(gpu, oracle, bits, m, n, k):
     check_every_kind(gpu, oracle, bits, m, n, k)
 
 
-@pytest.mark.parametrize("m,n,k", [(32, 2048, 1536), (17, 1536, 2048), (28, 2048, 2048)])
-def test_sixteen_row_blocks_snap_in_place(gpu, m, n, k):
-    # fewer than 48 Ki snaps on a CU: one launch with no codes buffer, so a stream's first call can be captured
-    print(f"fused snap m={m} n={n} k={k}", flush=True)
+@pytest.mark.parametrize("bits,m,n,k,xdt", [
+    # fewer than 48 Ki snaps on a CU: one launch with no codes buffer
+    (4, 32, 2048, 1536, np.float16), (4, 17, 1536, 2048, np.float16), (4, 28, 2048, 2048, np.float32),
+    # calls that snap in a pass of their own once a buffer is there
+    (4, 1024, 256, 2048, np.float32), (8, 1024, 121, 1536, np.float32), (4, 697, 361, 2048, np.float16),
+    (8, 697, 361, 2048, np.float32),
+])
+def test_first_call_inside_a_capture(gpu, bits, m, n, k, xdt):
+    print(f"captured first call bits={bits} m={m} n={n} k={k}", flush=True)
     g = np.random.default_rng(m)
-    x = gpu.DeviceBuffer.from_array(g.standard_normal((m, k)).astype(np.float16))
-    w = gpu.DeviceBuffer.from_array(g.integers(0, 256, (n, k // 2), dtype=np.uint8))
+    x = gpu.DeviceBuffer.from_array(g.standard_normal((m, k)).astype(xdt))
+    w = gpu.DeviceBuffer.from_array(g.integers(0, 256, (n, k * bits // 8), dtype=np.uint8))
     s = gpu.DeviceBuffer.from_array(g.uniform(0.005, 0.02, n).astype(np.float32))
     out, want = (gpu.DeviceBuffer.empty((m, n), np.int32) for _ in range(2))
     st = gpu.Stream()
-    graph = gpu.Graph(st, lambda: gpu.qgemm(4, w, s, x, out, k, n, m, 0.05, 0.1, stream=st.handle))
-    gpu.qgemm(4, w, s, x, want, k, n, m, 0.05, 0.1)
+    graph = gpu.Graph(st, lambda: gpu.qgemm(bits, w, s, x, out, k, n, m, 0.05, 0.1, stream=st.handle))
+    gpu.qgemm(bits, w, s, x, want, k, n, m, 0.05, 0.1)
     for _ in range(3):
         out.fill(0x7B, st.handle)
         graph.launch()
@@ -137,3 +142,19 @@ def test_sixteen_row_blocks_snap_in_place(gpu, m, n, k):
         assert np.array_equal(out.download(), want.download())
     graph.close()
     st.close()
+
+
+def test_noalloc_past_its_scratch(gpu):
+    # 12 Mi activation codes: more than the static array holds, served in one launch that needs none
+    m, n, k = 8192, 16, 1536
+    assert m * k > gpu.lib().g4_qgemm_noalloc_max_codes()
+    print(f"noalloc m={m} n={n} k={k} f32", flush=True)
+    g = np.random.default_rng(5)
+    x = gpu.DeviceBuffer.from_array(g.standard_normal((m, k)).astype(np.float32))
+    w = gpu.DeviceBuffer.from_array(g.integers(0, 256, (n, k // 2), dtype=np.uint8))
+    s = gpu.DeviceBuffer.from_array(g.uniform(0.005, 0.02, n).astype(np.float32))
+    outs = [gpu.DeviceBuffer.empty((m, n), np.int32) for _ in range(2)]
+    for fn, o in zip((gpu.qgemm_noalloc, gpu.qgemm), outs):
+        o.fill(0x7B)
+        fn(4, w, s, x, o, k, n, m, 0.05, 0.1)
+    assert np.array_equal(outs[0].download(), outs[1].download())
