@@ -1626,7 +1626,7 @@ static KernelChoice pick_kernel(int bits, int m, int n, int k, float in_scale, i
     if (in_scale == 0.0f) return bits == 8 && gemm_mode ? K_SERIAL8 : K_GEMV_F32;
     if (m <= 2) return K_GEMV;
     if (k % kTileBK != 0) return K_GEMV_COLS;
-    // the small kernel snaps all of x in each 16-row block: past 32768 rows (the tied head) the
+    // the small kernel copies or snaps all of x in each of its blocks: past 32768 rows (the tied head) the
     // re-reads outweigh the weights, and the 64-row tile (mostly padding rows) streams faster
     if (n >= 32768 && k >= 2 * kTileBK) return K_TILE128;
     if (m <= 16) return K_SKINNY16;

@@ -89,11 +89,11 @@ int g4_event_elapsed_ms(float *ms, void *start, void *end);
  * runs); the reference caches its per-token encode the same way (runtime.ts:702-767). Kernels of
  * this library never allocate or memset inside a capture. g4_qgemm / g4_linear with f16 or f32
  * activations at M > 32 (not every shape), and at M >= 3 for some shapes once M * K * ceil(N / 16) reaches
- * 4 Mi, snap them in one pass into a per-stream workspace: it must
- * already be large enough when
- * the capture starts (run the same shape once on the stream first); a call that would grow it
- * inside a capture is refused with G4_ERR_INVALID. A workspace whose address a capture took is never
- * freed (a graph may be replayed later, on any stream); g4_stream_destroy frees the stream's
+ * 4 Mi, snap them in one pass into a per-stream workspace: it must already be large enough when the
+ * capture starts (run the same shape once on the stream first); a call that would grow it inside a
+ * capture is refused with G4_ERR_INVALID, unless the small-M kernel can serve it in one launch without
+ * codes. A workspace whose address a capture took is never freed (a graph may be replayed later, on
+ * any stream); g4_stream_destroy frees the stream's
  * workspace otherwise. g4_graph_destroy waits for the graph's own last launch (an event recorded
  * after each g4_graph_launch, on the stream it was launched on, with a system-scope fence: what the
  * launch wrote to host memory can be read), not for the whole device, and releases the graph even
